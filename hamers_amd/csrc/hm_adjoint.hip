@@ -171,7 +171,7 @@ __device__ __forceinline__ void adj_face_flux(const AdjPatch& P, int64_t loc, co
         double cL, cR;
         load_stencil<D, A>(F, B, c0, c1, c2, V, cL, cR);
         const bool use_hll = sensor_hll();
-        face_adj_single_flux<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau},
+        face_adj_single_flux<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau, k.inv_thr},
                                                    use_hll, mb, h);
     }
 #pragma unroll
@@ -204,7 +204,7 @@ __device__ __forceinline__ void adj_face_recon(const AdjPatch& P, int64_t loc, c
     double* G = P.G[A];
     face_adj_single_recon<D, A, SCHEME, PP, QQ>(
         [&](int m, int e) { return ldg(pr + e * v4, iR + uint32_t(m - 3) * st); }, cL, cR,
-        LDConst{k.p, k.q, k.C, k.alpha_tau}, [&](int c) { return ldg(H + size_t(c) * mv, l32); },
+        LDConst{k.p, k.q, k.C, k.alpha_tau, k.inv_thr}, [&](int c) { return ldg(H + size_t(c) * mv, l32); },
         [&](int c, double v) { stg(G + size_t(c) * mv, l32, v); });
 }
 

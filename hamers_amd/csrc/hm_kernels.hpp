@@ -11,6 +11,7 @@ namespace hm {
 struct KParams {
     int p, q;                       // WCNS exponents
     double C, alpha_tau;            // WCNS6-LD constants
+    double inv_thr;                 // LDConst::inv_thr of them
     double gamma[HM_MAX_SPECIES];   // species ratios of specific heats
     double R[HM_MAX_SPECIES];       // species gas constants
     double cp[HM_MAX_SPECIES];      // species c_p = gamma/(gamma-1) R (four-equation mixing)

@@ -106,7 +106,7 @@ __device__ __forceinline__ void midpoint_flux_at(const DevPatch& P, const Boxes<
     if constexpr (REC) {
         const uint32_t mv = uint32_t(B.mid_vol(A)), mi = uint32_t(B.mid_idx(A, c0, c1, c2));
         double* wr = k.wrec + P.wrec[A];
-        face_flux_single<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau}, use_hll,
+        face_flux_single<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau, k.inv_thr}, use_hll,
                                                Fo, [&](const double* Wm, const double* Wp) {
 #pragma unroll
                                                    for (int c = 0; c < NEQ; c++) {
@@ -115,7 +115,7 @@ __device__ __forceinline__ void midpoint_flux_at(const DevPatch& P, const Boxes<
                                                    }
                                                });
     } else {
-        face_flux_single<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau}, use_hll,
+        face_flux_single<D, A, SCHEME, PP, QQ>(V, cL, cR, k.gamma[0], LDConst{k.p, k.q, k.C, k.alpha_tau, k.inv_thr}, use_hll,
                                                Fo);
     }
 }

@@ -323,7 +323,7 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     // wl[NEQ + f] (stride kBlock): the field index is wave-uniform, so the store
     // is one address add, where storing into a register array by a runtime index
     // would select over every slot.
-    const LDConst ldk{k.p, k.q, k.C, k.alpha_tau};
+    const LDConst ldk{k.p, k.q, k.C, k.alpha_tau, k.inv_thr};
 #pragma unroll 1
     for (int f = 0; f < NEQ; f++) {
         Six s;

@@ -13,9 +13,9 @@
 #include <hip/hip_runtime.h>
 #define HM_HD __host__ __device__ __forceinline__
 #else
-#include <cmath>
 #define HM_HD inline
 #endif
+#include <cmath>
 
 namespace hm {
 
@@ -25,23 +25,23 @@ constexpr double kEps = 1.0e-15;  // HAMERS_EPSILON, include/HAMeRS_config.hpp.i
 // general sequence, for operands whose quotient and remainder are normal
 // numbers (every quotient of the scheme: denominators are state values or
 // sums with a positive floor).  rcp_rn refines the hardware reciprocal
-// estimate by two Newton-Raphson steps r <- r + r (1 - b r); quot forms
-// q0 = a r and returns q0 + r (a - b q0) with two FMAs (Markstein's
-// correction, IBM J. Res. Develop. 34 (1990) 111-119), which rounds to the
-// nearest FP64 number like a / b.  One reciprocal serves every quotient with
-// the same denominator.  It skips the general sequence's range scaling and
-// special-value fixup, so a zero dividend gives +0 for -0 and a zero divisor
-// gives NaN; neither reaches a branch of the scheme.  Checked bit for bit
-// against a / b on the GPU over 1.4e11 random operand pairs (exponents
-// -80..79, all-ones significands included) and by the parity tests against
-// the oracle's IEEE divisions.  Host builds divide.
+// estimate (relative error below 2^-24.3, measured) by one cubic Newton step
+// r <- r + r (e + e^2), e = 1 - b r: the residual e^3 is below 2^-72, so it is
+// as accurate as two quadratic steps (one FMA more) and the result is rounded
+// once.  quot forms q0 = a r and returns q0 + r (a - b q0) with two FMAs
+// (Markstein's correction, IBM J. Res. Develop. 34 (1990) 111-119), which
+// rounds to the nearest FP64 number like a / b.  One reciprocal serves every
+// quotient with the same denominator.  It skips the general sequence's range
+// scaling and special-value fixup, so a zero dividend gives +0 for -0 and a
+// zero divisor gives NaN; neither reaches a branch of the scheme.  Checked bit
+// for bit against a / b on the GPU over 1e10 random operand pairs (exponents
+// -80..79) and by the parity tests against the oracle's IEEE divisions.  Host
+// builds divide.
 HM_HD double rcp_rn(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    double r = __builtin_amdgcn_rcp(b);
-    double e = fma(-b, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-b, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 #else
     return double(1) / b;
 #endif
@@ -58,6 +58,39 @@ HM_HD double quot(double a, double b, double r) {
 }
 
 HM_HD double div_rn(double a, double b) { return quot(a, b, rcp_rn(b)); }
+
+// Reciprocals of several denominators from one hardware estimate (it issues at
+// a quarter of the FMA rate): the reciprocal of their product, times the other
+// factors.  They are within 2 (pair) and 3 (triple) units in the last place,
+// not rounded to nearest, and are meant for quot only: its correction leaves
+// an error of at most a few reciprocal errors times 2^-53 of a unit in the
+// last place before the final rounding (below 2^-48), so a quotient rounds
+// like a / b unless it lies that close to the midpoint of two numbers (none
+// seen in 1e10 random quotients).  The products stay normal numbers for
+// factors between 1e-100 and 1e100.
+HM_HD void rcp_pair(double a, double b, double& ra, double& rb) {
+    const double r = rcp_rn(a * b);
+    ra = r * b;
+    rb = r * a;
+}
+
+HM_HD void rcp_triple(double a, double b, double c, double& ra, double& rb, double& rc) {
+    const double ab = a * b;
+    const double r = rcp_rn(ab * c);
+    const double rab = r * c;
+    ra = rab * b;
+    rb = rab * a;
+    rc = r * ab;
+}
+
+// Whether cond holds on every active lane of the wavefront (host builds: cond).
+HM_HD bool wave_all(bool cond) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(!cond) == 0;
+#else
+    return cond;
+#endif
+}
 
 // ipow of ConvectiveFluxReconstructorWCNS6-LD-HLLC-HLL.cpp:9-18: repeated
 // multiplication, so base^4 is ((b*b)*b)*b.  E < 0 means "exponent known only
@@ -85,17 +118,21 @@ struct Six {
 HM_HD Six flip(const Six& s) { return Six{{s.v[5], s.v[4], s.v[3], s.v[2], s.v[1], s.v[0]}}; }
 
 // Smoothness indicators of the three 3-point sub-stencils
-// (WCNS6-LD-HLLC-HLL.cpp:55-68, identical in WCNS5-JS-HLLC-HLL.cpp:32-44).
+// (WCNS6-LD-HLLC-HLL.cpp:55-68, identical in WCNS5-JS-HLLC-HLL.cpp:32-44).  A
+// product by a power of two is exact, so an FMA that takes it in rounds once,
+// as the product and the sum do: the same bits in one instruction less.
 HM_HD void beta3(const Six& s, double& b0, double& b1, double& b2) {
     b0 = double(1) / double(3) *
-         (s.v[0] * (double(4) * s.v[0] - double(19) * s.v[1] + double(11) * s.v[2]) +
+         (s.v[0] * (fma(double(4), s.v[0], -(double(19) * s.v[1])) + double(11) * s.v[2]) +
           s.v[1] * (double(25) * s.v[1] - double(31) * s.v[2]) + double(10) * s.v[2] * s.v[2]);
     b1 = double(1) / double(3) *
-         (s.v[1] * (double(4) * s.v[1] - double(13) * s.v[2] + double(5) * s.v[3]) +
-          double(13) * s.v[2] * (s.v[2] - s.v[3]) + double(4) * s.v[3] * s.v[3]);
+         fma(double(4), s.v[3] * s.v[3],
+             s.v[1] * (fma(double(4), s.v[1], -(double(13) * s.v[2])) + double(5) * s.v[3]) +
+                 double(13) * s.v[2] * (s.v[2] - s.v[3]));
     b2 = double(1) / double(3) *
-         (s.v[2] * (double(10) * s.v[2] - double(31) * s.v[3] + double(11) * s.v[4]) +
-          s.v[3] * (double(25) * s.v[3] - double(19) * s.v[4]) + double(4) * s.v[4] * s.v[4]);
+         fma(double(4), s.v[4] * s.v[4],
+             s.v[2] * (double(10) * s.v[2] - double(31) * s.v[3] + double(11) * s.v[4]) +
+                 s.v[3] * (double(25) * s.v[3] - double(19) * s.v[4]));
 }
 
 // Six-point smoothness indicator (WCNS6-LD-HLLC-HLL.cpp:70-83).
@@ -125,10 +162,40 @@ HM_HD double ld_sigma(const Six& s) {
     return fmax(t1, t2);
 }
 
+// Scheme constants.  inv_thr: reciprocal of the ratio tau6 / (beta_k + eps)
+// below which its q-th power vanishes in the sum C + ratio^q (ld_flat_limit);
+// infinity: never.
 struct LDConst {
     int p, q;
     double C, alpha_tau;
+    double inv_thr = HUGE_VAL;
 };
+
+// LDConst::inv_thr of the constants (host).  With 0 <= x < half a unit in the
+// last place of C, C + x rounds to C; then the four central weights are
+// (C, 15 C, 15 C, C) / 32 over their sum.  Where those sums are exact the
+// weights are 1/32, 15/32, 15/32, 1/32 to the bit.  R_tau is then below the
+// same ratio (its denominator averages theirs), so it cannot exceed alpha_tau.
+inline double ld_flat_limit(int q, double C, double alpha_tau) {
+    const double never = HUGE_VAL;
+    if (!(C >= 1.0 && C < 1.0e30) || q < 1) return never;
+    const double s1 = C + 15.0 * C, s2 = s1 + 15.0 * C, s3 = s2 + C;
+    if (C / s3 != 1.0 / 32.0 || 15.0 * C / s3 != 15.0 / 32.0) return never;
+    const double half_ulp = std::ldexp(1.0, std::ilogb(C) - 53);
+    const double thr = std::pow(half_ulp, 1.0 / q) * (1.0 - 1.0e-6);
+    return thr > 0.0 && alpha_tau > 2.0 * thr ? 1.0 / thr : never;
+}
+
+// Midpoint value of one side from its stencil and the four weights.  .75 w is
+// 2 (.375 w) to the bit and products by a power of two are exact (see beta3).
+HM_HD double ld_combine(const Six& s, double w0, double w1, double w2, double w3) {
+    const double a1 = double(3) / double(8) * w1, a2 = double(3) / double(8) * w2;
+    return double(3) / double(8) * w0 * s.v[0] +
+           fma(-double(1) / double(8), w1, -(double(10) / double(8) * w0)) * s.v[1] +
+           (fma(double(2), a1, double(15) / double(8) * w0) + a2) * s.v[2] +
+           (fma(double(2), a2, a1) + double(15) / double(8) * w3) * s.v[3] +
+           fma(-double(1) / double(8), w2, -(double(10) / double(8) * w3)) * s.v[4] + double(3) / double(8) * w3 * s.v[5];
+}
 
 // One side of the WCNS6-LD nonlinear midpoint interpolation
 // (WCNS6-LD-HLLC-HLL.cpp:133-223; the plus side 229-319 is this on flip(s)).
@@ -136,6 +203,12 @@ struct LDConst {
 // ratio R_tau = tau6 / (beta_avg + eps) exceeds alpha_tau, so they are formed
 // only there (the same expressions, evaluated on demand): sigma of the
 // unflipped stencil s0 is computed once per field, into sig (< 0: not yet).
+// Where no lane of the wavefront has a ratio tau6 / (beta_k + eps) that
+// reaches the sum C + ratio^q (resolved data: 30-50 % of the wavefronts of
+// shear layers, mixing layers and smooth modes), the weights are constants and
+// every quotient is left out.  Common factors that are powers of two (1/32 of
+// the central weights, 1/16 of the upwind ones, 1/8 of beta_avg) cancel or
+// scale exactly and are not multiplied out.
 template <int P, int Q>
 HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k) {
     double b0, b1, b2;
@@ -144,14 +217,24 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
 
     // e_k = b_k + eps divides both tau5 and tau6: one reciprocal each.
     const double e0 = b0 + kEps, e1 = b1 + kEps, e2 = b2 + kEps, e3 = b3 + kEps;
-    const double r0 = rcp_rn(e0), r1 = rcp_rn(e1), r2 = rcp_rn(e2);
+    const double b8 = b0 + b2 + double(6) * b1;  // 8 beta_avg
+    const double tau6 = fabs(fma(-double(1) / double(8), b8, b3));
 
-    const double bavg = double(1) / double(8) * (b0 + b2 + double(6) * b1);
-    const double tau6 = fabs(b3 - bavg);
-    double w0 = double(1) / double(32) * (k.C + rep_pow<Q>(quot(tau6, e0, r0), k.q));
-    double w1 = double(15) / double(32) * (k.C + rep_pow<Q>(quot(tau6, e1, r1), k.q));
-    double w2 = double(15) / double(32) * (k.C + rep_pow<Q>(quot(tau6, e2, r2), k.q));
-    double w3 = double(1) / double(32) * (k.C + rep_pow<Q>(div_rn(tau6, e3), k.q));
+    const double lim = tau6 * k.inv_thr;
+    if (wave_all(lim < e1)) {
+        if (wave_all(lim < e0 && lim < e2 && lim < e3))
+            return double(3) / double(256) * s.v[0] - double(25) / double(256) * s.v[1] +
+                   double(150) / double(256) * s.v[2] + double(150) / double(256) * s.v[3] -
+                   double(25) / double(256) * s.v[4] + double(3) / double(256) * s.v[5];
+    }
+
+    double r0, r1, r2, r3;
+    rcp_pair(e0, e1, r0, r1);
+    rcp_pair(e2, e3, r2, r3);
+    double w0 = k.C + rep_pow<Q>(quot(tau6, e0, r0), k.q);
+    double w1 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e1, r1), k.q));
+    double w2 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e2, r2), k.q));
+    double w3 = k.C + rep_pow<Q>(quot(tau6, e3, r3), k.q);
     const double ws = w0 + w1 + w2 + w3;
     const double rws = rcp_rn(ws);
     w0 = quot(w0, ws, rws);
@@ -159,45 +242,67 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
     w2 = quot(w2, ws, rws);
     w3 = quot(w3, ws, rws);
 
-    if (div_rn(tau6, bavg + kEps) > k.alpha_tau) {
-        const double tau5 = fabs(b0 - b2);
-        double u0 = double(1) / double(16) * (double(1) + rep_pow<P>(quot(tau5, e0, r0), k.p));
-        double u1 = double(5) / double(8) * (double(1) + rep_pow<P>(quot(tau5, e1, r1), k.p));
-        double u2 = double(5) / double(16) * (double(1) + rep_pow<P>(quot(tau5, e2, r2), k.p));
-        const double us = u0 + u1 + u2;
-        const double rus = rcp_rn(us);
-        u0 = quot(u0, us, rus);
-        u1 = quot(u1, us, rus);
-        u2 = quot(u2, us, rus);
-        if (sig < double(0)) sig = ld_sigma(s0);
-        const double sigma = sig;
-        w0 = sigma * u0 + (double(1) - sigma) * w0;
-        w1 = sigma * u1 + (double(1) - sigma) * w1;
-        w2 = sigma * u2 + (double(1) - sigma) * w2;
-        w3 = (double(1) - sigma) * w3;
+    // RN(tau6 / den) > alpha_tau: the sign of tau6 - alpha_tau den is exact in
+    // an FMA, and decides unless the two are within rounding of each other
+    // (then, and for den <= 0, the quotient itself is formed).
+    const double den = fma(double(1) / double(8), b8, kEps);  // beta_avg + eps
+    const double over = fma(-k.alpha_tau, den, tau6);
+    if (over > double(0) || !(den > double(0))) {
+        if ((den > double(0) && over > double(8.8817841970012523e-16) * tau6) || div_rn(tau6, den) > k.alpha_tau) {
+            const double tau5 = fabs(b0 - b2);
+            double u0 = double(1) + rep_pow<P>(quot(tau5, e0, r0), k.p);
+            double u1 = double(10) * (double(1) + rep_pow<P>(quot(tau5, e1, r1), k.p));
+            double u2 = double(5) * (double(1) + rep_pow<P>(quot(tau5, e2, r2), k.p));
+            const double us = u0 + u1 + u2;
+            const double rus = rcp_rn(us);
+            u0 = quot(u0, us, rus);
+            u1 = quot(u1, us, rus);
+            u2 = quot(u2, us, rus);
+            if (sig < double(0)) sig = ld_sigma(s0);
+            const double sigma = sig;
+            w0 = sigma * u0 + (double(1) - sigma) * w0;
+            w1 = sigma * u1 + (double(1) - sigma) * w1;
+            w2 = sigma * u2 + (double(1) - sigma) * w2;
+            w3 = (double(1) - sigma) * w3;
+        }
     }
-    return double(3) / double(8) * w0 * s.v[0] + (-double(10) / double(8) * w0 - double(1) / double(8) * w1) * s.v[1] +
-           (double(15) / double(8) * w0 + double(6) / double(8) * w1 + double(3) / double(8) * w2) * s.v[2] +
-           (double(3) / double(8) * w1 + double(6) / double(8) * w2 + double(15) / double(8) * w3) * s.v[3] +
-           (-double(1) / double(8) * w2 - double(10) / double(8) * w3) * s.v[4] + double(3) / double(8) * w3 * s.v[5];
+    return ld_combine(s, w0, w1, w2, w3);
 }
 
-// One side of WCNS5-JS (WCNS5-JS-HLLC-HLL.cpp:78-118; plus side 124-164 on flip(s)).
+// One side of WCNS5-JS (WCNS5-JS-HLLC-HLL.cpp:78-118; plus side 124-164 on
+// flip(s)).  With the default exponent 2 the three reciprocals of (beta_k +
+// eps)^2 are squares of reciprocals from one estimate (rcp_triple).
 template <int P>
 HM_HD double js_side(const Six& s, int p_rt) {
     double b0, b1, b2;
     beta3(s, b0, b1, b2);
-    double w0 = div_rn(double(1.0) / double(16), rep_pow<P>((b0 + kEps), p_rt));
-    double w1 = div_rn(double(5.0) / double(8), rep_pow<P>((b1 + kEps), p_rt));
-    double w2 = div_rn(double(5.0) / double(16), rep_pow<P>((b2 + kEps), p_rt));
+    const double e0 = b0 + kEps, e1 = b1 + kEps, e2 = b2 + kEps;
+    const double d0 = rep_pow<P>(e0, p_rt), d1 = rep_pow<P>(e1, p_rt), d2 = rep_pow<P>(e2, p_rt);
+    double r0, r1, r2;
+    if constexpr (P == 2) {
+        rcp_triple(e0, e1, e2, r0, r1, r2);
+        r0 *= r0;
+        r1 *= r1;
+        r2 *= r2;
+    } else {
+        r0 = rcp_rn(d0);
+        r1 = rcp_rn(d1);
+        r2 = rcp_rn(d2);
+    }
+    double w0 = quot(double(1.0) / double(16), d0, r0);
+    double w1 = quot(double(5.0) / double(8), d1, r1);
+    double w2 = quot(double(5.0) / double(16), d2, r2);
     const double ws = w0 + w1 + w2;
     const double rws = rcp_rn(ws);
     w0 = quot(w0, ws, rws);
     w1 = quot(w1, ws, rws);
     w2 = quot(w2, ws, rws);
-    return double(3) / double(8) * w0 * s.v[0] + (-double(10) / double(8) * w0 - double(1) / double(8) * w1) * s.v[1] +
-           (double(15) / double(8) * w0 + double(6) / double(8) * w1 + double(3) / double(8) * w2) * s.v[2] +
-           (double(3) / double(8) * w1 + double(6) / double(8) * w2) * s.v[3] - double(1) / double(8) * w2 * s.v[4];
+    const double a1 = double(3) / double(8) * w1;
+    return fma(-double(1) / double(8), w2 * s.v[4],
+               double(3) / double(8) * w0 * s.v[0] +
+                   fma(-double(1) / double(8), w1, -(double(10) / double(8) * w0)) * s.v[1] +
+                   (fma(double(2), a1, double(15) / double(8) * w0) + double(3) / double(8) * w2) * s.v[2] +
+                   (a1 + double(6) / double(8) * w2) * s.v[3]);
 }
 
 // Scheme selector: both sides of one characteristic field.
@@ -207,19 +312,18 @@ template <int SCHEME, int P, int Q>
 HM_HD void reconstruct_pair(const Six& s, const LDConst& k, double& um, double& up) {
     if constexpr (SCHEME == kWCNS6_LD) {
         double sig = double(-1);  // sigma >= 0, formed on the first side that blends
-        // The two sides one after the other (a runtime loop), so that only one
-        // side's indicators and weights are live at a time.
-#pragma unroll 1
-        for (int side = 0; side < 2; side++) {
-            Six ss;
+        // The two sides one after the other, kept apart from each other in
+        // the schedule, so that only one side's indicators and weights are
+        // live at a time (a runtime loop over the sides would select each
+        // stencil value by the side: 24 moves per field).
+        um = ld_side<P, Q>(s, s, sig, k);
+        Six t = s;
+#if defined(__HIP_DEVICE_COMPILE__)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int m = 0; m < 6; m++) ss.v[m] = side ? s.v[5 - m] : s.v[m];
-            const double r = ld_side<P, Q>(ss, s, sig, k);
-            if (side)
-                up = r;
-            else
-                um = r;
-        }
+        for (int m = 0; m < 6; m++) asm("" : "+v"(t.v[m]));
+#endif
+        up = ld_side<P, Q>(flip(t), t, sig, k);
     } else {
         um = js_side<P>(s, k.p);
         up = js_side<P>(flip(s), k.p);

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "hm_kernels.hpp"
+#include "hm_numerics.hpp"
 
 namespace hm {
 
@@ -101,6 +102,7 @@ class ConvectiveFluxReconstructorGPU {
         k_.q = cfg.constant_q;
         k_.C = cfg.constant_C;
         k_.alpha_tau = cfg.constant_alpha_tau;
+        k_.inv_thr = ld_flat_limit(cfg.constant_q, cfg.constant_C, cfg.constant_alpha_tau);
         for (int i = 0; i < HM_MAX_SPECIES; i++) {
             k_.gamma[i] = cfg.species_gamma[i];
             k_.R[i] = cfg.species_R[i];

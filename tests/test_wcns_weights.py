@@ -1,0 +1,67 @@
+"""WCNS midpoint interpolation: the kernels' rearranged weights (shared
+reciprocals, exact products taken into FMAs, constant weights where the ratios
+vanish in the sum with C, the upwind switch decided without its quotient)
+against the formulas written out term by term, bit for bit: on the host over
+random stencils (wcns_weights_check.cpp), and on the GPU against the oracle
+over the scheme constants that turn the constant-weight rule on and off, on a
+patch whose wavefronts hold resolved data, rough data and both."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from hamers_amd import workloads as W
+from oracle import oracle as O
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_host_weights_match_plain_formulas(tmp_path):
+    exe = tmp_path / "weights_check"
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-Wno-unknown-pragmas",
+                           os.path.join(ROOT, "tests", "wcns_weights_check.cpp"), "-o", str(exe)])
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    print(out.stdout)
+    assert out.returncode == 0, out.stdout
+
+
+CONSTANTS = [(1, 2, 4, 1e9, 35.0), (1, 2, 4, 1.0, 35.0), (1, 2, 4, 1e9, 1e-3), (1, 2, 4, 1e31, 35.0), (1, 3, 1, 1e6, 35.0),
+             (1, 1, 8, 123456789.123, 2.0), (0, 2, 4, 1e9, 35.0), (0, 3, 4, 1e9, 35.0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 1e7])
+@pytest.mark.parametrize("scheme,p,q,C,alpha", CONSTANTS)
+def test_constants_against_oracle(scheme, p, q, C, alpha, scale):
+    """Same bits as the oracle (its quotients and sums round as the kernel's do); pressures scaled to 1e7 as in SI units."""
+    import torch
+
+    from hamers_amd import ConvectiveFluxReconstructor, PatchData
+
+    assert torch.cuda.is_available(), "GPU tests need a visible GPU"
+    n, g = (150, 37), 4
+    rng = np.random.default_rng(3)
+    y, x = np.meshgrid(*[np.arange(-g, v + g) / v for v in (n[1], n[0])], indexing="ij")
+    rough = np.where(x > 0.6, 0.05, np.where(x > 0.5, 1e-12, 0.0)) * rng.uniform(-1, 1, x.shape)
+    rho = 1.0 + 0.3 * np.sin(2 * np.pi * (x + y)) + rough
+    u = 0.3 + 0.2 * np.cos(2 * np.pi * x) + rough
+    v = np.where(y > 0.5, 0.1 * np.sin(2 * np.pi * y), 0.0)
+    pr = scale * (1.0 + 0.2 * np.cos(2 * np.pi * (x - y)) + np.where(x > 0.8, 2.0, 0.0))
+    s = np.sqrt(scale)
+    Q = W.conservative_from_primitive_single(rho, [s * u, s * v], pr, 1.4)
+    key = "WCNS6_LD_HLLC_HLL" if scheme == 1 else "WCNS5_JS_HLLC_HLL"
+    rec = ConvectiveFluxReconstructor("weights", 2, "SINGLE_SPECIES", key, species_gamma=(1.4,), constant_p=p, constant_q=q,
+                                      constant_C=C, constant_alpha_tau=alpha)
+    F = [torch.full(O.face_shape(4, n, a), np.nan, dtype=torch.float64, device="cuda:0") for a in range(2)]
+    S = torch.zeros((4, n[1], n[0]), dtype=torch.float64, device="cuda:0")
+    dx, dt = (1.0 / n[0], 1.0 / n[1]), 1e-3
+    rec.computeConvectiveFluxAndSourceOnPatch(PatchData(n, (g, g), dx, torch.from_numpy(Q).to("cuda:0"), F, S), 0.0, dt)
+    torch.cuda.synchronize()
+    Fr, _ = O.rhs_patch(O.Params(dim=2, scheme=scheme, p=p, q=q, C=C, alpha_tau=alpha), Q, n, g, dx, dt)
+    for a in range(2):
+        got = F[a].cpu().numpy()
+        print(f"axis {a}: {int(np.sum(got != Fr[a]))} of {got.size} differ", flush=True)
+        assert np.array_equal(got, Fr[a])

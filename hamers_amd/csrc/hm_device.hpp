@@ -37,6 +37,26 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb) {
     return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// The same 64-bit value in every lane of the wavefront (lane 0's).
+__device__ __forceinline__ int64_t wave_uniform(int64_t v) {
+    const int lo = __builtin_amdgcn_readfirstlane(int(uint64_t(v) & 0xffffffffu));
+    const int hi = __builtin_amdgcn_readfirstlane(int(uint64_t(v) >> 32));
+    return int64_t((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
+}
+
+// Element at byte offset `byte` of a wave-uniform base, for loads of several
+// blocks of code at one offset.  The compiler moves the offset's extension to
+// 64 bits out of loops and branches and then forms one 64-bit vector address
+// per load instead of taking the base in scalar registers; pin_offset in the
+// block of the load keeps the 32-bit value there.
+__device__ __forceinline__ double ldg_byte(const double* base, uint32_t byte) {
+    typedef __attribute__((address_space(1))) const char gchar;
+    typedef __attribute__((address_space(1))) const double gdouble;
+    return *(gdouble*)((gchar*)base + byte);
+}
+
+__device__ __forceinline__ void pin_offset(uint32_t& byte) { asm volatile("" : "+v"(byte)); }
+
 // Store counterpart of ldg.
 __device__ __forceinline__ void stg(double* base, uint32_t i, double v) {
     typedef __attribute__((address_space(1))) char gchar;
@@ -57,6 +77,8 @@ struct DevPatch {
     double* sens;                 // scratch: theta, Omega over the 2-ghost box
     double* fmid[3];              // scratch: midpoint flux per axis, neq comps over (n_a+3) x n_b box
     double* ustar[3];             // scratch: HLLC normal velocity per axis (advective models)
+    int tile[3][4];               // shape of the axis' multi-species flux tiles (mtile_shape), and a multiplier that
+                                  // divides a thread number by a tile row (mtile_row)
     int64_t wrec[3];              // offset of this patch's axis-a chunk in a face-state slot (KParams::wrec), -1: none
 };
 
@@ -114,6 +136,16 @@ __device__ __forceinline__ int64_t q_idx(const DevPatch& P, int i, int j, int k)
 // patches.  Numbers in [start+cnt, next start) are holes.
 constexpr int kSegAlign = 64;
 
+// p as a pointer whose reads are scalar loads: the pointee must be wave-uniform
+// and not written while the kernel runs (the work tables).  Without it a read
+// after a store through another pointer becomes a vector load and a move back
+// to scalar registers.
+template <class T>
+__device__ __forceinline__ const T* as_constant(const T* p) {
+    typedef __attribute__((address_space(4))) const T ctype;
+    return (const T*)(ctype*)p;
+}
+
 template <class T>
 struct SegSingleT {  // one patch, up to 4 segments (one per axis, one extra), all by value
     T p;
@@ -131,13 +163,6 @@ struct SegSingleT {  // one patch, up to 4 segments (one per axis, one extra), a
         return true;
     }
 };
-
-// The same 64-bit value in every lane of the wavefront (lane 0's).
-__device__ __forceinline__ int64_t wave_uniform(int64_t v) {
-    const int lo = __builtin_amdgcn_readfirstlane(int(uint64_t(v) & 0xffffffffu));
-    const int hi = __builtin_amdgcn_readfirstlane(int(uint64_t(v) >> 32));
-    return int64_t((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
-}
 
 template <class T>
 struct SegTableT {  // many patches: device arrays
@@ -165,11 +190,48 @@ struct SegTableT {  // many patches: device arrays
         loc = gid - start[lo];
         if (loc >= cnt[lo]) return false;
         const int pd = seg[lo];
-        P = patches + (pd >> 2);
+        P = as_constant(patches + (pd >> 2));
         seg_axis = pd & 3;
         return true;
     }
 };
+
+// Block lookup: the segment of the block's first item and the number of whole
+// 256-item blocks before it in the segment, for stages whose segments are whole
+// blocks.  Everything is block-uniform (scalar loads and registers).
+template <class T>
+__device__ __forceinline__ bool find_block(const SegTableT<T>& w, uint32_t block, const T*& P, int& seg_axis,
+                                           uint32_t& tile) {
+    const int64_t first = int64_t(block) * kBlock;
+    const int64_t* start = as_constant(w.start);
+    if (first >= start[w.nseg]) return false;
+    int lo = 0, hi = w.nseg - 1;  // last segment with start <= first
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start[mid] <= first)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    tile = uint32_t((first - start[lo]) / kBlock);
+    const int pd = *as_constant(w.seg + lo);
+    P = as_constant(w.patches + (pd >> 2));
+    seg_axis = pd & 3;
+    return true;
+}
+
+template <class T>
+__device__ __forceinline__ bool find_block(const SegSingleT<T>& w, uint32_t block, const T*& P, int& seg_axis,
+                                           uint32_t& tile) {
+    const int64_t first = int64_t(block) * kBlock;
+    if (first >= w.start[w.nseg]) return false;
+    int s = 0;
+    while (s + 1 < w.nseg && first >= w.start[s + 1]) s++;
+    tile = uint32_t((first - w.start[s]) / kBlock);
+    P = &w.p;
+    seg_axis = s;
+    return true;
+}
 
 using SegSingle = SegSingleT<DevPatch>;
 using SegTable = SegTableT<DevPatch>;

@@ -127,6 +127,11 @@ __host__ __device__ inline void mtile_shape(int nA, int& R, int& W, int& ntA) {
     W = 256 / R;
 }
 
+// Multiplier m of an exact division of a thread number (< 256) by d <= 256:
+// x / d = x m >> 16.  m d exceeds 2^16 by less than d, so the product is off by
+// less than x d < 2^16, under one in the quotient's last place.
+__host__ __device__ inline uint32_t small_div_mul(uint32_t d) { return (65536u + d - 1u) / d; }
+
 // Work items of the fused axis-a segment of one patch: 256 per tile.
 __host__ __device__ inline int64_t mtile_items(int axis, const int* n, int dim) {
     int64_t trans = 1;  // columns: positions across the axis

@@ -30,8 +30,8 @@
 #include "hm_sensor.hpp"
 
 // Waves per SIMD the multi-species midpoint-flux kernels are compiled for, in
-// 3D and in 1D/2D (measured on the uneven 3D five-equation level: 4 waves with
-// 36 B of spill beat 3 waves without by 2.5 %; the 2D kernel would spill 70 B).
+// 3D and in 1D/2D (two species need 123 registers in 3D and spill nothing at 4
+// waves; the 1D and 2D kernels reach 4 or 5 waves by themselves).
 #ifndef HM_MIDFLUX_MULTI_WAVES_3D
 #define HM_MIDFLUX_MULTI_WAVES_3D 4
 #endif
@@ -240,7 +240,12 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
         double rho = double(0);
 #pragma unroll
         for (int si = 0; si < NS; si++) rho += V[si];
-        bool ok = true;
+        bool ok = V[NS + D] > double(0) && rho < double(1.0e100);
+        // with every partial density positive the mass fractions lie in (0, 1]
+#pragma unroll
+        for (int si = 0; si < NS; si++) ok = ok && V[si] > double(0);
+        if (ok) return true;
+        ok = true;
         const double rrho = rcp_rn(rho);
 #pragma unroll
         for (int si = 0; si < NS; si++) {
@@ -266,6 +271,19 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
     double rho = double(0);
 #pragma unroll
     for (int si = 0; si < NS; si++) rho += V[si];
+    const double p = V[NS + D];
+#pragma unroll
+    for (int si = 0; si < NS; si++) ok = ok && (V[si] > double(0));
+    if (!ok) return false;
+    // With every partial density positive the mass fractions lie in (0, 1], and
+    // with a positive pressure and xi below 1e15 Gamma and c^2 are positive
+    // (the ranges keep the quotients normal numbers): no quotient is needed.
+    double xi = double(0);
+#pragma unroll
+    for (int si = 0; si < NS; si++) xi += Z[si] * k.igm1[si];
+    if (p > double(1.0e-100) && p < double(1.0e100) && rho > double(1.0e-100) && rho < double(1.0e100) &&
+        xi > double(1.0e-100) && xi < double(1.0e15))
+        return true;
     double Y[NS];
     const double rrho = rcp_rn(rho);
 #pragma unroll
@@ -273,9 +291,6 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
         Y[si] = quot(V[si], rho, rrho);
         ok = ok && (Y[si] > double(-0.001) && Y[si] < double(1.001));
     }
-#pragma unroll
-    for (int si = 0; si < NS; si++) ok = ok && (V[si] > double(0));
-    const double p = V[NS + D];
     const double Gamma = mix_gamma_all<NS>(k, Z) - double(1);
     double c2 = quot(Gamma * p, rho, rrho);
     if constexpr (A == 0) {
@@ -288,6 +303,11 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
     return ok && (c2 > double(0));
 }
 
+// Bound by VALU issue: on the uneven 3D five-equation level of 2744 patches the
+// fused flux issues 3246 VALU instructions per wavefront at 82 % of the rate
+// (4357 at 75 % before its loads took scalar bases, a field's loads went out
+// together and the WENO weights lost a quarter of their instructions): 36.4 ms
+// -> 25.6 ms.
 // Midpoint flux Fo of the face normal to axis A between cells (c0, c1, c2)
 // - e_A and (c0, c1, c2), and its HLLC normal velocity u* (five-equation).
 // The prim and sensor arrays are read at 32-bit offsets from per-component
@@ -305,9 +325,11 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 
     const int64_t v4 = B.vol(kGc);
     const int64_t st = (A == 0) ? 1 : (A == 1) ? int64_t(B.ext(0, kGc)) : int64_t(B.ext(0, kGc)) * B.ext(1, kGc);
-    const int64_t iR = B.idx(kGc, c0, c1, c2);
+    uint32_t off = uint32_t(B.idx(kGc, c0, c1, c2)) * 8u;
     const double* pr = P.prim;
-    auto ld = [&](int comp, int m) { return pr[comp * v4 + iR + (m - 3) * st]; };
+    // component and stencil position in the wave-uniform base, so that every
+    // load takes the same 32-bit vector offset
+    auto ld = [&](int comp, int m) { return ldg_byte(pr + (comp * v4 + (m - 3) * st), off); };
 
     // Projection variables (FlowModelBasicUtilitiesFiveEqnAllaire.cpp:7474-8207).
     double Zra[NS];
@@ -318,37 +340,50 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 
     // Characteristic fields (FlowModelBasicUtilitiesFiveEqnAllaire.cpp:8232-9178),
     // one at a time: a runtime loop keeps a single field's WENO interpolation
-    // live, so the kernel fits the register file with room for more waves.
-    // Each field's two reconstructed values go to this thread's LDS slots wl[f],
-    // wl[NEQ + f] (stride kBlock): the field index is wave-uniform, so the store
-    // is one address add, where storing into a register array by a runtime index
-    // would select over every slot.
+    // live.  A field is one component of V, plus a multiple of the pressure for
+    // the acoustic fields and the partial densities; the pressure's six stencil
+    // values stay in registers (four of the seven fields of two species use
+    // them) and the multiples wait in this thread's LDS slots wl[f].  All loads
+    // of a field are issued before the first use: with one variant per kind of
+    // field the compiler waited for each pair of loads in turn and kept the
+    // load addresses of all variants in registers.  Each field's two
+    // reconstructed values go to wl[f], wl[NEQ + f] (stride kBlock): the field
+    // index is wave-uniform, so the store is one address add, where storing
+    // into a register array by a runtime index would select over every slot.
     const LDConst ldk{k.p, k.q, k.C, k.alpha_tau, k.inv_thr};
+    double ps[6];
+#pragma unroll
+    for (int m = 0; m < 6; m++) ps[m] = ld(IP, m);
+    {
+        const double rc = ra * ca;
+        const double irc = div_rn(double(1), rc);
+        wl[0] = -irc;
+        wl[(NEQ - 1) * kBlock] = irc;
+        const double rcc = rc * ca, r = rcp_rn(rcc);
+#pragma unroll
+        for (int si = 0; si < NS; si++) wl[(1 + si) * kBlock] = -quot(Zra[si], rcc, r);
+    }
+    // component of V of field f, four bits each
+    constexpr uint64_t comps = [] {
+        uint64_t c = uint64_t(IU) | uint64_t(IU) << (4 * (NEQ - 1));
+        for (int f = 1; f < NEQ - 1; f++) {
+            const int t = f - NS - 1;  // transverse slot
+            const int comp = f <= NS ? f - 1 : f < NS + D ? NS + (t < A ? t : t + 1) : IZ + (f - NS - D);
+            c |= uint64_t(comp) << (4 * f);
+        }
+        return c;
+    }();
 #pragma unroll 1
     for (int f = 0; f < NEQ; f++) {
+        const int comp = int(comps >> (4 * f)) & 15;
+        pin_offset(off);
         Six s;
-        if (f == 0) {
 #pragma unroll
-            for (int m = 0; m < 6; m++) s.v[m] = ld(IU, m) - div_rn(double(1), ra * ca) * ld(IP, m);
-        } else if (f <= NS) {
-            const int si = f - 1;
-            double z = Zra[0];
+        for (int m = 0; m < 6; m++) s.v[m] = ld(comp, m);
+        if (f <= NS || f == NEQ - 1) {
+            const double cf = wl[f * kBlock];
 #pragma unroll
-            for (int q = 1; q < NS; q++)
-                if (q == si) z = Zra[q];
-#pragma unroll
-            for (int m = 0; m < 6; m++) s.v[m] = ld(si, m) - div_rn(z, ra * ca * ca) * ld(IP, m);
-        } else if (f < NS + D) {
-            const int t = f - NS - 1;             // transverse slot
-            const int b = (t < A) ? t : t + 1;    // its axis
-#pragma unroll
-            for (int m = 0; m < 6; m++) s.v[m] = ld(NS + b, m);
-        } else if (f < NEQ - 1) {
-#pragma unroll
-            for (int m = 0; m < 6; m++) s.v[m] = ld(IZ + (f - NS - D), m);
-        } else {
-#pragma unroll
-            for (int m = 0; m < 6; m++) s.v[m] = ld(IU, m) + div_rn(double(1), ra * ca) * ld(IP, m);
+            for (int m = 0; m < 6; m++) s.v[m] = s.v[m] + cf * ps[m];
         }
         double wm, wp;
         reconstruct_pair<SCHEME, PP, QQ>(s, ldk, wm, wp);
@@ -391,6 +426,7 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 
     // Bounds on both sides, else first-order values (WCNS56-HLLC-HLL.cpp:947-1032).
     if (!(bounded_multi<D, NS, FOUR, A>(VL, k) && bounded_multi<D, NS, FOUR, A>(VR, k))) {
+        pin_offset(off);
 #pragma unroll
         for (int e = 0; e < NEQ; e++) {
             VL[e] = ld(e, 2);
@@ -747,33 +783,42 @@ __global__ __launch_bounds__(kBlock) void k_faceflux_multi(W w, KParams k) {
 static_assert(kBlock == 256, "a fused multi-species tile is one 256-thread block");
 
 template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
-__device__ __forceinline__ void flux_multi_tile(const DevPatch& P, int64_t loc, const KParams& k, double* wlds) {
+__device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile, const KParams& k, double* wlds) {
     constexpr int NEQ = Multi<D, NS, FOUR>::NEQ;
     const Boxes<D> B(P);
     const int nA = B.n[A];
-    int R, W, ntA;
-    mtile_shape(nA, R, W, ntA);
-    const uint32_t tile = uint32_t(loc) >> 8, lane = uint32_t(loc) & 255u;
-    const uint32_t tA = tile % uint32_t(ntA), tw = tile / uint32_t(ntA);
+    const int R = P.tile[A][0], W = P.tile[A][1], ntA = P.tile[A][2];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
     uint32_t r, w;
     if constexpr (A == 0) {
-        w = lane / uint32_t(R);
+        w = (lane * uint32_t(P.tile[A][3])) >> 16;  // lane / R
         r = lane - w * uint32_t(R);
     } else {
-        r = lane / uint32_t(W);
+        r = (lane * uint32_t(P.tile[A][3])) >> 16;  // lane / W
         w = lane - r * uint32_t(W);
     }
     const int j = int(tA) * (R - 2) + int(r);
-    // columns: positions across the axis, x fastest over the other axes
+    // columns: positions across the axis, x fastest over the other axes; the
+    // tile's first one is block-uniform, the others follow within a few rows
     constexpr int U = (A == 0) ? 1 : 0;  // first axis across
     constexpr int V = (A == 2) ? 1 : 2;  // second axis across
-    const uint32_t t = tw * uint32_t(W) + w;
-    const uint32_t nU = uint32_t(B.n[U]);
-    const uint32_t tv = t / nU;
+    const uint32_t nU = uint32_t(B.n[U]), t0 = tw * uint32_t(W);
+    const uint32_t v0 = t0 / nU;
+    uint32_t cu = t0 - v0 * nU + w, tv;
+    if (nU >= uint32_t(W)) {  // at most one row on
+        const bool over = cu >= nU;
+        tv = v0 + (over ? 1u : 0u);
+        cu -= over ? nU : 0u;
+    } else {  // cu < nU + W < 256
+        const uint32_t q = (cu * small_div_mul(nU)) >> 16;
+        tv = v0 + q;
+        cu -= q * nU;
+    }
     const bool in = lane < uint32_t(R * W) && j < nA + 3 && tv < uint32_t(B.n[V]);
     int c[3];
     c[A] = j - 1;
-    c[U] = int(t - tv * nU);
+    c[U] = int(cu);
     c[V] = int(tv);
     double* wl = wlds + threadIdx.x;
     if (in) {
@@ -805,18 +850,17 @@ template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
     D == 3 ? HM_MIDFLUX_MULTI_WAVES_3D : HM_MIDFLUX_MULTI_WAVES))) void k_flux_multi(W w, KParams k) {
     __shared__ double wlds[2 * Multi<D, NS, FOUR>::NEQ * kBlock];
-    const int64_t gid = int64_t(rhs_block(k)) * kBlock + threadIdx.x;
     const DevPatch* P;
     int ax;
-    int64_t loc;
-    if (!w.find(gid, P, ax, loc)) return;  // whole blocks only
+    uint32_t tile;
+    if (!find_block(w, rhs_block(k), P, ax, tile)) return;
     if (ax == 0) {
-        flux_multi_tile<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, loc, k, wlds);
+        flux_multi_tile<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, tile, k, wlds);
     } else if constexpr (D > 1) {
         if (ax == 1) {
-            flux_multi_tile<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, loc, k, wlds);
+            flux_multi_tile<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, tile, k, wlds);
         } else if constexpr (D > 2) {
-            flux_multi_tile<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, loc, k, wlds);
+            flux_multi_tile<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, tile, k, wlds);
         }
     }
 }

@@ -172,7 +172,7 @@ int hm_compute_convective_flux_and_source_on_patches(hm_ctx* ctx, const hm_patch
  *              midpoint and face flux fused, one block per tile of the patch's
  *              columns.  Single-species: 0
  * Without a pinned schedule a list uses the built-in rule (tile rows by the
- * call's size, xcd_remap 1 for the single-species model, order 0).
+ * call's size, xcd_remap 1, order 0).
  * hm_autotune_on_patches times every candidate schedule on these views
  * (`repetitions` timed RHS calls each after one warm-up, median, HIP events on
  * `stream`), pins the fastest for the list and returns it with its time and

@@ -13,12 +13,11 @@
 //   dt_level = min(min over patches of dt_patch, 1 / sum_a s_a)
 //   dt       = dt_level * cfl                  (cfl = min(cfl_init, cfl))
 //
-// The maxima are reductions of non-negative doubles: each wavefront reduces
-// its lanes with fmax (which, like the reference's fmax, passes over NaN) and
-// one lane per wavefront folds the result into an accumulator with a 64-bit
-// unsigned atomic max on the value's bits (non-negative doubles order as their
-// bit patterns), so the result does not depend on the order of the work.  A
-// one-thread kernel then forms the dt, which stays in device memory: the RHS
+// The maxima are reductions of non-negative doubles with fmax (which, like the
+// reference's fmax, passes over NaN): a bounded number of blocks each write
+// their partial maxima, and a one-block kernel reduces those, so the result
+// does not depend on the order of the work, and no accumulator is cleared.  The
+// same kernel forms the dt, which stays in device memory: the RHS
 // kernels of a level step read it there (KParams::dtp), so a captured step
 // serves every dt with no host round trip.
 #pragma once
@@ -40,18 +39,21 @@ enum : int {
     kDtTime = 6,      // sum of the step dts since the last reset
     kDtSlots = 8
 };
-constexpr int kDtAcc = 4;  // accumulators: s_0..s_2, max of the per-cell sums
+// Blocks of the spectral-radius kernel (8 per CU fill the chip), each with four
+// partial maxima: s_0..s_2 and the per-cell sums.
+constexpr int kDtBlocks = 2048;
+constexpr size_t kDtPartBytes = sizeof(double) * 4 * kDtBlocks;
 
-// Device buffers of one dt reduction: kDtAcc accumulators, then kDtSlots results.
+// Device buffers of one dt reduction: kDtPartBytes of partials, kDtSlots results.
 struct DtBuffers {
-    unsigned long long* acc = nullptr;
+    double* part = nullptr;
     double* res = nullptr;
 };
 
 // Work of the spectral-radius kernel: interior cells of every patch, one
 // segment per patch (DevPatch: n, gq, dx and the conservative arrays Q only).
-// Launches: clear the accumulators, the per-cell maxima, the one-thread
-// finish, which also adds the step's dt to the time sum kDtTime.
+// Launches: the partial maxima, then the one-block finish, which also adds the
+// step's dt to the time sum kDtTime.
 hipError_t launch_stable_dt(const hm_config& cfg, const SegTableT<DevPatch>& work, int64_t items, const KParams& k,
                             double cfl, const DtBuffers& buf, hipStream_t s);
 

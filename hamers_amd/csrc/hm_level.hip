@@ -1329,7 +1329,7 @@ class Level {
             tab.add(p, 0, cells);
         }
         const size_t tb = tab.bytes();
-        const size_t bytes = tb + up256(sizeof(unsigned long long) * kDtAcc) + up256(sizeof(double) * kDtSlots);
+        const size_t bytes = tb + kDtPartBytes + up256(sizeof(double) * kDtSlots);
         if (hipMalloc(&dt_mem_, bytes) != hipSuccess) {
             dt_mem_ = nullptr;
             return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level dt tables");
@@ -1337,9 +1337,8 @@ class Level {
         std::vector<char> img(bytes, 0);
         dt_work_ = tab.write(img.data(), static_cast<char*>(dt_mem_));
         dt_items_ = tab.total;
-        dt_buf_.acc = reinterpret_cast<unsigned long long*>(static_cast<char*>(dt_mem_) + tb);
-        dt_buf_.res = reinterpret_cast<double*>(static_cast<char*>(dt_mem_) + tb +
-                                                up256(sizeof(unsigned long long) * kDtAcc));
+        dt_buf_.part = reinterpret_cast<double*>(static_cast<char*>(dt_mem_) + tb);
+        dt_buf_.res = reinterpret_cast<double*>(static_cast<char*>(dt_mem_) + tb + kDtPartBytes);
         if (hipMemcpy(dt_mem_, img.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
             return rec_->fail(HM_ERR_DEVICE, "level dt table upload failed");
         return HM_OK;

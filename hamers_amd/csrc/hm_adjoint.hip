@@ -359,7 +359,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells(W w, KParams k) {
     }
     // Derived-data Jacobian.
     // Reciprocals instead of quotients: the adjoint carries no bit-exactness requirement.
-    const double irho = rcp_rn(rho), i2cr = rcp_rn(2.0 * cs * rho);
+    const double irho = rcp_two(rho), i2cr = rcp_two(2.0 * cs * rho);
     const double pb = Vb[IP] + cb * gam * i2cr;
     double rhob = Vb[0] - cb * gam * p * i2cr * irho;
     double ke = 0.0;

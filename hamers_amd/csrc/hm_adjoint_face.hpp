@@ -23,7 +23,7 @@ namespace hm {
 HM_HD double sgn(double x) { return x > 0.0 ? 1.0 : (x < 0.0 ? -1.0 : 0.0); }
 
 // The reverse sweep multiplies by reciprocals of shared denominators
-// (rcp_rn): its outputs carry no bit-exactness requirement, and one multiply
+// (rcp_two): its outputs are not the oracle's to the bit, and one multiply
 // replaces a quotient.  Quotients that decide a branch (R_tau > alpha_tau,
 // t1 >= t2, s* > 0, ...) are recomputed with the forward pass's correctly
 // rounded quotients (div_rn, quot), so every branch goes the forward's way.
@@ -106,13 +106,13 @@ HM_HD void ld_sigma_adj(const Six& s, double sigb, double* sb) {
     const double t2 = div_rn(fabs(x2), den2);
     double a1b = 0.0, a2b = 0.0, a3b = 0.0;
     if (t1 >= t2) {
-        const double id = rcp_rn(den1);
+        const double id = rcp_two(den1);
         const double xb = sigb * sgn(x1) * id;
         const double db = -sigb * t1 * id;
         a1b += xb + db * sgn(a1);
         a2b += -xb + db * sgn(a2);
     } else {
-        const double id = rcp_rn(den2);
+        const double id = rcp_two(den2);
         const double xb = sigb * sgn(x2) * id;
         const double db = -sigb * t2 * id;
         a2b += xb + db * sgn(a2);
@@ -136,8 +136,8 @@ HM_HD void ld_side_adj(const Six& s, double sigma, const LDConst& k, double ob, 
     double b0, b1, b2;
     beta3(s, b0, b1, b2);
     const double b3 = beta6(s);
-    const double ie0 = rcp_rn(b0 + kEps), ie1 = rcp_rn(b1 + kEps), ie2 = rcp_rn(b2 + kEps),
-                 ie3 = rcp_rn(b3 + kEps);
+    const double ie0 = rcp_two(b0 + kEps), ie1 = rcp_two(b1 + kEps), ie2 = rcp_two(b2 + kEps),
+                 ie3 = rcp_two(b3 + kEps);
     const double bavg = double(1) / double(8) * (b0 + b2 + double(6) * b1);
     const double d3 = b3 - bavg;
     const double tau6 = fabs(d3);
@@ -147,7 +147,7 @@ HM_HD void ld_side_adj(const Six& s, double sigma, const LDConst& k, double ob, 
     const double w1 = double(15) / double(32) * (k.C + rep_pow<Q>(q1, k.q));
     const double w2 = double(15) / double(32) * (k.C + rep_pow<Q>(q2, k.q));
     const double w3 = double(1) / double(32) * (k.C + rep_pow<Q>(q3, k.q));
-    const double iws = rcp_rn(w0 + w1 + w2 + w3);
+    const double iws = rcp_two(w0 + w1 + w2 + w3);
     const double wh0 = w0 * iws, wh1 = w1 * iws, wh2 = w2 * iws, wh3 = w3 * iws;
     const double* v = s.v;
     const double Wb0 = ob * (3.0 / 8.0 * v[0] - 10.0 / 8.0 * v[1] + 15.0 / 8.0 * v[2]);
@@ -166,7 +166,7 @@ HM_HD void ld_side_adj(const Six& s, double sigma, const LDConst& k, double ob, 
         const double u0 = double(1) / double(16) * (double(1) + rep_pow<P>(r0, k.p));
         const double u1 = double(5) / double(8) * (double(1) + rep_pow<P>(r1, k.p));
         const double u2 = double(5) / double(16) * (double(1) + rep_pow<P>(r2, k.p));
-        const double ius = rcp_rn(u0 + u1 + u2);
+        const double ius = rcp_two(u0 + u1 + u2);
         const double uh0 = u0 * ius, uh1 = u1 * ius, uh2 = u2 * ius;
         const double om = double(1) - sigma;
         W0 = sigma * uh0 + om * wh0;
@@ -236,11 +236,11 @@ HM_HD void js_side_adj(const Six& s, int p_rt, double ob, double* sb) {
     if (ob == 0.0) return;
     double b0, b1, b2;
     beta3(s, b0, b1, b2);
-    const double ie0 = rcp_rn(b0 + kEps), ie1 = rcp_rn(b1 + kEps), ie2 = rcp_rn(b2 + kEps);
+    const double ie0 = rcp_two(b0 + kEps), ie1 = rcp_two(b1 + kEps), ie2 = rcp_two(b2 + kEps);
     const double w0 = double(1.0) / double(16) * rep_pow<P>(ie0, p_rt);
     const double w1 = double(5.0) / double(8) * rep_pow<P>(ie1, p_rt);
     const double w2 = double(5.0) / double(16) * rep_pow<P>(ie2, p_rt);
-    const double iws = rcp_rn(w0 + w1 + w2);
+    const double iws = rcp_two(w0 + w1 + w2);
     const double W0 = w0 * iws, W1 = w1 * iws, W2 = w2 * iws;
     const double* v = s.v;
     sb[0] += ob * (3.0 / 8.0 * W0);
@@ -418,7 +418,7 @@ HM_HD void riemann_single_adj(const double* VL, const double* VR, double gam, bo
             const double be2 = double(1) - be1;
             double be1b = 0.0, be2b = 0.0;
             const double dsl = sR - sL;
-            const double idsl = rcp_rn(dsl);
+            const double idsl = rcp_two(dsl);
 #pragma unroll
             for (int e = 0; e < NEQ; e++) {
                 const bool hyb = (e == 0) || (e >= 1 && e <= D && e != 1 + A);
@@ -451,13 +451,13 @@ HM_HD void riemann_single_adj(const double* VL, const double* VR, double gam, bo
             }
             be1b -= be2b;
             if (!tiny) {
-                const double iS = rcp_rn(Ssum);
+                const double iS = rcp_two(Ssum);
                 const double al1b = be1b * 0.5 * al2 * (iS * iS);
                 double al2b = -be1b * 0.5 * al1 * (iS * iS);
                 double a1b = al1b;
-                if (al2 > 0.0) a1b += al2b * (-al1 * rcp_rn(al2));
+                if (al2 > 0.0) a1b += al2b * (-al1 * rcp_two(al2));
                 const double dua = du[A];
-                const double ivm = rcp_rn(vm);  // vm >= kEps here
+                const double ivm = rcp_two(vm);  // vm >= kEps here
                 const double duab = a1b * sgn(dua) * ivm;
                 const double vmb = -a1b * al1 * ivm;
                 const double dsqb = vmb * 0.5 * ivm;
@@ -504,14 +504,14 @@ HM_HD void riemann_single_adj(const double* VL, const double* VR, double gam, bo
         const double hb = innerb * (s_star - uK);
         rhoKb += hb * s_star;
         sstb += hb * rhoK;
-        const double ig = rcp_rn(g);
+        const double ig = rcp_two(g);
         pKb += hb * ig;
         const double gb = -hb * pK * (ig * ig);
         sKb += gb;
         uKb -= gb;
     }
     {
-        const double ib2 = rcp_rn(sK - s_star);
+        const double ib2 = rcp_two(sK - s_star);
         const double ab = chib * ib2;
         const double b2b = -chib * chi * ib2;
         sKb += ab + b2b;
@@ -575,7 +575,7 @@ HM_HD void riemann_single_adj(const double* VL, const double* VR, double gam, bo
     }
     // s* = num / den
     {
-        const double iden = rcp_rn(den);
+        const double iden = rcp_two(den);
         const double numb = sstb * iden;
         const double denb = -sstb * s_star * iden;
         Vb[1][IP] += numb;
@@ -609,12 +609,12 @@ HM_HD void riemann_single_adj(const double* VL, const double* VR, double gam, bo
     csb[1] += 0.5 * cavgb;
     // c = sqrt(gam p / rho), eps = p / ((gam - 1) rho)
     const double css[2] = {csL, csR};
-    const double igm1 = rcp_rn(gam - 1.0);
+    const double igm1 = rcp_two(gam - 1.0);
 #pragma unroll
     for (int x = 0; x < 2; x++) {
         const double* V = Vs[x];
-        const double irho = rcp_rn(V[0]);
-        const double ab = csb[x] * 0.5 * rcp_rn(css[x]);
+        const double irho = rcp_two(V[0]);
+        const double ab = csb[x] * 0.5 * rcp_two(css[x]);
         Vb[x][IP] += ab * gam * irho + epsb[x] * igm1 * irho;
         Vb[x][0] -= ab * gam * V[IP] * (irho * irho) + epsb[x] * epss[x] * irho;
     }
@@ -713,7 +713,7 @@ HM_HD void face_adj_single_after_recon(const double* Wm, const double* Wp, const
     }
     // Back-projection adjoint for both sides.
     double rab = 0.0, cab = 0.0;
-    const double ica = rcp_rn(ca), ira = rcp_rn(ra);
+    const double ica = rcp_two(ca), ira = rcp_two(ra);
     auto back_adj = [&](const double* W, const double* Vob, double* Wb) {
         const double ic2 = div_rn(double(1), ca * ca);
         const double irc = div_rn(double(1), ra * ca);
@@ -798,7 +798,7 @@ HM_HD void face_adj_single_recon(const VAt& vat, double cL, double cR, const LDC
     const double ra = double(1) / double(2) * (vat(2, 0) + vat(3, 0));
     const double ca = double(1) / double(2) * (cL + cR);
     double rab = hat(2 * NEQ), cab = hat(2 * NEQ + 1);
-    const double ic3 = rcp_rn(ca * ca * ca);
+    const double ic3 = rcp_two(ca * ca * ca);
 #pragma unroll 1
     for (int f = 0; f < NEQ; f++) {
         Six s;
@@ -844,7 +844,7 @@ HM_HD void face_record_to_point(double flag, const GAt& gat, double ra, double c
     Vbm[1 + A] += g0 * -0.5 * ra * ca;
     Vbm[IP] += 0.5 * g0;
     Vbm[0] += g1;
-    Vbm[IP] -= g1 * rcp_rn(ca * ca);
+    Vbm[IP] -= g1 * rcp_two(ca * ca);
     int t = 2;
     for (int b = 0; b < D; b++) {
         if (b == A) continue;

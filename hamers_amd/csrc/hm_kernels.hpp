@@ -43,6 +43,9 @@ struct KParams {
     // contiguous range of block numbers (xcd_block), 0 keeps the hardware's
     // round-robin order.
     int xcd;
+    // 1: the advective source is set instead of accumulated (a level's stage
+    // sources start at zero); 0: accumulated, as the reference does.
+    int s_set;
     // Work-queue counter of the persistent midpoint-flux kernel (one unsigned
     // in device memory, cleared in-stream before each launch); NULL otherwise.
     unsigned* queue;

@@ -5,10 +5,17 @@
 //   fill ghosts of the scratch state (same level + periodic images,
 //   then the physical boundary conditions)                              :1568
 //   for each stage sn:
-//     intermediate[sn] <- scratch (whole ghost box)                       :1677
+//     intermediate[sn] <- scratch                                         :1677
 //     sn > 0: fill ghosts of intermediate[sn] (the same fill)             :1686-1711
 //     S[sn] <- 0, F[sn], S[sn] <- batched convective RHS of intermediate  Euler.cpp:904-1001
 //     scratch interior <- stage update from intermediate[0..sn]           Euler.cpp:1003-1680
+//
+// No state is copied between buffers: a stage's update writes the next stage's
+// intermediate (the last one's the scratch state), intermediate 0 is the
+// scratch state itself, which the last update overwrites cell by cell, and
+// only ghost cells that no fill covers are carried over.  (The coarse level of
+// a hierarchy keeps a copy of its start state.)  The copies and the zero fill
+// of the sources took 0.5 ms of a 7.9 ms step of 5.5 M five-equation cells.
 //
 // One step is a fixed sequence of launches on one stream, so it is captured
 // once into a hipGraph and replayed.  Ghost cells inside the domain that no
@@ -142,19 +149,19 @@ __global__ __launch_bounds__(kBlock) void k_copy_state(SegTableT<LevelPatch> w, 
     for (int c = 0; c < nq; c++) P->Q[to][c * P->gvol + loc] = P->Q[from][c * P->gvol + loc];
 }
 
-// Zero the source of one stage (Euler.cpp:913-926); a kernel, not a memset, so
-// that the step can be captured in a graph.  Only the advective equations'
-// components (from first on) are ever written by the RHS; the others stay at
-// the zero the storage was allocated with.
-__global__ __launch_bounds__(kBlock) void k_zero_source(SegTableT<LevelPatch> w, int stage, int first) {
-    const int64_t gid = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    const LevelPatch* P;
-    int ax;
-    int64_t loc;
-    if (!w.find(gid, P, ax, loc)) return;
-    P->S[stage][int64_t(first) * P->n[0] * P->n[1] * P->n[2] + loc] = 0.0;
+// Copies listed cells (patch, ghost-box index) between two state buffers: the
+// ghost cells that neither a same-level copy nor a boundary condition fills.
+struct CellRef {
+    int patch, idx;
+};
+__global__ __launch_bounds__(kBlock) void k_copy_cells(const CellRef* cells, int64_t n, const LevelPatch* patches,
+                                                       int from, int to, int nq) {
+    const int64_t t = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (t >= n) return;
+    const CellRef c = cells[t];
+    const LevelPatch& P = patches[c.patch];
+    for (int e = 0; e < nq; e++) P.Q[to][e * P.gvol + c.idx] = P.Q[from][e * P.gvol + c.idx];
 }
-
 
 // ----------------------------------------------------------------------------
 // Adjoint of the stage loop (discrete adjoint of one level's RK steps).
@@ -436,10 +443,7 @@ class Level {
         if (hipDeviceSynchronize() != hipSuccess ||
             hipMemcpy(h.data(), patch_[p].Q[0], h.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
             return rec_->fail(HM_ERR_DEVICE, "hipMemcpy from the level failed");
-        const double* src = Q;
-        const int64_t vol = ivol(p);
-        for (int c = 0; c < nq_; c++)
-            for (int64_t l = 0; l < vol; l++) h[size_t(c) * gvol(p) + gidx_of_interior(p, l)] = src[c * vol + l];
+        for_interior_rows(p, nq_, [&](int64_t l, int64_t gi, size_t b) { std::memcpy(&h[gi], Q + l, b); });
         if (hipMemcpy(patch_[p].Q[0], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
             return rec_->fail(HM_ERR_DEVICE, "hipMemcpy to the level failed");
         return HM_OK;
@@ -451,9 +455,7 @@ class Level {
         if (hipDeviceSynchronize() != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "device synchronize failed");
         if (hipMemcpy(h.data(), patch_[p].Q[0], h.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
             return rec_->fail(HM_ERR_DEVICE, "hipMemcpy from the level failed");
-        const int64_t vol = ivol(p);
-        for (int c = 0; c < nq_; c++)
-            for (int64_t l = 0; l < vol; l++) Q[c * vol + l] = h[size_t(c) * gvol(p) + gidx_of_interior(p, l)];
+        for_interior_rows(p, nq_, [&](int64_t l, int64_t gi, size_t b) { std::memcpy(Q + l, &h[gi], b); });
         return HM_OK;
     }
 
@@ -507,20 +509,22 @@ class Level {
         drop_graphs();
         hipLaunchKernelGGL(k_copy_state, dim3(blocks_for(copy_items_)), dim3(kBlock), 0, s, copy_, 0, 1, nq_);
         if (int st = launch_halo(1, s)) return st;
-        if (zero_items_ > 0)
-            hipLaunchKernelGGL(k_zero_source, dim3(blocks_for(zero_items_)), dim3(kBlock), 0, s, zero_, 0, src_first_);
+        // on a copy of the state (buffer 1), whichever buffer the steps' first stage reads
+        std::vector<hm_patch_view> views = views_[0];
+        for (int p = 0; p < np_; p++)
+            for (int e = 0; e < nq_; e++) views[p].Q[e] = patch_[p].Q[1] + size_t(e) * gvol(p);
         const bool single = rec_->config().model == HM_MODEL_SINGLE_SPECIES;
         ConvectiveFluxReconstructorGPU::OwnedPlan trial;
-        const Schedule dflt = rec_->defaultSchedule(views_[0].data(), np_);
+        const Schedule dflt = rec_->defaultSchedule(views.data(), np_);
         int st = rec_->tuneSchedules(
             s, reps,
             [&](const Schedule& sc) {
                 if (hipStreamSynchronize(s) != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "stream synchronize failed");
-                return rec_->buildOwnedPlan(views_[0].data(), np_, static_cast<double*>(rhs_scratch_), trial,
+                return rec_->buildOwnedPlan(views.data(), np_, static_cast<double*>(rhs_scratch_), trial,
                                             single ? wst_off_.data() : nullptr, &sc);
             },
             [&]() {
-                if (int e = rec_->runOwnedPlan(trial, dt, s)) return e;
+                if (int e = rec_->runOwnedPlan(trial, dt, s, nullptr, nullptr, true)) return e;
                 if (diff_) return diff_->runOwnedPlan(diff_plan_[0], dt, s);
                 return int(HM_OK);
             },
@@ -540,10 +544,26 @@ class Level {
     }
     const Schedule& schedule() const { return sched_; }
 
+    // The start state of each step stays in buffer 1 (a hierarchy's coarse
+    // level interpolates and synchronizes from it): the first stage then reads
+    // a copy there.  Drops the captured steps (their tables change).
+    int keepStartState() {
+        if (first_buf_ == 1) return HM_OK;
+        if (hipDeviceSynchronize() != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "device synchronize failed");
+        drop_graphs();
+        first_buf_ = 1;
+        for (int p = 0; p < np_; p++)
+            for (int e = 0; e < nq_; e++) views_[0][p].Q[e] = patch_[p].Q[1] + size_t(e) * gvol(p);
+        if (int st = build_rhs_plans()) return st;
+        if (diff_)
+            if (int st = build_diff_plan(0)) return st;
+        return build_rk_tables();
+    }
+
     // Flux sums for the synchronization of a two-level hierarchy: F_acc of
-    // every axis and S_acc accumulate gamma_s F_s and gamma_s S_s over the
-    // stages of every step (Euler.cpp:1230-1270, 1360-1420, 1560-1660) until
-    // clearFluxSums; in the Navier-Stokes form also Fd_acc the diffusive
+    // every axis and S_acc hold the sums of gamma_s F_s and gamma_s S_s over
+    // the stages of the last step (Euler.cpp:1230-1270, 1360-1420, 1560-1660);
+    // in the Navier-Stokes form also Fd_acc those of the diffusive
     // fluxes (a flux variable of its own, NavierStokes.cpp:393-402).  Drops
     // the captured steps (their tables change).
     int enableFluxSums() {
@@ -569,7 +589,6 @@ class Level {
             return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level flux sums");
         }
         if (hipMemset(acc_mem_, 0, total) != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "flux-sum clear");
-        acc_bytes_ = total;
         facc_.assign(size_t(np_) * 3, nullptr);
         fdacc_.assign(size_t(np_) * 3, nullptr);
         sacc_.assign(size_t(np_), nullptr);
@@ -585,17 +604,16 @@ class Level {
         return build_tables();
     }
 
-    int clearFluxSums(hipStream_t s) {
-        if (!acc_mem_) return HM_OK;
-        return hipMemsetAsync(acc_mem_, 0, acc_bytes_, s) == hipSuccess ? HM_OK
-                                                                        : rec_->fail(HM_ERR_DEVICE, "flux-sum clear");
-    }
-
     // Pieces of the level a two-level hierarchy drives.
     int stepOnce(double dt, hipStream_t s) { return step(dt, s); }
     int fillGhostsOf(int buf, hipStream_t s) { return launch_halo(buf, s); }
     const LevelPatch* devPatches() const { return patch_dev(); }
     const LevelPatch& hostPatch(int p) const { return patch_[p]; }
+    // Stage fluxes and the step's gamma terms over them (the fine level's sums
+    // are formed only on the faces that are refluxed).
+    const double* stageFlux(int p, int stage, int a) const { return fl_[(size_t(p) * kMaxRK + stage) * 3 + a]; }
+    const double* stageDiffusiveFlux(int p, int stage, int a) const { return fdl_[(size_t(p) * kMaxRK + stage) * 3 + a]; }
+    const AccTerms& stepTerms() const { return step_terms_; }
     double* fluxSum(int p, int a) const { return facc_[size_t(p) * 3 + a]; }
     double* diffusiveFluxSum(int p, int a) const { return fdacc_.empty() ? nullptr : fdacc_[size_t(p) * 3 + a]; }
     double* sourceSum(int p) const { return sacc_[p]; }
@@ -828,18 +846,21 @@ class Level {
         for (int a = 0; a < d_; a++) v *= n_[3 * p + a] + (a == ax);
         return v;
     }
-    int64_t gidx_of_interior(int p, int64_t l) const {
+    // Copies the interior of patch p between an interior array and a ghost-box
+    // array of nc components on the host, row by row.
+    template <class Copy>
+    void for_interior_rows(int p, int nc, Copy&& copy) const {
         const int* n = &n_[3 * p];
-        int c[3] = {0, 0, 0};
-        c[0] = int(l % n[0]);
-        if (d_ > 1) c[1] = int((l / n[0]) % n[1]);
-        if (d_ > 2) c[2] = int(l / (int64_t(n[0]) * n[1]));
-        int64_t idx = 0, st = 1;
-        for (int a = 0; a < d_; a++) {
-            idx += (c[a] + g_) * st;
-            st *= n[a] + 2 * g_;
-        }
-        return idx;
+        const int n1 = d_ > 1 ? n[1] : 1, n2 = d_ > 2 ? n[2] : 1;
+        const int64_t e0 = n[0] + 2 * g_, e1 = d_ > 1 ? n[1] + 2 * g_ : 1;
+        const int64_t gv = gvol(p), vol = ivol(p);
+        for (int c = 0; c < nc; c++)
+            for (int k = 0; k < n2; k++)
+                for (int j = 0; j < n1; j++) {
+                    const int64_t l = (int64_t(k) * n1 + j) * n[0];
+                    const int64_t gi = (int64_t(k + (d_ > 2 ? g_ : 0)) * e1 + j + (d_ > 1 ? g_ : 0)) * e0 + g_;
+                    copy(c * vol + l, c * gv + gi, size_t(n[0]) * sizeof(double));
+                }
     }
 
     int allocate() {
@@ -894,7 +915,7 @@ class Level {
                     v.ghost[a] = a < d_ ? g_ : 0;
                     v.dx[a] = dx_[a];
                 }
-                for (int e = 0; e < nq_; e++) v.Q[e] = patch_[p].Q[1 + s] + size_t(e) * gvol(p);
+                for (int e = 0; e < nq_; e++) v.Q[e] = patch_[p].Q[stage_buf(s)] + size_t(e) * gvol(p);
                 for (int a = 0; a < d_; a++) v.F[a] = fl_[(size_t(p) * kMaxRK + s) * 3 + a];
                 v.S = patch_[p].S[s];
                 views_[s][p] = v;
@@ -919,25 +940,14 @@ class Level {
         sched_ = rec_->defaultSchedule(views_[0].data(), np_);
         if (int st = build_rhs_plans()) return st;
         if (diff_) {
-            // Diffusive RHS of every intermediate buffer into the stage's
-            // diffusive fluxes; the stages share one scratch region.
-            std::vector<hm_patch_view> dv(np_);
-            for (int s = 0; s < kMaxRK; s++) {
-                for (int p = 0; p < np_; p++) {
-                    dv[p] = views_[s][p];
-                    for (int a = 0; a < d_; a++) dv[p].F[a] = fdl_[(size_t(p) * kMaxRK + s) * 3 + a];
-                    dv[p].S = nullptr;
-                }
-                if (s == 0) {
-                    const size_t dd = diff_->scratchDoubles(dv.data(), np_);
-                    if (hipMalloc(&diff_scratch_, dd * sizeof(double)) != hipSuccess) {
-                        diff_scratch_ = nullptr;
-                        return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level diffusive scratch");
-                    }
-                }
-                if (int st = diff_->buildOwnedPlan(dv.data(), np_, static_cast<double*>(diff_scratch_), diff_plan_[s]))
-                    return st;
+            // The stages share one scratch region.
+            const size_t dd = diff_->scratchDoubles(views_[0].data(), np_);
+            if (hipMalloc(&diff_scratch_, dd * sizeof(double)) != hipSuccess) {
+                diff_scratch_ = nullptr;
+                return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level diffusive scratch");
             }
+            for (int s = 0; s < kMaxRK; s++)
+                if (int st = build_diff_plan(s)) return st;
         }
         if (hipStreamCreateWithFlags(&cap_stream_, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&ev_a_, hipEventDisableTiming) != hipSuccess ||
@@ -954,6 +964,63 @@ class Level {
                                               single ? wst_off_.data() : nullptr, &sched_))
                 return st;
         return HM_OK;
+    }
+
+    // Diffusive RHS of stage s's intermediate into the stage's diffusive fluxes.
+    int build_diff_plan(int s) {
+        std::vector<hm_patch_view> dv = views_[s];
+        for (int p = 0; p < np_; p++) {
+            for (int a = 0; a < d_; a++) dv[p].F[a] = fdl_[(size_t(p) * kMaxRK + s) * 3 + a];
+            dv[p].S = nullptr;
+        }
+        return diff_->buildOwnedPlan(dv.data(), np_, static_cast<double*>(diff_scratch_), diff_plan_[s]);
+    }
+
+    // State buffer of stage s's intermediate (0: the scratch state).
+    int stage_buf(int s) const { return s == 0 ? first_buf_ : 1 + s; }
+
+    // Ghost cells that no same-level copy and no boundary condition fills.
+    // The fills of disjoint patches are disjoint, so a patch whose fills add up
+    // to its ghost cells has none; the others' cells are marked one by one.
+    std::vector<CellRef> uncovered(const std::vector<HaloItem>& halo, const std::vector<BcItem>& bc) const {
+        std::vector<int64_t> open(np_);
+        bool overlap = false;
+        for (int p = 0; p < np_; p++) open[p] = gvol(p) - ivol(p);
+        for (const HaloItem& it : halo) {
+            open[it.dst] -= int64_t(it.ext[0]) * it.ext[1] * it.ext[2];
+            bool inside = true;  // a copy into the patch's own interior: overlapping patches
+            for (int a = 0; a < d_; a++)
+                inside = inside && it.lo[a] + it.ext[a] > g_ && it.lo[a] < g_ + n_[3 * it.dst + a];
+            overlap = overlap || inside;
+        }
+        for (const BcItem& it : bc) open[it.dst] -= int64_t(it.ext[0]) * it.ext[1] * it.ext[2];
+        std::vector<std::vector<char>> mark(np_);
+        auto cover = [&](int p, const int* lo, const int* ext) {
+            if (mark[p].empty()) return;
+            const int e0 = n_[3 * p] + 2 * g_, e1 = d_ > 1 ? n_[3 * p + 1] + 2 * g_ : 1;
+            for (int z = 0; z < ext[2]; z++)
+                for (int y = 0; y < ext[1]; y++) {
+                    char* row = &mark[p][(size_t(lo[2] + z) * e1 + (lo[1] + y)) * e0 + lo[0]];
+                    std::fill(row, row + ext[0], 1);
+                }
+        };
+        for (int p = 0; p < np_; p++) {
+            if (open[p] == 0 && !overlap) continue;
+            mark[p].assign(size_t(gvol(p)), 0);
+            int lo[3], ext[3];
+            for (int a = 0; a < 3; a++) {
+                lo[a] = a < d_ ? g_ : 0;
+                ext[a] = a < d_ ? n_[3 * p + a] : 1;
+            }
+            cover(p, lo, ext);
+        }
+        for (const HaloItem& it : halo) cover(it.dst, it.lo, it.ext);
+        for (const BcItem& it : bc) cover(it.dst, it.lo, it.ext);
+        std::vector<CellRef> out;
+        for (int p = 0; p < np_; p++)
+            for (size_t i = 0; i < mark[p].size(); i++)
+                if (!mark[p][i]) out.push_back(CellRef{p, int(i)});
+        return out;
     }
 
     // Same-level ghost copies, periodic images included.
@@ -1103,24 +1170,18 @@ class Level {
         bc_bad_ = false;
         build_bc(bc);
         if (bc_bad_) return rec_->fail(HM_ERR_INVALID_ARGUMENT, "boundary-condition source outside a ghost box");
-        TableImage<LevelPatch> copy, zero;
+        TableImage<LevelPatch> copy;
         copy.items = patch_;
-        zero.items = patch_;
-        // advective equations: the five-equation model's volume fractions
-        const hm_config& cfg = rec_->config();
-        const int nadv = cfg.model == HM_MODEL_FIVE_EQN_ALLAIRE ? cfg.num_species - 1 : 0;
-        src_first_ = cfg.model == HM_MODEL_FIVE_EQN_ALLAIRE ? cfg.num_species + d_ + 1 : 0;
-        for (int p = 0; p < np_; p++) {
-            copy.add(p, 0, gvol(p));
-            if (nadv > 0) zero.add(p, 0, int64_t(nadv) * ivol(p));
-        }
+        for (int p = 0; p < np_; p++) copy.add(p, 0, gvol(p));
+        const std::vector<CellRef> bare = uncovered(halo.items, bc.items);
         halo_host_ = halo.items;
         halo_items_ = halo.total;
         bc_items_ = bc.total;
         copy_items_ = copy.total;
-        zero_items_ = zero.total;
+        bare_items_ = int64_t(bare.size());
+        const size_t bare_bytes = up256(sizeof(CellRef) * bare.size());
         const size_t dir_bytes = up256(sizeof(double) * 6 * size_t(nq_));
-        const size_t bytes = halo.bytes() + bc.bytes() + dir_bytes + copy.bytes() + zero.bytes() + rk_bytes();
+        const size_t bytes = halo.bytes() + bc.bytes() + dir_bytes + copy.bytes() + bare_bytes + rk_bytes();
         if (tables_) (void)hipFree(tables_);
         tables_ = nullptr;
         if (hipMalloc(&tables_, bytes) != hipSuccess) return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level tables");
@@ -1136,8 +1197,9 @@ class Level {
         o += dir_bytes;
         copy_ = copy.write(h.data() + o, d + o);
         o += copy.bytes();
-        zero_ = zero.write(h.data() + o, d + o);
-        o += zero.bytes();
+        if (!bare.empty()) std::memcpy(h.data() + o, bare.data(), sizeof(CellRef) * bare.size());
+        bare_ = reinterpret_cast<const CellRef*>(d + o);
+        o += bare_bytes;
         rk_off_ = o;
         if (hipMemcpy(tables_, h.data(), o, hipMemcpyHostToDevice) != hipSuccess)
             return rec_->fail(HM_ERR_DEVICE, "level table upload");
@@ -1183,9 +1245,10 @@ class Level {
                     R.gq[a] = R.gi[a] = a < d_ ? g_ : 0;
                     R.dx[a] = dx_[a];
                 }
-                for (int e = 0; e < nq_; e++) R.Q[e] = patch_[p].Q[0] + size_t(e) * gvol(p);
+                const int out = s + 1 < nst_ ? stage_buf(s + 1) : 0;
+                for (int e = 0; e < nq_; e++) R.Q[e] = patch_[p].Q[out] + size_t(e) * gvol(p);
                 for (int m = 0; m <= s && m < kMaxRK; m++) {
-                    for (int e = 0; e < nq_; e++) R.Qi[m][e] = patch_[p].Q[1 + m] + size_t(e) * gvol(p);
+                    for (int e = 0; e < nq_; e++) R.Qi[m][e] = patch_[p].Q[stage_buf(m)] + size_t(e) * gvol(p);
                     for (int a = 0; a < d_; a++) R.Fi[m][a] = fl_[(size_t(p) * kMaxRK + m) * 3 + a];
                     if (diff_)
                         for (int a = 0; a < d_; a++) R.Fdi[m][a] = fdl_[(size_t(p) * kMaxRK + m) * 3 + a];
@@ -1217,6 +1280,7 @@ class Level {
             r.nz = five ? ns - 1 : 0;
             r.zfirst = five ? ns + d_ + 1 : 0;
             r.last_beta = -1;
+            r.s_first = five ? ns + d_ + 1 : neq_;  // only the volume fractions have a source
             r.ns = diff_ ? 1 : 0;  // Navier-Stokes form with the diffusive fluxes, else Euler
             for (int m = 0; m < kMaxRK; m++) {
                 r.alpha[m] = alpha_[s][m];
@@ -1228,6 +1292,7 @@ class Level {
         // the flux sums' terms of a whole step: stage by stage, intermediates in order
         step_terms_ = AccTerms{};
         step_terms_.neq = neq_;
+        step_terms_.init = 1;
         for (int s = 0; s < nst_; s++)
             for (int m = 0; m <= s; m++)
                 if (gamma_[s][m] != 0.0) {
@@ -1272,17 +1337,20 @@ class Level {
     int step(double dt, hipStream_t s, int record_slot = -1, int face_slot = -1, const double* dtp = nullptr) {
         if (int st = launch_halo(0, s)) return st;
         for (int sn = 0; sn < nst_; sn++) {
-            hipLaunchKernelGGL(k_copy_state, dim3(blocks_for(copy_items_)), dim3(kBlock), 0, s, copy_, 0, 1 + sn, nq_);
-            if (sn > 0)
-                if (int st = launch_halo(1 + sn, s)) return st;
+            const int buf = stage_buf(sn);
+            if (sn == 0 && buf != 0)
+                hipLaunchKernelGGL(k_copy_state, dim3(blocks_for(copy_items_)), dim3(kBlock), 0, s, copy_, 0, buf, nq_);
+            if (sn > 0) {
+                if (bare_items_ > 0)
+                    hipLaunchKernelGGL(k_copy_cells, dim3(blocks_for(bare_items_)), dim3(kBlock), 0, s, bare_,
+                                       bare_items_, patch_dev(), 0, buf, nq_);
+                if (int st = launch_halo(buf, s)) return st;
+            }
             if (record_slot >= 0)
-                if (int st = store_op(1 + sn, record_slot + sn, 0, s)) return st;
-            if (zero_items_ > 0)
-                hipLaunchKernelGGL(k_zero_source, dim3(blocks_for(zero_items_)), dim3(kBlock), 0, s, zero_, sn,
-                                   src_first_);
+                if (int st = store_op(buf, record_slot + sn, 0, s)) return st;
             if (hipGetLastError() != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "level launch failed");
             if (int st = rec_->runOwnedPlan(rhs_plan_[sn], dt, s, face_slot >= 0 ? face_states(face_slot + sn) : nullptr,
-                                            dtp))
+                                            dtp, true))
                 return st;
             if (diff_)
                 if (int st = diff_->runOwnedPlan(diff_plan_[sn], dt, s, dtp)) return st;
@@ -1478,17 +1546,14 @@ class Level {
         std::vector<double> h(size_t(neq_) * gvol(p), 0.0);
         if (hipDeviceSynchronize() != hipSuccess) return rec_->fail(HM_ERR_DEVICE, "device synchronize failed");
         double* dev = lam_base_[size_t(p) * (kMaxRK + 1) + nst_];
-        const int64_t vol = ivol(p);
         if (write) {
-            for (int c = 0; c < neq_; c++)
-                for (int64_t l = 0; l < vol; l++) h[size_t(c) * gvol(p) + gidx_of_interior(p, l)] = host[c * vol + l];
+            for_interior_rows(p, neq_, [&](int64_t l, int64_t gi, size_t b) { std::memcpy(&h[gi], host + l, b); });
             if (hipMemcpy(dev, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
                 return rec_->fail(HM_ERR_DEVICE, "adjoint upload failed");
         } else {
             if (hipMemcpy(h.data(), dev, h.size() * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
                 return rec_->fail(HM_ERR_DEVICE, "adjoint download failed");
-            for (int c = 0; c < neq_; c++)
-                for (int64_t l = 0; l < vol; l++) host[c * vol + l] = h[size_t(c) * gvol(p) + gidx_of_interior(p, l)];
+            for_interior_rows(p, neq_, [&](int64_t l, int64_t gi, size_t b) { std::memcpy(host + l, &h[gi], b); });
         }
         return HM_OK;
     }
@@ -1712,18 +1777,18 @@ class Level {
     bool has_bc_ = false;
     bool bc_bad_ = false;
     Schedule sched_{};  // schedule of the batched RHS plans
-    SegTableT<LevelPatch> copy_{}, zero_{};
+    SegTableT<LevelPatch> copy_{};
     SegTableT<RKPatch> rk_[kMaxRK] = {};
     SegTableT<RKPatch> acc_[kMaxRK] = {};
     int64_t acc_items_ = 0;
     void* acc_mem_ = nullptr;           // flux sums (enableFluxSums)
-    size_t acc_bytes_ = 0;
     std::vector<double*> facc_, sacc_;  // per patch and axis / per patch
     std::vector<double*> fdacc_;        // diffusive flux sums per patch and axis (Navier-Stokes form)
     AccTerms step_terms_{};             // gamma terms of one step's flux sums
     RKParams rkp_[kMaxRK] = {};
-    int64_t halo_items_ = 0, copy_items_ = 0, zero_items_ = 0, rk_items_ = 0;
-    int src_first_ = 0;  // first source component k_zero_source clears
+    int64_t halo_items_ = 0, copy_items_ = 0, bare_items_ = 0, rk_items_ = 0;
+    int first_buf_ = 0;              // state buffer of the first stage's intermediate (keepStartState)
+    const CellRef* bare_ = nullptr;  // ghost cells no fill covers
     size_t rk_off_ = 0;
     hipStream_t cap_stream_ = nullptr;
     hipEvent_t ev_a_ = nullptr, ev_b_ = nullptr;
@@ -1999,20 +2064,26 @@ __global__ __launch_bounds__(kBlock) void k_cf_fill(const CfItem* items, int64_t
 // (RungeKuttaLevelIntegrator::postprocessFluxAndSourceData,
 // RungeKuttaLevelIntegrator.cpp:2920-2967, 3060-3180; algs_upfluxsum2d.m4).
 // fsum holds [item][fine face j < 4][equation].
+//
+// The step's sum is formed here, from the fine stage fluxes, only on the faces
+// that are refluxed (the additions of k_rk_accumulate in its order): summing
+// every face of the fine level, and clearing the sums before, took 8 % of the
+// two-level step.
 __global__ __launch_bounds__(kBlock) void k_fsum_add(const RefluxItem* items, int64_t n_items,
-                                                     double* const* fine_facc, const int64_t* fine_fvol, int neq,
-                                                     double* fsum, int first) {
-    const int64_t t = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+                                                     const double* const* fine_f, AccTerms terms,
+                                                     const int64_t* fine_fvol, int neq, double* fsum, int first) {
+    // one thread per item, fine face and equation: its place in fsum
+    const int64_t gid = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    const int64_t r = gid / neq, t = r >> 2;
     if (t >= n_items) return;
-    const RefluxItem it = items[t];
-    const double* ff = fine_facc[it.fp * 3 + it.axis];
-    const int64_t fv = fine_fvol[it.fp * 3 + it.axis];
-    for (int j = 0; j < it.nf; j++)
-        for (int e = 0; e < neq; e++) {
-            double* o = fsum + (t * 4 + j) * neq + e;
-            const double v = ff[e * fv + it.fface[j]];
-            *o = first ? 0.0 + v : *o + v;
-        }
+    const int e = int(gid - r * neq), j = int(r & 3);
+    const RefluxItem& it = items[t];
+    if (j >= it.nf) return;
+    const double* const* ff = fine_f + (size_t(it.fp) * 3 + it.axis) * kMaxRK;
+    const int64_t at = e * fine_fvol[it.fp * 3 + it.axis] + it.fface[j];
+    double v = double(0);
+    for (int i = 0; i < terms.n; i++) v += terms.gamma[i] * ff[terms.src[i]][at];
+    fsum[gid] = first ? 0.0 + v : fsum[gid] + v;
 }
 
 // A coarse face on the coarse-fine boundary takes the area average of the
@@ -2127,7 +2198,7 @@ class Hierarchy {
                     return rec->fail(HM_ERR_INVALID_ARGUMENT, "fine patch boxes must start and end on coarse cells");
         g_ = c_->ghost();
         if (int st = c_->enableFluxSums()) return st;
-        if (int st = f_->enableFluxSums()) return st;
+        if (int st = c_->keepStartState()) return st;
         return build();
     }
 
@@ -2139,11 +2210,9 @@ class Hierarchy {
         if (int st = rec->selectDevice()) return st;
         const int d = c_->dim();
         for (int it = 0; it < nsteps; it++) {
-            if (int st = c_->clearFluxSums(s)) return st;
             if (int st = c_->stepOnce(dt, s)) return st;
             if (int st = c_->fillGhostsOf(0, s)) return st;  // the coarse state at the end of the step
             for (int k = 0; k < 2; k++) {
-                if (int st = f_->clearFluxSums(s)) return st;  // the fine step's own flux sums
                 // coarse-fine ghosts first: the fine step's own fill (same level,
                 // then the physical boundary conditions, which may read them) follows
                 if (ncf_ > 0) {
@@ -2156,11 +2225,11 @@ class Hierarchy {
                 }
                 if (int st = f_->stepOnce(0.5 * dt, s)) return st;
                 if (nrf_ > 0) {
-                    hipLaunchKernelGGL(k_fsum_add, dim3(blocks_for(nrf_)), dim3(kBlock), 0, s, rf_, nrf_, ffacc_, ffvol_,
-                                       c_->numEqn(), fsum_, int(k == 0));
+                    hipLaunchKernelGGL(k_fsum_add, dim3(blocks_for(nrf_ * 4 * c_->numEqn())), dim3(kBlock), 0, s, rf_, nrf_, ff_, f_->stepTerms(),
+                                       ffvol_, c_->numEqn(), fsum_, int(k == 0));
                     if (ns_)
-                        hipLaunchKernelGGL(k_fsum_add, dim3(blocks_for(nrf_)), dim3(kBlock), 0, s, rf_, nrf_, ffdacc_,
-                                           ffvol_, c_->numEqn(), fsumd_, int(k == 0));
+                        hipLaunchKernelGGL(k_fsum_add, dim3(blocks_for(nrf_ * 4 * c_->numEqn())), dim3(kBlock), 0, s, rf_, nrf_, ffd_,
+                                           f_->stepTerms(), ffvol_, c_->numEqn(), fsumd_, int(k == 0));
                 }
             }
             if (nrf_ > 0) {
@@ -2369,12 +2438,14 @@ class Hierarchy {
             for (int a = 0; a < d; a++) v *= c_->patchN(q)[a];
             sync.add(q, 0, v);
         }
-        std::vector<double*> ffacc(size_t(nfp) * 3, nullptr), ffdacc(size_t(nfp) * 3, nullptr);
+        std::vector<const double*> ff(size_t(nfp) * 3 * kMaxRK, nullptr), ffd(ff.size(), nullptr);  // [patch][axis][stage]
         std::vector<int64_t> ffvol(size_t(nfp) * 3, 0);
         for (int p = 0; p < nfp; p++)
             for (int a = 0; a < d; a++) {
-                ffacc[size_t(p) * 3 + a] = f_->fluxSum(p, a);
-                ffdacc[size_t(p) * 3 + a] = f_->diffusiveFluxSum(p, a);
+                for (int m = 0; m < kMaxRK; m++) {
+                    ff[(size_t(p) * 3 + a) * kMaxRK + m] = f_->stageFlux(p, m, a);
+                    if (ns_) ffd[(size_t(p) * 3 + a) * kMaxRK + m] = f_->stageDiffusiveFlux(p, m, a);
+                }
                 int64_t v = 1;
                 for (int b = 0; b < d; b++) v *= f_->patchN(p)[b] + (b == a);
                 ffvol[size_t(p) * 3 + a] = v;
@@ -2382,7 +2453,7 @@ class Hierarchy {
         const size_t fsum_bytes = up256(sizeof(double) * rf.size() * 4 * size_t(c_->numEqn()));
         const size_t bytes = up256(sizeof(CfItem) * cf.size()) + up256(sizeof(RefluxItem) * rf.size()) +
                              up256(sizeof(CoarsenItem) * cs.size()) + sync.bytes() +
-                             2 * up256(sizeof(double*) * ffacc.size()) + up256(sizeof(int64_t) * ffvol.size()) +
+                             2 * up256(sizeof(double*) * ff.size()) + up256(sizeof(int64_t) * ffvol.size()) +
                              fsum_bytes * (ns_ ? 2 : 1);
         if (hipMalloc(&mem_, bytes) != hipSuccess) {
             mem_ = nullptr;
@@ -2403,8 +2474,8 @@ class Hierarchy {
         sync_ = sync.write(h.data() + o, dv + o);
         sync_items_ = sync.total;
         o += sync.bytes();
-        ffacc_ = reinterpret_cast<double* const*>(put(ffacc.data(), sizeof(double*) * ffacc.size()));
-        ffdacc_ = reinterpret_cast<double* const*>(put(ffdacc.data(), sizeof(double*) * ffdacc.size()));
+        ff_ = reinterpret_cast<const double* const*>(put(ff.data(), sizeof(double*) * ff.size()));
+        ffd_ = reinterpret_cast<const double* const*>(put(ffd.data(), sizeof(double*) * ffd.size()));
         ffvol_ = reinterpret_cast<const int64_t*>(put(ffvol.data(), sizeof(int64_t) * ffvol.size()));
         fsum_ = reinterpret_cast<double*>(dv + o);  // written by k_fsum_add before it is read
         o += fsum_bytes;
@@ -2428,8 +2499,8 @@ class Hierarchy {
     const RefluxItem* rf_ = nullptr;
     const CoarsenItem* cs_ = nullptr;
     SegTableT<SyncPatch> sync_{};
-    double* const* ffacc_ = nullptr;
-    double* const* ffdacc_ = nullptr;  // the fine diffusive flux sums (Navier-Stokes form)
+    const double* const* ff_ = nullptr;   // the fine stage fluxes
+    const double* const* ffd_ = nullptr;  // the fine diffusive stage fluxes (Navier-Stokes form)
     const int64_t* ffvol_ = nullptr;
     double* fsum_ = nullptr;
     double* fsumd_ = nullptr;  // the fine diffusive flux sums over the coarse step

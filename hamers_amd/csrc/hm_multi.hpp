@@ -904,7 +904,8 @@ __global__ __launch_bounds__(kBlock) void k_source_five(W w, KParams k) {
 #pragma unroll
     for (int si = 0; si < NS - 1; si++) {
         const int e = NS + D + 1 + si;
-        P->S[e * svol + loc] += kdt(k) * P->Q[e][iq] * acc;
+        const double s0 = k.s_set ? double(0) : P->S[e * svol + loc];
+        P->S[e * svol + loc] = s0 + kdt(k) * P->Q[e][iq] * acc;
     }
 }
 

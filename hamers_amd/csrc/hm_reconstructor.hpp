@@ -122,6 +122,7 @@ class ConvectiveFluxReconstructorGPU {
         k_.lam_scale = 0.0;
         k_.qoff = 0;
         k_.xcd = 0;
+        k_.s_set = 0;
         k_.queue = nullptr;
         has_advective_ = (cfg.model == HM_MODEL_FIVE_EQN_ALLAIRE && cfg.num_species > 1);
         fused_ = (cfg.model == HM_MODEL_SINGLE_SPECIES);
@@ -410,20 +411,22 @@ class ConvectiveFluxReconstructorGPU {
 
     // All five stages of an owned plan; no profiling events (graph capture
     // safe).  wrec: face-state slot to record into (single-species model,
-    // plans built with wrec_off), NULL for none.
+    // plans built with wrec_off), NULL for none.  set_source: the advective
+    // source is written instead of accumulated.
     int runOwnedPlan(const OwnedPlan& p, double dt, hipStream_t s, double* wrec = nullptr,
-                     const double* dtp = nullptr) {
-        return runOwnedPlanStages(p, dt, 0, kStages, s, wrec, 0, dtp);
+                     const double* dtp = nullptr, bool set_source = false) {
+        return runOwnedPlanStages(p, dt, 0, kStages, s, wrec, 0, dtp, set_source);
     }
 
     // Pipeline stages [first, last) of an owned plan.
     int runOwnedPlanStages(const OwnedPlan& p, double dt, int first, int last, hipStream_t s, double* wrec = nullptr,
-                           int64_t qoff = 0, const double* dtp = nullptr) {
+                           int64_t qoff = 0, const double* dtp = nullptr, bool set_source = false) {
         KParams k = k_;
         k.dt = dt;
         k.dtp = dtp;
         k.wrec = wrec;
         k.qoff = qoff;
+        k.s_set = set_source ? 1 : 0;
         return run_stages(p.plan, k, s, first, last);
     }
 

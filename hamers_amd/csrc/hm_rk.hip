@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kBlock) void k_rk_update(W w, RKParams r) {
                 double t = -diff(0) / P->dx[0];
                 if constexpr (D > 1) t = t - diff(1) / P->dx[1];
                 if constexpr (D > 2) t = t - diff(2) / P->dx[2];
-                q += r.beta[n] * (t + P->Si[n][e * svol + loc]);
+                q += r.beta[n] * (t + (e >= r.s_first ? P->Si[n][e * svol + loc] : double(0)));
                 snap = q;
             }
         }
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kBlock) void k_rk_accumulate(W w, AccTerms t) {
     for (int e = 0; e < t.neq; e++) {
         double* acc = (ax == D) ? P->Sacc : P->Facc[ax];
         if (acc) {
-            double v = acc[e * vol + loc];
+            double v = t.init ? double(0) : acc[e * vol + loc];
             for (int i = 0; i < t.n; i++) {
                 const int n = t.src[i];
                 const double* src = (ax == D) ? P->Si[n] : P->Fi[n][ax];
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kBlock) void k_rk_accumulate(W w, AccTerms t) {
         }
         double* dacc = (ax == D) ? nullptr : P->Fdacc[ax];
         if (dacc) {
-            double v = dacc[e * vol + loc];
+            double v = t.init ? double(0) : dacc[e * vol + loc];
             for (int i = 0; i < t.n; i++) {
                 const int n = t.src[i];
                 if (!P->Fdi[n][ax]) continue;

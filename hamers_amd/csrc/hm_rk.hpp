@@ -30,6 +30,7 @@ struct RKParams {
     int zfirst;     // first volume-fraction equation (five-equation model)
     int nz;         // number of evolved volume fractions (0: no last-fraction update)
     int last_beta;  // index of the last nonzero beta, -1 if none
+    int s_first;    // equations below it have a zero source, which is not read (0: every source is read)
     int ns;         // some patch carries intermediate diffusive fluxes (Navier-Stokes form)
     double alpha[kMaxRK], beta[kMaxRK], gamma[kMaxRK];
 };
@@ -42,6 +43,7 @@ constexpr int kMaxAccTerms = kMaxRK * (kMaxRK + 1) / 2;
 struct AccTerms {
     int n;
     int neq;
+    int init;  // 1: the sums start at zero instead of the accumulated values
     int src[kMaxAccTerms];
     double gamma[kMaxAccTerms];
 };

@@ -197,12 +197,12 @@ struct SegTableT {  // many patches: device arrays
 };
 
 // Block lookup: the segment of the block's first item and the number of whole
-// 256-item blocks before it in the segment, for stages whose segments are whole
-// blocks.  Everything is block-uniform (scalar loads and registers).
-template <class T>
+// blocks of NB items before it in the segment, for stages whose segments are
+// whole blocks.  Everything is block-uniform (scalar loads and registers).
+template <int NB = kBlock, class T>
 __device__ __forceinline__ bool find_block(const SegTableT<T>& w, uint32_t block, const T*& P, int& seg_axis,
                                            uint32_t& tile) {
-    const int64_t first = int64_t(block) * kBlock;
+    const int64_t first = int64_t(block) * NB;
     const int64_t* start = as_constant(w.start);
     if (first >= start[w.nseg]) return false;
     int lo = 0, hi = w.nseg - 1;  // last segment with start <= first
@@ -213,21 +213,21 @@ __device__ __forceinline__ bool find_block(const SegTableT<T>& w, uint32_t block
         else
             hi = mid - 1;
     }
-    tile = uint32_t((first - start[lo]) / kBlock);
+    tile = uint32_t((first - start[lo]) / NB);
     const int pd = *as_constant(w.seg + lo);
     P = as_constant(w.patches + (pd >> 2));
     seg_axis = pd & 3;
     return true;
 }
 
-template <class T>
+template <int NB = kBlock, class T>
 __device__ __forceinline__ bool find_block(const SegSingleT<T>& w, uint32_t block, const T*& P, int& seg_axis,
                                            uint32_t& tile) {
-    const int64_t first = int64_t(block) * kBlock;
+    const int64_t first = int64_t(block) * NB;
     if (first >= w.start[w.nseg]) return false;
     int s = 0;
     while (s + 1 < w.nseg && first >= w.start[s + 1]) s++;
-    tile = uint32_t((first - w.start[s]) / kBlock);
+    tile = uint32_t((first - w.start[s]) / NB);
     P = &w.p;
     seg_axis = s;
     return true;

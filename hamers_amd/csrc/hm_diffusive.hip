@@ -35,22 +35,39 @@ __device__ __forceinline__ int64_t dq_idx(const DiffPatch& P, int i, int j, int 
     return (i + P.gq[0]) + int64_t(j + gy) * e0 + int64_t(k + gz) * e0 * e1;
 }
 
-// Component slots of the derived cell data.
+// Component slots of the derived cell data: only what the node fluxes
+// differentiate, and the pressure.  The density is the sum of the caller's
+// partial densities, and the enthalpies and the mixture's transport
+// coefficients follow from Y_i, p and T where a node uses them.  Bound by HBM:
+// twelve stored components instead of seven took 1.06 ms on a level of 448
+// uneven patches, now 0.73 (5.6 TB/s).
 template <int D, int NS>
 struct DiffSlots {
-    static constexpr int RHO = 0, Y = 1, U = 1 + NS, T = 1 + NS + D, H = 2 + NS + D, MU = 2 + 2 * NS + D,
-                         MUV = 3 + 2 * NS + D, KAP = 4 + 2 * NS + D;
+    static constexpr int Y = 0, U = NS, T = NS + D, P = NS + D + 1;
 };
 
-// Cells of the 6-ghost box: density, mass fractions, velocity, pressure of the
+// Element i of one component.  The diffusive flux takes patches of up to 2^31
+// cells, so the byte offset does not fit the 32 bits of ldg.
+__device__ __forceinline__ double ldw(const double* base, uint32_t i) {
+    typedef __attribute__((address_space(1))) const double gdouble;
+    return ((gdouble*)base)[i];
+}
+__device__ __forceinline__ void stw(double* base, uint32_t i, double v) {
+    typedef __attribute__((address_space(1))) double gdouble;
+    ((gdouble*)base)[i] = v;
+}
+
+// Block numbers are XCD-contiguous in both kernels: the rows that neighbouring
+// blocks' stencils share then sit in one L2.
+__device__ __forceinline__ uint32_t diff_block() { return xcd_block(blockIdx.x, gridDim.x); }
+
+// Cells of the 6-ghost box: mass fractions, velocity, pressure of the
 // four-equation model (FlowModelFourEqnConservative.cpp:5034-5086), temperature
-// p / ((gamma - 1) c_v rho) (EquationOfStateIdealGas.cpp:6951), species
-// densities p / (R_i T) (:8357) and enthalpies gamma_i p / ((gamma_i - 1) rho_i)
-// (:6464), mixture viscosities and conductivity sum(x_i w_i) / sum(w_i),
-// w_i = Y_i / sqrt(M_i) (EquationOfShearViscosityMixingRulesConstant.cpp:497-528).
+// p / ((gamma - 1) c_v rho) (EquationOfStateIdealGas.cpp:6951).  Quotients
+// through quot / div_rn round as the divisions do.
 template <int D, int NS, class W>
 __global__ __launch_bounds__(kBlock) void k_diff_cells(W w, DParams k) {
-    const int64_t gid = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    const int64_t gid = int64_t(diff_block()) * kBlock + threadIdx.x;
     const DiffPatch* P;
     int ax;
     int64_t loc;
@@ -62,16 +79,20 @@ __global__ __launch_bounds__(kBlock) void k_diff_cells(W w, DParams k) {
     const int i = int(uint32_t(loc) - r * uint32_t(e0)) - kGd;
     const int j = (D > 1) ? int((D > 2) ? r % uint32_t(e1) : r) - kGd : 0;
     const int kk = (D > 2) ? int(r / uint32_t(e1)) - kGd : 0;
-    const int64_t iq = dq_idx<D>(*P, i, j, kk);
+    const uint32_t iq = uint32_t(dq_idx<D>(*P, i, j, kk));
+    double q[NS + D + 1];
+#pragma unroll
+    for (int e = 0; e < NS + D + 1; e++) q[e] = ldw(P->Q[e], iq);
     double rho = double(0);
     double Y[NS];
 #pragma unroll
-    for (int si = 0; si < NS; si++) rho += P->Q[si][iq];
+    for (int si = 0; si < NS; si++) rho += q[si];
+    const double rrho = rcp_rn(rho);
 #pragma unroll
-    for (int si = 0; si < NS; si++) Y[si] = P->Q[si][iq] / rho;
+    for (int si = 0; si < NS; si++) Y[si] = quot(q[si], rho, rrho);
     double u[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int b = 0; b < D; b++) u[b] = P->Q[NS + b][iq] / rho;
+    for (int b = 0; b < D; b++) u[b] = quot(q[NS + b], rho, rrho);
     double ke;
     if constexpr (D == 1)
         ke = u[0] * u[0];
@@ -79,115 +100,95 @@ __global__ __launch_bounds__(kBlock) void k_diff_cells(W w, DParams k) {
         ke = u[0] * u[0] + u[1] * u[1];
     else
         ke = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-    const double E = P->Q[NS + D][iq];
-    const double eps_int = E / rho - double(1) / double(2) * ke;
+    const double eps_int = quot(q[NS + D], rho, rrho) - double(1) / double(2) * ke;
     double c_p = double(0), c_v = double(0);
 #pragma unroll
     for (int si = 0; si < NS; si++) {
         c_p += Y[si] * k.cp[si];
         c_v += Y[si] * k.cv[si];
     }
-    const double gmix = c_p / c_v;
+    const double gmix = div_rn(c_p, c_v);
     const double p = (gmix - double(1)) * rho * eps_int;
-    const double T = p / ((gmix - double(1)) * c_v * rho);
+    const double T = div_rn(p, (gmix - double(1)) * c_v * rho);
     const int64_t vol = dvol<D>(*P);
-    const int64_t c = dcell<D>(*P, i, j, kk);
+    const uint32_t c = uint32_t(loc);  // the segment numbers the box's cells
     double* out = P->cell;
-    double mu_n = double(0), mu_d = double(0), mv_n = double(0), mv_d = double(0), ka_n = double(0),
-           ka_d = double(0);
 #pragma unroll
-    for (int si = 0; si < NS; si++) {
-        const double rho_i = p / (k.R[si] * T);
-        out[(S::H + si) * vol + c] = k.gamma[si] * p / ((k.gamma[si] - double(1)) * rho_i);
-        const double wgt = Y[si] * k.wfac[si];
-        mu_n += k.mu[si] * wgt;
-        mu_d += wgt;
-        mv_n += k.mu_v[si] * wgt;
-        mv_d += wgt;
-        ka_n += k.kappa[si] * wgt;
-        ka_d += wgt;
-    }
-    out[S::RHO * vol + c] = rho;
+    for (int si = 0; si < NS; si++) stw(out + (S::Y + si) * vol, c, Y[si]);
 #pragma unroll
-    for (int si = 0; si < NS; si++) out[(S::Y + si) * vol + c] = Y[si];
-#pragma unroll
-    for (int b = 0; b < D; b++) out[(S::U + b) * vol + c] = u[b];
-    out[S::T * vol + c] = T;
-    out[S::MU * vol + c] = mu_n / mu_d;
-    out[S::MUV * vol + c] = mv_n / mv_d;
-    out[S::KAP * vol + c] = ka_n / ka_d;
+    for (int b = 0; b < D; b++) stw(out + (S::U + b) * vol, c, u[b]);
+    stw(out + S::T * vol, c, T);
+    stw(out + S::P * vol, c, p);
 }
 
-// Sixth-order central first derivative along axis B of cell-data component
-// `comp` at cell c (DiffusiveFluxReconstructorNodeSixthOrder.cpp:77-112).
-__device__ __forceinline__ double deriv6(const double* f, int64_t c, int64_t st, double dxinv) {
+// Node fluxes of axis A at the cell of index c in the 6-ghost box and q in the
+// caller's; col[comp * kDTile + m * step] holds component comp (Y, u, T) of the
+// cell m along A.  Per equation, the terms of derivative axes b = 0..D-1 in the
+// reference's order, each diffusivity * derivative added to a sum that starts
+// at zero (DiffusiveFluxReconstructorNode.cpp:920-1070), from sixth-order
+// central first derivatives (DiffusiveFluxReconstructorNodeSixthOrder.cpp:
+// 77-112).  Species densities p / (R_i T) (EquationOfStateIdealGas.cpp:8357),
+// enthalpies gamma_i p / ((gamma_i - 1) rho_i) (:6464), mixture viscosities and
+// conductivity sum(x_i w_i) / sum(w_i), w_i = Y_i / sqrt(M_i)
+// (EquationOfShearViscosityMixingRulesConstant.cpp:497-528).
+template <int D, int NS, int A>
+__device__ __forceinline__ void diff_node(const DiffPatch& P, uint32_t c, uint32_t q, const DParams& k,
+                                          const double* col, int step, double (&Fn)[NS + D + 1]) {
+    using S = DiffSlots<D, NS>;
+    const int64_t vol = dvol<D>(P);
+    const int64_t st[3] = {1, dext<D>(P, 0), int64_t(dext<D>(P, 0)) * dext<D>(P, 1)};
+    const double* cd = P.cell;
+    auto at = [&](int comp, int64_t shift) { return ldw(cd + (comp * vol + shift), c); };
     const double a_n = double(3) / double(4);
     const double b_n = -double(3) / double(20);
     const double c_n = double(1) / double(60);
-    return (a_n * (f[c + st] - f[c - st]) + b_n * (f[c + 2 * st] - f[c - 2 * st]) +
-            c_n * (f[c + 3 * st] - f[c - 3 * st])) *
-           dxinv;
-}
-
-// Node fluxes of axis A on nodes [-3, n_A + 3) x interior: per equation, the
-// terms of derivative axes b = 0..D-1 in the reference's order, each
-// diffusivity * derivative added to a sum that starts at zero
-// (DiffusiveFluxReconstructorNode.cpp:920-1070).
-template <int D, int NS, class W>
-__global__ __launch_bounds__(kBlock) void k_diff_nodes(W w, DParams k) {
-    const int64_t gid = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    const DiffPatch* P;
-    int A;
-    int64_t loc;
-    if (!w.find(gid, P, A, loc)) return;
-    using S = DiffSlots<D, NS>;
-    constexpr int NEQ = NS + D + 1;
-    int ext[3];
+    auto along = [&](int comp, int m) { return col[comp * kDTile + m * step]; };
+    auto deriv6 = [&](int comp, int b) {
+        if (b == A)
+            return (a_n * (along(comp, 1) - along(comp, -1)) + b_n * (along(comp, 2) - along(comp, -2)) +
+                    c_n * (along(comp, 3) - along(comp, -3))) *
+                   P.dxinv[b];
+        return (a_n * (at(comp, st[b]) - at(comp, -st[b])) + b_n * (at(comp, 2 * st[b]) - at(comp, -2 * st[b])) +
+                c_n * (at(comp, 3 * st[b]) - at(comp, -3 * st[b]))) *
+               P.dxinv[b];
+    };
+    double rho = double(0);
 #pragma unroll
-    for (int b = 0; b < 3; b++) ext[b] = (b < D) ? P->n[b] + ((b == A) ? 6 : 0) : 1;
-    int idx[3];
-    // 32-bit index arithmetic (a work segment has fewer than 2^31 items).
-    const uint32_t r = uint32_t(loc) / uint32_t(ext[0]);
-    idx[0] = int(uint32_t(loc) - r * uint32_t(ext[0]));
-    idx[1] = int(r % uint32_t(ext[1]));
-    idx[2] = int(r / uint32_t(ext[1]));
-    idx[A] -= 3;
-    const int64_t c = dcell<D>(*P, idx[0], idx[1], idx[2]);
-    const int64_t vol = dvol<D>(*P);
-    int64_t st[3];
-    st[0] = 1;
-    st[1] = dext<D>(*P, 0);
-    st[2] = int64_t(dext<D>(*P, 0)) * dext<D>(*P, 1);
-    const double* cd = P->cell;
-    const double rho = cd[S::RHO * vol + c];
-    const double mu = cd[S::MU * vol + c];
-    const double mu_v = cd[S::MUV * vol + c];
+    for (int si = 0; si < NS; si++) rho += ldw(P.Q[si], q);
+    const double p = at(S::P, 0), T = along(S::T, 0);
     double Y[NS], h[NS], u[D];
+    double mu_n = double(0), mv_n = double(0), ka_n = double(0), w_d = double(0);
 #pragma unroll
     for (int si = 0; si < NS; si++) {
-        Y[si] = cd[(S::Y + si) * vol + c];
-        h[si] = cd[(S::H + si) * vol + c];
+        Y[si] = along(S::Y + si, 0);
+        const double rho_i = div_rn(p, k.R[si] * T);
+        h[si] = div_rn(k.gamma[si] * p, (k.gamma[si] - double(1)) * rho_i);
+        const double wgt = Y[si] * k.wfac[si];
+        mu_n += k.mu[si] * wgt;
+        mv_n += k.mu_v[si] * wgt;
+        ka_n += k.kappa[si] * wgt;
+        w_d += wgt;
     }
+    const double rw = rcp_rn(w_d);
+    const double mu = quot(mu_n, w_d, rw), mu_v = quot(mv_n, w_d, rw), kap = quot(ka_n, w_d, rw);
 #pragma unroll
-    for (int b = 0; b < D; b++) u[b] = cd[(S::U + b) * vol + c];
+    for (int b = 0; b < D; b++) u[b] = along(S::U + b, 0);
 
     // Derivatives along A of Y_i, u_c, T; along b != A of u_A and u_b.
-    const double dA = P->dxinv[A];
     double dY[NS], dU[D], dT;
 #pragma unroll
-    for (int si = 0; si < NS; si++) dY[si] = deriv6(cd + (S::Y + si) * vol, c, st[A], dA);
+    for (int si = 0; si < NS; si++) dY[si] = deriv6(S::Y + si, A);
 #pragma unroll
-    for (int b = 0; b < D; b++) dU[b] = deriv6(cd + (S::U + b) * vol, c, st[A], dA);
-    dT = deriv6(cd + S::T * vol, c, st[A], dA);
+    for (int b = 0; b < D; b++) dU[b] = deriv6(S::U + b, A);
+    dT = deriv6(S::T, A);
     double dUa[3] = {0.0, 0.0, 0.0}, dUb[3] = {0.0, 0.0, 0.0};  // d u_A / dx_b, d u_b / dx_b
 #pragma unroll
     for (int b = 0; b < D; b++) {
         if (b == A) continue;
-        dUa[b] = deriv6(cd + (S::U + A) * vol, c, st[b], P->dxinv[b]);
-        dUb[b] = deriv6(cd + (S::U + b) * vol, c, st[b], P->dxinv[b]);
+        dUa[b] = deriv6(S::U + A, b);
+        dUb[b] = deriv6(S::U + b, b);
     }
 
-    double Fn[NEQ];
     // Mass equations: -rho D_si dY_si + sum_j rho Y_si D_sj dY_sj (derivative along A only).
 #pragma unroll
     for (int si = 0; si < NS; si++) {
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(kBlock) void k_diff_nodes(W w, DParams k) {
                     else
                         acc += -u[cc] * mu * dU[cc];
                 }
-                acc += -cd[S::KAP * vol + c] * dT;
+                acc += -kap * dT;
 #pragma unroll
                 for (int si = 0; si < NS; si++) {
                     acc += -rho * k.D[si] * h[si] * dY[si];
@@ -246,82 +247,112 @@ __global__ __launch_bounds__(kBlock) void k_diff_nodes(W w, DParams k) {
         }
         Fn[NS + D] = acc;
     }
-    int64_t nvol = 1;
-#pragma unroll
-    for (int b = 0; b < 3; b++) nvol *= ext[b];
-    double* out = P->fnode[A];
-#pragma unroll
-    for (int e = 0; e < NEQ; e++) out[e * nvol + loc] = Fn[e];
 }
 
-// Face fluxes of axis A (DiffusiveFluxReconstructorNodeSixthOrder.cpp:507-690):
+// Diffusive flux of axis A over one tile (dtile_shape): R consecutive cells
+// along A of W columns, one per thread, staged in LDS (Y, u, T), so that the
+// derivatives along A read LDS.  The threads of the cells 3 from either end form
+// node fluxes, which then take the cells' places, and the threads with three
+// nodes below and two above the output faces
+// (DiffusiveFluxReconstructorNodeSixthOrder.cpp:507-690):
 // F_face = 0 + dt (a_r (F_L + F_R) + b_r (F_LL + F_RR) + c_r (F_LLL + F_RRR)).
-template <int D, int NS, class W>
-__global__ __launch_bounds__(kBlock) void k_diff_faces(W w, DParams k) {
-    const int64_t gid = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    const DiffPatch* P;
-    int A;
-    int64_t loc;
-    if (!w.find(gid, P, A, loc)) return;
+// Every output face has one such thread.  Bound by the caches' load rate: with
+// node fluxes to memory and a second kernel the pair took 2.75 + 1.47 ms on a
+// level of 448 uneven patches (Navier-Stokes, 6-cell halos) and moved 13 GB;
+// fused with every derivative from memory 3.09 ms, now 2.66.  Blocks of 512 threads keep a
+// tile's rows 6 to 15 cells wide, XCD-contiguous blocks the lines at their edges
+// in one L2.
+template <int D, int NS, int A>
+__device__ __forceinline__ void diff_tile(const DiffPatch& P, uint32_t tile, const DParams& k, double* lds) {
     constexpr int NEQ = NS + D + 1;
-    int fext[3], next[3];
+    const int nA = P.n[A];
+    const int R = P.tile[A][0], W = P.tile[A][1], ntA = P.tile[A][2];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
+    const uint32_t first = small_div(lane, uint32_t(P.tile[A][3]));  // lane / R on axis 0, lane / W on the others
+    const uint32_t rest = lane - first * uint32_t(A == 0 ? R : W);
+    const uint32_t r = A == 0 ? rest : first, w = A == 0 ? first : rest;
+    const int x = int(tA) * (R - 11) - 6 + int(r);  // cell along A
+    constexpr int U = (A == 0) ? 1 : 0;  // first axis across
+    constexpr int V = (A == 2) ? 1 : 2;  // second axis across
+    uint32_t cu, tv;
+    tile_column(tw * uint32_t(W), w, uint32_t(W), uint32_t(D > U ? P.n[U] : 1), cu, tv);
+    const bool in = lane < uint32_t(R * W) && x < nA + 6 && tv < uint32_t(D > V ? P.n[V] : 1);
+    int i[3];
+    i[A] = x;
+    i[U] = int(cu);
+    i[V] = int(tv);
+    const int step = A == 0 ? 1 : W;  // thread distance of neighbouring rows
+    const uint32_t c = uint32_t(dcell<D>(P, i[0], i[1], i[2]));
+    const int64_t vol = dvol<D>(P);
+    if (in) {
 #pragma unroll
-    for (int b = 0; b < 3; b++) {
-        fext[b] = (b < D) ? P->n[b] + ((b == A) ? 1 : 0) : 1;
-        next[b] = (b < D) ? P->n[b] + ((b == A) ? 6 : 0) : 1;
+        for (int e = 0; e < NEQ; e++) lds[e * kDTile + lane] = ldw(P.cell + e * vol, c);  // Y, u, T
     }
-    int idx[3];
-    // 32-bit index arithmetic (a work segment has fewer than 2^31 items).
-    const uint32_t r = uint32_t(loc) / uint32_t(fext[0]);
-    idx[0] = int(uint32_t(loc) - r * uint32_t(fext[0]));
-    idx[1] = int(r % uint32_t(fext[1]));
-    idx[2] = int(r / uint32_t(fext[1]));
-    // node of cell m along A sits at m + 3; the face f reads cells f-3 .. f+2
-    idx[A] += 3;
-    const int64_t nst = (A == 0) ? 1 : (A == 1) ? int64_t(next[0]) : int64_t(next[0]) * next[1];
-    const int64_t n0 = idx[0] + int64_t(idx[1]) * next[0] + int64_t(idx[2]) * next[0] * next[1];
-    const int64_t nvol = int64_t(next[0]) * next[1] * next[2];
-    const int64_t fvol = int64_t(fext[0]) * fext[1] * fext[2];
+    __syncthreads();
+    const bool node = in && int(r) >= 3 && int(r) < R - 3 && x < nA + 3;
+    double Fn[NEQ];
+    if (node)
+        diff_node<D, NS, A>(P, c, uint32_t(dq_idx<D>(P, i[0], i[1], i[2])), k, lds + lane, step, Fn);
+    __syncthreads();
+    if (node) {
+#pragma unroll
+        for (int e = 0; e < NEQ; e++) lds[e * kDTile + lane] = Fn[e];
+    }
+    __syncthreads();
+    if (!in || int(r) < 6 || int(r) > R - 6 || x > nA) return;  // face x: nodes x - 3 .. x + 2
+    const uint32_t f0 = uint32_t(P.n[0] + (A == 0)), f1 = uint32_t(D > 1 ? P.n[1] + (A == 1) : 1);
+    const uint32_t fi = uint32_t(i[0]) + f0 * (uint32_t(i[1]) + f1 * uint32_t(i[2]));
+    const int64_t fvol = int64_t(f0) * f1 * (D > 2 ? P.n[2] + (A == 2) : 1);
     const double a_n = double(3) / double(4);
     const double b_n = -double(3) / double(20);
     const double c_n = double(1) / double(60);
     const double a_r = a_n + b_n + c_n;
     const double b_r = b_n + c_n;
     const double c_r = c_n;
-    const double* Fn = P->fnode[A];
-    double* out = P->F[A];
+    double* out = P.F[A];
     const double dt = k.dtp ? *k.dtp : k.dt;
 #pragma unroll
     for (int e = 0; e < NEQ; e++) {
-        const double* f = Fn + e * nvol + n0;
+        auto f = [&](int m) { return lds[e * kDTile + int(lane) + m * step]; };
         double acc = double(0);
-        acc += dt * (a_r * (f[-nst] + f[0]) + b_r * (f[-2 * nst] + f[nst]) + c_r * (f[-3 * nst] + f[2 * nst]));
-        out[e * fvol + loc] = acc;
+        acc += dt * (a_r * (f(-1) + f(0)) + b_r * (f(-2) + f(1)) + c_r * (f(-3) + f(2)));
+        stw(out + e * fvol, fi, acc);
     }
 }
 
-template <class W>
-unsigned dblocks(const DPlan<W>& plan, int stage) {
-    return unsigned((plan.items[stage] + kBlock - 1) / kBlock);
+template <int D, int NS, class W>
+__global__ __launch_bounds__(kDTile) void k_diff_flux(W w, DParams k) {
+    __shared__ double lds[(NS + D + 1) * kDTile];
+    const DiffPatch* P;
+    int A;
+    uint32_t tile;
+    if (!find_block<kDTile>(w, diff_block(), P, A, tile)) return;  // whole blocks
+    if (A == 0) {
+        diff_tile<D, NS, 0>(*P, tile, k, lds);
+    } else if constexpr (D > 1) {
+        if (A == 1) {
+            diff_tile<D, NS, 1>(*P, tile, k, lds);
+        } else if constexpr (D > 2) {
+            diff_tile<D, NS, 2>(*P, tile, k, lds);
+        }
+    }
 }
 
 template <int D, int NS, class W>
-hipError_t launch_dn(const DPlan<W>& plan, const DParams& k, hipStream_t s, int first, int last) {
-    if (first <= 0 && last > 0 && plan.items[0] > 0)
-        hipLaunchKernelGGL((k_diff_cells<D, NS, W>), dim3(dblocks(plan, 0)), dim3(kBlock), 0, s, plan.work[0], k);
-    if (first <= 1 && last > 1 && plan.items[1] > 0)
-        hipLaunchKernelGGL((k_diff_nodes<D, NS, W>), dim3(dblocks(plan, 1)), dim3(kBlock), 0, s, plan.work[1], k);
-    if (first <= 2 && last > 2 && plan.items[2] > 0)
-        hipLaunchKernelGGL((k_diff_faces<D, NS, W>), dim3(dblocks(plan, 2)), dim3(kBlock), 0, s, plan.work[2], k);
+hipError_t launch_dn(const DPlan<W>& plan, const DParams& k, hipStream_t s) {
+    const unsigned cells = unsigned((plan.items[0] + kBlock - 1) / kBlock), tiles = unsigned(plan.items[1] / kDTile);
+    if (cells) hipLaunchKernelGGL((k_diff_cells<D, NS, W>), dim3(cells), dim3(kBlock), 0, s, plan.work[0], k);
+    if (tiles) hipLaunchKernelGGL((k_diff_flux<D, NS, W>), dim3(tiles), dim3(kDTile), 0, s, plan.work[1], k);
     return hipGetLastError();
 }
 
 template <int D, class W>
-hipError_t launch_d(const DPlan<W>& plan, const DParams& k, hipStream_t s, int first, int last) {
+hipError_t launch_d(const DPlan<W>& plan, const DParams& k, hipStream_t s) {
     switch (k.num_species) {
-        case 1: return launch_dn<D, 1, W>(plan, k, s, first, last);
-        case 2: return launch_dn<D, 2, W>(plan, k, s, first, last);
-        case 3: return launch_dn<D, 3, W>(plan, k, s, first, last);
+        case 1: return launch_dn<D, 1, W>(plan, k, s);
+        case 2: return launch_dn<D, 2, W>(plan, k, s);
+        case 3: return launch_dn<D, 3, W>(plan, k, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -329,20 +360,19 @@ hipError_t launch_d(const DPlan<W>& plan, const DParams& k, hipStream_t s, int f
 }  // namespace
 
 template <class W>
-hipError_t launch_diffusive_four(int dim, const DPlan<W>& plan, const DParams& k, hipStream_t s, int first,
-                                 int last) {
+hipError_t launch_diffusive_four(int dim, const DPlan<W>& plan, const DParams& k, hipStream_t s) {
     switch (dim) {
-        case 1: return launch_d<1, W>(plan, k, s, first, last);
-        case 2: return launch_d<2, W>(plan, k, s, first, last);
-        case 3: return launch_d<3, W>(plan, k, s, first, last);
+        case 1: return launch_d<1, W>(plan, k, s);
+        case 2: return launch_d<2, W>(plan, k, s);
+        case 3: return launch_d<3, W>(plan, k, s);
         default: return hipErrorInvalidValue;
     }
 }
 
 template hipError_t launch_diffusive_four<SegSingleT<DiffPatch>>(int, const DPlan<SegSingleT<DiffPatch>>&,
-                                                                 const DParams&, hipStream_t, int, int);
+                                                                 const DParams&, hipStream_t);
 template hipError_t launch_diffusive_four<SegTableT<DiffPatch>>(int, const DPlan<SegTableT<DiffPatch>>&,
-                                                                const DParams&, hipStream_t, int, int);
+                                                                const DParams&, hipStream_t);
 
 }  // namespace hm
 

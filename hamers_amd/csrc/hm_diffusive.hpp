@@ -9,10 +9,11 @@
 // reports failures through it.
 //
 // Pipeline (per call, all patches at once on the batched path):
-//   k_diff_cells  cells of the 6-ghost box: rho, Y_i, u, T, h_i, mu, mu_v, kappa
-//   k_diff_nodes  node fluxes F_node[e] = sum_b sum_terms D * d(var)/dx_b on the
-//                 nodes [-3, n_a + 3) along each axis a
-//   k_diff_faces  face fluxes dt (a_r (F_L + F_R) + b_r (F_LL + F_RR) + c_r (F_LLL + F_RRR))
+//   k_diff_cells  cells of the 6-ghost box: Y_i, u, T, p
+//   k_diff_flux   over tiles of whole columns: node fluxes F_node[e] = sum_b
+//                 sum_terms D * d(var)/dx_b on the nodes [-3, n_a + 3) along
+//                 each axis a, kept in LDS, and from them the face fluxes
+//                 dt (a_r (F_L + F_R) + b_r (F_LL + F_RR) + c_r (F_LLL + F_RRR))
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,7 +29,22 @@
 namespace hm {
 
 constexpr int kGd = 6;  // diffusive ghost width (DiffusiveFluxReconstructorNodeSixthOrder.cpp:22)
-constexpr int kDiffStages = 3;
+constexpr int kDiffStages = 2;
+
+// Tile of the diffusive flux (k_diff_flux): a block of kDTile threads takes R
+// consecutive cells along the axis by W columns (R W <= kDTile) and outputs
+// R - 11 faces of each column (a face takes six nodes, a node seven cells).  A
+// column of n_A + 12 cells (n_A + 1 faces) takes ntA tiles of equal length that
+// share eleven cells, of at most 74 faces in 2D and 3D (W >= 6 columns, so that
+// a row of them is most of a cache line), of as many as the block holds in 1D.
+constexpr int kDTile = 512;
+
+inline void dtile_shape(int dim, int nA, int& R, int& W, int& ntA) {
+    const int most = dim == 1 ? kDTile - 11 : 74;
+    ntA = (nA + 1 + most - 1) / most;
+    R = (nA + 1 + ntA - 1) / ntA + 11;
+    W = kDTile / R;
+}
 
 struct DiffPatch {
     int n[3];                     // interior extents (1 on unused axes)
@@ -37,7 +53,7 @@ struct DiffPatch {
     const double* Q[HM_MAX_EQN];  // conservative variables over the Q ghost box
     double* F[3];                 // output diffusive flux per axis (component-major)
     double* cell;                 // scratch: derived cell data over the 6-ghost box
-    double* fnode[3];             // scratch: node fluxes per axis, neq comps over (n_a+6) x n_b
+    int tile[3][4];               // dtile_shape of each axis, and small_div_mul of a tile row
 };
 
 struct DParams {
@@ -62,8 +78,7 @@ struct DPlan {
 };
 
 template <class W>
-hipError_t launch_diffusive_four(int dim, const DPlan<W>& plan, const DParams& k, hipStream_t s, int first,
-                                 int last);
+hipError_t launch_diffusive_four(int dim, const DPlan<W>& plan, const DParams& k, hipStream_t s);
 
 class DiffusiveFluxReconstructorGPU {
    public:
@@ -107,7 +122,7 @@ class DiffusiveFluxReconstructorGPU {
         const Layout L = layout(v);
         if (order_.enter(s) != hipSuccess) return rec_.fail(HM_ERR_DEVICE, "hipStreamWaitEvent failed");
         if (int st = ensure_arena(L.total, s)) return st;
-        const DiffPatch p = make_patch(v, arena_, L);
+        const DiffPatch p = make_patch(v, arena_);
         DPlan<SegSingleT<DiffPatch>> plan{};
         const int d = rec_.config().dim;
         const Ext e = extents(v);
@@ -118,7 +133,7 @@ class DiffusiveFluxReconstructorGPU {
             const int nseg = (stage == 0) ? 1 : d;
             for (int a = 0; a < nseg; a++) {
                 w.start[a] = acc;
-                w.cnt[a] = (stage == 0) ? e.cells : (stage == 1) ? e.nodes[a] : e.faces[a];
+                w.cnt[a] = (stage == 0) ? e.cells : e.tiles[a];
                 acc += (w.cnt[a] + kSegAlign - 1) / kSegAlign * kSegAlign;
             }
             w.nseg = nseg;
@@ -195,10 +210,10 @@ class DiffusiveFluxReconstructorGPU {
     }
 
     struct Ext {
-        int64_t cells, nodes[3], faces[3];
+        int64_t cells, tiles[3];  // items of the two stages
     };
     struct Layout {
-        size_t cell, fnode[3], total;
+        size_t cell, total;
     };
     struct CachedPlan {
         std::vector<hm_patch_view> views;
@@ -208,8 +223,8 @@ class DiffusiveFluxReconstructorGPU {
         uint64_t use = 0;
     };
 
-    // Derived components per cell: rho, Y_i, u (dim), T, h_i, mu, mu_v, kappa.
-    int cell_comps() const { return 2 * k_.num_species + rec_.config().dim + 5; }
+    // Derived components per cell: Y_i, u (dim), T, p.
+    int cell_comps() const { return k_.num_species + rec_.config().dim + 2; }
 
     Ext extents(const hm_patch_view& v) const {
         const int d = rec_.config().dim;
@@ -217,15 +232,14 @@ class DiffusiveFluxReconstructorGPU {
         e.cells = 1;
         for (int a = 0; a < d; a++) e.cells *= v.n[a] + 2 * kGd;
         for (int a = 0; a < 3; a++) {
-            e.nodes[a] = e.faces[a] = 0;
+            e.tiles[a] = 0;
             if (a >= d) continue;
-            int64_t m = 1, f = 1;
-            for (int b = 0; b < d; b++) {
-                m *= (b == a) ? v.n[b] + 6 : v.n[b];
-                f *= (b == a) ? v.n[b] + 1 : v.n[b];
-            }
-            e.nodes[a] = m;
-            e.faces[a] = f;
+            int64_t trans = 1;
+            for (int b = 0; b < d; b++)
+                if (b != a) trans *= v.n[b];
+            int R, W, ntA;
+            dtile_shape(d, v.n[a], R, W, ntA);
+            e.tiles[a] = int64_t(kDTile) * ntA * ((trans + W - 1) / W);
         }
         return e;
     }
@@ -235,14 +249,10 @@ class DiffusiveFluxReconstructorGPU {
         Layout L{};
         L.cell = align_up(size_t(cell_comps()) * size_t(e.cells), kAlignDoubles);
         L.total = L.cell;
-        for (int a = 0; a < 3; a++) {
-            L.fnode[a] = align_up(size_t(neq_) * size_t(e.nodes[a]), kAlignDoubles);
-            L.total += L.fnode[a];
-        }
         return L;
     }
 
-    DiffPatch make_patch(const hm_patch_view& v, double* base, const Layout& L) const {
+    DiffPatch make_patch(const hm_patch_view& v, double* base) const {
         DiffPatch p{};
         const int d = rec_.config().dim;
         for (int a = 0; a < 3; a++) {
@@ -250,15 +260,12 @@ class DiffusiveFluxReconstructorGPU {
             p.gq[a] = (a < d) ? v.ghost[a] : 0;
             p.dxinv[a] = (a < d) ? double(1) / v.dx[a] : 1.0;
             p.F[a] = (a < d) ? v.F[a] : nullptr;
+            int* t = p.tile[a];
+            dtile_shape(d, p.n[a], t[0], t[1], t[2]);
+            t[3] = int(small_div_mul(uint32_t(a == 0 ? t[0] : t[1])));
         }
         for (int e = 0; e < HM_MAX_EQN; e++) p.Q[e] = (e < neq_) ? v.Q[e] : nullptr;
-        double* q = base;
-        p.cell = q;
-        q += L.cell;
-        for (int a = 0; a < 3; a++) {
-            p.fnode[a] = L.fnode[a] ? q : nullptr;
-            q += L.fnode[a];
-        }
+        p.cell = base;
         return p;
     }
 
@@ -359,13 +366,12 @@ class DiffusiveFluxReconstructorGPU {
         for (auto& t : img) t.items.resize(np);
         for (int i = 0; i < np; i++) {
             const Layout L = layout(views[i]);
-            const DiffPatch dp = make_patch(views[i], base, L);
+            const DiffPatch dp = make_patch(views[i], base);
             base += L.total;
             for (auto& t : img) t.items[i] = dp;
             const Ext e = extents(views[i]);
             img[0].add(i, 0, e.cells);
-            for (int a = 0; a < d; a++) img[1].add(i, a, e.nodes[a]);
-            for (int a = 0; a < d; a++) img[2].add(i, a, e.faces[a]);
+            for (int a = 0; a < d; a++) img[1].add(i, a, e.tiles[a]);
         }
         size_t bytes = 0;
         for (auto& t : img) bytes += t.bytes();
@@ -388,7 +394,7 @@ class DiffusiveFluxReconstructorGPU {
 
     template <class W>
     int launch(const DPlan<W>& plan, const DParams& k, hipStream_t s) {
-        const hipError_t e = launch_diffusive_four<W>(rec_.config().dim, plan, k, s, 0, kDiffStages);
+        const hipError_t e = launch_diffusive_four<W>(rec_.config().dim, plan, k, s);
         if (e != hipSuccess)
             return rec_.fail(HM_ERR_DEVICE, std::string("diffusive kernel launch failed: ") + hipGetErrorString(e));
         return HM_OK;

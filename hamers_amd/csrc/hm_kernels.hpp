@@ -130,10 +130,28 @@ __host__ __device__ inline void mtile_shape(int nA, int& R, int& W, int& ntA) {
     W = 256 / R;
 }
 
-// Multiplier m of an exact division of a thread number (< 256) by d <= 256:
-// x / d = x m >> 16.  m d exceeds 2^16 by less than d, so the product is off by
-// less than x d < 2^16, under one in the quotient's last place.
-__host__ __device__ inline uint32_t small_div_mul(uint32_t d) { return (65536u + d - 1u) / d; }
+// Exact division of a thread number x by d, both up to 512, as a product: m d
+// exceeds 2^20 by less than d, so x m is off by less than x d < 2^20, under one
+// in the quotient's last place.
+__host__ __device__ inline uint32_t small_div_mul(uint32_t d) { return ((1u << 20) + d - 1u) / d; }
+__host__ __device__ inline uint32_t small_div(uint32_t x, uint32_t m) { return (x * m) >> 20; }
+
+// Column (u, v) of a tile's position w: columns run u fastest over nU by nV
+// positions, the tile's first one is t0 (block-uniform), W of them per tile.
+__device__ __forceinline__ void tile_column(uint32_t t0, uint32_t w, uint32_t W, uint32_t nU, uint32_t& u,
+                                            uint32_t& v) {
+    const uint32_t v0 = t0 / nU;
+    u = t0 - v0 * nU + w;
+    if (nU >= W) {  // at most one row on
+        const bool over = u >= nU;
+        v = v0 + (over ? 1u : 0u);
+        u -= over ? nU : 0u;
+    } else {  // u < nU + W
+        const uint32_t q = small_div(u, small_div_mul(nU));
+        v = v0 + q;
+        u -= q * nU;
+    }
+}
 
 // Work items of the fused axis-a segment of one patch: 256 per tile.
 __host__ __device__ inline int64_t mtile_items(int axis, const int* n, int dim) {

@@ -792,10 +792,10 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
     const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
     uint32_t r, w;
     if constexpr (A == 0) {
-        w = (lane * uint32_t(P.tile[A][3])) >> 16;  // lane / R
+        w = small_div(lane, uint32_t(P.tile[A][3]));  // lane / R
         r = lane - w * uint32_t(R);
     } else {
-        r = (lane * uint32_t(P.tile[A][3])) >> 16;  // lane / W
+        r = small_div(lane, uint32_t(P.tile[A][3]));  // lane / W
         w = lane - r * uint32_t(W);
     }
     const int j = int(tA) * (R - 2) + int(r);
@@ -803,18 +803,8 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
     // tile's first one is block-uniform, the others follow within a few rows
     constexpr int U = (A == 0) ? 1 : 0;  // first axis across
     constexpr int V = (A == 2) ? 1 : 2;  // second axis across
-    const uint32_t nU = uint32_t(B.n[U]), t0 = tw * uint32_t(W);
-    const uint32_t v0 = t0 / nU;
-    uint32_t cu = t0 - v0 * nU + w, tv;
-    if (nU >= uint32_t(W)) {  // at most one row on
-        const bool over = cu >= nU;
-        tv = v0 + (over ? 1u : 0u);
-        cu -= over ? nU : 0u;
-    } else {  // cu < nU + W < 256
-        const uint32_t q = (cu * small_div_mul(nU)) >> 16;
-        tv = v0 + q;
-        cu -= q * nU;
-    }
+    uint32_t cu, tv;
+    tile_column(tw * uint32_t(W), w, uint32_t(W), uint32_t(B.n[U]), cu, tv);
     const bool in = lane < uint32_t(R * W) && j < nA + 3 && tv < uint32_t(B.n[V]);
     int c[3];
     c[A] = j - 1;

@@ -1,8 +1,8 @@
-"""Tiles of the fused multi-species flux: the block-uniform column arithmetic
-(the kernel's multiplications in place of divisions) visits every midpoint face
-and writes every output face once for all small extents (on the CPU), and
-patches whose tiles wrap over several rows, hold single columns or end part
-filled equal the oracle (on the GPU)."""
+"""Tiles of the fused multi-species flux and of the diffusive flux: the
+block-uniform column arithmetic (the kernels' multiplications in place of
+divisions) visits every midpoint face or node and writes every output face once
+for all small extents (on the CPU), and patches whose tiles wrap over several
+rows, hold single columns or end part filled equal the oracle (on the GPU)."""
 import numpy as np
 import pytest
 
@@ -10,43 +10,42 @@ from hamers_amd import workloads as W
 from oracle import oracle as O
 
 
-def _shape(nA):
-    """mtile_shape of hm_kernels.hpp."""
-    nt = (nA + 1 + 61) // 62
-    R = (nA + 1 + nt - 1) // nt + 2
-    return R, 256 // R, nt
+def _shape(nA, kind):
+    """Rows, columns and tiles per column: mtile_shape of hm_kernels.hpp, dtile_shape of hm_diffusive.hpp."""
+    threads, most, shared = {"flux": (256, 62, 2), "diff": (512, 74, 11), "diff1d": (512, 501, 11)}[kind]
+    nt = (nA + 1 + most - 1) // most
+    R = (nA + 1 + nt - 1) // nt + shared
+    return R, threads // R, nt, threads, shared
 
 
-def _mul(d):
-    return (65536 + d - 1) // d
+def _div(x, d):
+    """small_div of hm_kernels.hpp."""
+    return (x * (((1 << 20) + d - 1) // d)) >> 20
 
 
 def test_small_divisions_are_exact():
-    x = np.arange(256)
-    for d in range(1, 257):
-        assert np.array_equal((x * _mul(d)) >> 16, x // d), d
-    # column wrap: cu < nU + W < 256 with nU < W <= 85
-    for nU in range(1, 85):
-        x = np.arange(nU + 85)
-        assert np.array_equal((x * _mul(nU)) >> 16, x // nU), nU
+    x = np.arange(512)
+    for d in range(1, 513):
+        assert np.array_equal(_div(x, d), x // d), d
 
 
+@pytest.mark.parametrize("kind", ["flux", "diff", "diff1d"])
 @pytest.mark.parametrize("axis", [0, 1])
-def test_tiles_cover_every_face_once(axis):
-    lane = np.arange(256)
-    for nA in (1, 2, 7, 8, 61, 62, 64, 123, 124, 125, 200):
-        R, Wd, nt = _shape(nA)
-        assert R * Wd <= 256
+def test_tiles_cover_every_face_once(axis, kind):
+    for nA in (1, 2, 7, 8, 61, 62, 64, 73, 74, 123, 124, 125, 148, 200, 500, 501, 502):
+        R, Wd, nt, threads, shared = _shape(nA, kind)
+        lane = np.arange(threads)
+        assert R * Wd <= threads
         for nU, nV in ((1, 1), (1, 9), (3, 5), (8, 8), (Wd, 2), (Wd + 1, 3), (200, 1)):
-            first = (lane * _mul(R if axis == 0 else Wd)) >> 16
+            first = _div(lane, R if axis == 0 else Wd)
             rest = lane - first * (R if axis == 0 else Wd)
             w, r = (first, rest) if axis == 0 else (rest, first)
             out = np.zeros((nU * nV, nA + 1), dtype=int)
-            mid = np.zeros((nU * nV, nA + 3), dtype=int)
+            mid = np.zeros((nU * nV, nA + 1 + shared), dtype=int)
             tiles = nt * -(-nU * nV // Wd)
             for tile in range(tiles):
                 tw, tA = tile // nt, tile % nt
-                j = tA * (R - 2) + r
+                j = tA * (R - shared) + r
                 t0 = tw * Wd
                 v0 = t0 // nU
                 cu = t0 - v0 * nU + w
@@ -54,13 +53,16 @@ def test_tiles_cover_every_face_once(axis):
                     over = cu >= nU
                     tv, cu = v0 + over, cu - over * nU
                 else:
-                    q = (cu * _mul(nU)) >> 16
+                    q = _div(cu, nU)
                     tv, cu = v0 + q, cu - q * nU
-                inside = (lane < R * Wd) & (j < nA + 3) & (tv < nV)
+                inside = (lane < R * Wd) & (j < nA + 1 + shared) & (tv < nV)
                 col = tv * nU + cu
-                mid[col[inside], j[inside]] += 1
-                writes = inside & (r >= 1) & (r <= R - 2) & (j <= nA + 1)
-                np.add.at(out, (col[writes], j[writes] - 1), 1)
+                np.add.at(mid, (col[inside], j[inside]), 1)
+                if kind == "flux":
+                    writes, face = inside & (r >= 1) & (r <= R - 2) & (j <= nA + 1), j - 1
+                else:
+                    writes, face = inside & (r >= 6) & (r <= R - 6) & (j - 6 <= nA), j - 6
+                np.add.at(out, (col[writes], face[writes]), 1)
             assert np.all(out == 1), (nA, nU, nV)
             assert np.all(mid >= 1), (nA, nU, nV)
 
@@ -106,3 +108,39 @@ def test_tile_shapes_against_oracle(n, model, scheme):
         for a in range(3):
             assert np.array_equal(F[a].cpu().numpy(), Fr[a]), a
         assert np.array_equal(S.cpu().numpy(), Sr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(3, 2, 70), (150, 1, 5), (1, 1, 9), (75, 74), (1, 160), (600,), (5,)])
+def test_diffusive_tile_shapes_against_oracle(n):
+    """Same bits as the oracle, batched and per patch, on tiles of one to several rows and columns (ghost width 7)."""
+    import torch
+
+    from hamers_amd import ConvectiveFluxReconstructor, DiffusiveFluxReconstructor, PatchData, PatchList
+
+    assert torch.cuda.is_available(), "GPU tests need a visible GPU"
+    d, g, gamma, R = len(n), 7, (1.4, 1.67), (1.0, 2.0)
+    rng = np.random.default_rng(sum(n))
+    shp = tuple(v + 2 * g for v in reversed(n))
+    Y = 0.5 + 0.4 * rng.uniform(-1, 1, shp)
+    vel = [rng.uniform(-1, 1, shp) for _ in range(d)]
+    Q = W.conservative_from_primitive_four([Y, 0.3 * (1 - Y)], vel, 1.0 + 0.5 * rng.uniform(0, 1, shp), gamma, R)
+    dx, dt = tuple(1.0 / v for v in n), 1e-3
+    tr = {"mu": (1e-3, 2e-3), "mu_v": (2e-4, 3e-4), "kappa": (1.5e-3, 2.5e-3), "D": (1e-3, 1.2e-3), "M": (1.0, 4.0)}
+    rec = ConvectiveFluxReconstructor("tiles", d, "FOUR_EQN_CONSERVATIVE", "WCNS5_JS_HLLC_HLL", num_species=2,
+                                      species_gamma=gamma, species_R=R)
+    diff = DiffusiveFluxReconstructor(rec, *(tr[k] for k in ("mu", "mu_v", "kappa", "D", "M")))
+    prm = O.Params(dim=d, model=O.FOUR_EQN_CONSERVATIVE, num_species=2, scheme=0, gamma=list(gamma), R=list(R))
+    want = O.diffusive_patch(prm, O.Transport(*(list(tr[k]) for k in ("mu", "mu_v", "kappa", "D", "M"))), Q, n, g, dx, dt)
+    for batched in (False, True):
+        F = [torch.full(O.face_shape(rec.num_eqn, n, a), np.nan, dtype=torch.float64, device="cuda:0") for a in range(d)]
+        pd = PatchData(n, (g,) * d, dx, torch.from_numpy(Q).to("cuda:0"), F, None)
+        if batched:
+            diff.computeDiffusiveFluxOnPatches(PatchList([pd, pd], rec.num_eqn), 0.0, dt)
+        else:
+            diff.computeDiffusiveFluxOnPatch(pd, 0.0, dt)
+        torch.cuda.synchronize()
+        for a in range(d):
+            got = F[a].cpu().numpy()
+            print(f"{n} batched {batched} axis {a}: {int(np.sum(got != want[a]))} of {got.size} differ", flush=True)
+            assert np.array_equal(got, want[a])

@@ -73,12 +73,14 @@ struct DevPatch {
     const double* Q[HM_MAX_EQN];  // conservative variables, per equation, over the Q ghost box
     double* F[3];                 // output face flux per axis (component-major)
     double* S;                    // output source (component-major interior)
-    double* prim;                 // scratch: V[0..neq) and c over the 4-ghost box
+    double* prim;                 // scratch over the 4-ghost box: V[0..neq) and c, or (multi-species) u.., p and c
     double* sens;                 // scratch: theta, Omega over the 2-ghost box
     double* fmid[3];              // scratch: midpoint flux per axis, neq comps over (n_a+3) x n_b box
     double* ustar[3];             // scratch: HLLC normal velocity per axis (advective models)
     int tile[3][4];               // shape of the axis' multi-species flux tiles (mtile_shape), and a multiplier that
                                   // divides a thread number by a tile row (mtile_row)
+    const double* vb[HM_MAX_EQN]; // multi-species: component base of each variable of the reconstruction (Q or prim)
+    int64_t vst[3][2];            // cell stride along axis a of the prim box and of Q's box
     int64_t wrec[3];              // offset of this patch's axis-a chunk in a face-state slot (KParams::wrec), -1: none
 };
 
@@ -144,6 +146,14 @@ template <class T>
 __device__ __forceinline__ const T* as_constant(const T* p) {
     typedef __attribute__((address_space(4))) const T ctype;
     return (const T*)(ctype*)p;
+}
+
+// One wave-uniform word of such memory by a runtime index, as a scalar load.
+template <class T>
+__device__ __forceinline__ T ld_constant(const T* p) {
+    typedef __attribute__((address_space(4))) const uint64_t cword;
+    static_assert(sizeof(T) == sizeof(uint64_t));
+    return (T)*(cword*)p;
 }
 
 template <class T>

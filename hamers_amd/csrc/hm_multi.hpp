@@ -13,8 +13,9 @@
 // mixture EOS mixes c_p and c_v with mass fractions
 // (EquationOfStateMixingRulesIdealGas.cpp:4677-4737).
 //
-// Scratch prim holds V = (partial densities, u.., p[, Z_i (NS-1)]), then c,
-// then the mixture density rho, over the 4-ghost box.
+// Scratch prim holds what the conservative arrays do not: u.., p, c over the
+// 4-ghost box.  The partial densities and volume fractions of V are read from
+// the caller's arrays, and rho is their sum.
 //
 // Pipeline: k_derived_multi (with the dilatation and vorticity on the 2-ghost
 // box), k_flux_multi (midpoint and face flux fused over tiles; five-equation:
@@ -47,6 +48,7 @@ struct Multi {
     static constexpr int NEQ = FOUR ? NS + D + 1 : D + 2 * NS;
     static constexpr int NZ = FOUR ? 0 : NS - 1;  // evolved volume fractions
     static constexpr int IP = NS + D;             // pressure slot of V
+    static constexpr int PU = 0, PP = D, PC = D + 1;  // components of the scratch prim: u.., p, c
     static constexpr int IZ = NS + D + 1;         // first volume-fraction slot of V
 };
 
@@ -172,7 +174,10 @@ __device__ __forceinline__ void cell_state_multi(const KParams& k, QF&& q, uint3
 
 // ----------------------------------------------------------------------------
 // Derived cell data (FlowModelFiveEqnAllaire.cpp:3734-4876,
-// FlowModelFourEqnConservative.cpp:3877-5440).
+// FlowModelFourEqnConservative.cpp:3877-5440).  Bound by HBM writes (a copy
+// reaches 4.2 TB/s here, read and written): with the partial densities, volume
+// fractions and rho stored too, nine components instead of five, it took 5.30 ms
+// on the uneven 3D five-equation level of 2744 patches, 4.34 ms without them.
 // ----------------------------------------------------------------------------
 template <int D, int NS, bool FOUR, class W>
 __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
@@ -182,7 +187,6 @@ __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
     int64_t loc;
     if (!w.find(gid, P, ax, loc)) return;
     using M = Multi<D, NS, FOUR>;
-    constexpr int NEQ = M::NEQ;
     const Boxes<D> B(*P);
     const int e0 = B.ext(0, kGc), e1 = B.ext(1, kGc);
     // 32-bit index arithmetic (a work segment has fewer than 2^31 items).
@@ -201,14 +205,9 @@ __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
     double* pr = P->prim;
     const uint32_t l32 = uint32_t(loc);
 #pragma unroll
-    for (int si = 0; si < NS; si++) stg(pr + si * vol, l32, Zr[si]);
-#pragma unroll
-    for (int b = 0; b < D; b++) stg(pr + (NS + b) * vol, l32, u[b]);
-    stg(pr + (NS + D) * vol, l32, p);
-#pragma unroll
-    for (int si = 0; si < M::NZ; si++) stg(pr + (NS + D + 1 + si) * vol, l32, Z[si]);
-    stg(pr + NEQ * vol, l32, sqrt(c2));
-    stg(pr + (NEQ + 1) * vol, l32, rho);
+    for (int b = 0; b < D; b++) stg(pr + (M::PU + b) * vol, l32, u[b]);
+    stg(pr + M::PP * vol, l32, p);
+    stg(pr + M::PC * vol, l32, sqrt(c2));
 
     if constexpr (D > 1) {
         // dilatation and vorticity on the 2-ghost box, from the neighbours'
@@ -307,7 +306,7 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
 // fused flux issues 3246 VALU instructions per wavefront at 82 % of the rate
 // (4357 at 75 % before its loads took scalar bases, a field's loads went out
 // together and the WENO weights lost a quarter of their instructions): 36.4 ms
-// -> 25.6 ms.
+// -> 24.2 ms.
 // Midpoint flux Fo of the face normal to axis A between cells (c0, c1, c2)
 // - e_A and (c0, c1, c2), and its HLLC normal velocity u* (five-equation).
 // The prim and sensor arrays are read at 32-bit offsets from per-component
@@ -327,16 +326,33 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     const int64_t st = (A == 0) ? 1 : (A == 1) ? int64_t(B.ext(0, kGc)) : int64_t(B.ext(0, kGc)) * B.ext(1, kGc);
     uint32_t off = uint32_t(B.idx(kGc, c0, c1, c2)) * 8u;
     const double* pr = P.prim;
+    // the caller's box
+    const int64_t qst = (A == 0)   ? 1
+                        : (A == 1) ? int64_t(P.n[0] + 2 * P.gq[0])
+                                   : int64_t(P.n[0] + 2 * P.gq[0]) * (P.n[1] + 2 * P.gq[1]);
+    uint32_t qoff = uint32_t(q_idx<D>(P, c0, c1, c2)) * 8u;
     // component and stencil position in the wave-uniform base, so that every
-    // load takes the same 32-bit vector offset
-    auto ld = [&](int comp, int m) { return ldg_byte(pr + (comp * v4 + (m - 3) * st), off); };
+    // load of an array takes the same 32-bit vector offset
+    auto ldp = [&](int comp, int m) { return ldg_byte(pr + (comp * v4 + (m - 3) * st), off); };
+    auto ldq = [&](int e, int m) { return ldg_byte(P.Q[e] + (m - 3) * qst, qoff); };
+    // variable e of V
+    auto ldv = [&](int e, int m) {
+        if (e < NS || e > IP) return ldq(e, m);
+        return ldp(M::PU + (e - NS), m);  // u.., p
+    };
 
     // Projection variables (FlowModelBasicUtilitiesFiveEqnAllaire.cpp:7474-8207).
     double Zra[NS];
+    double rL = double(0), rR = double(0);  // rho of the two cells (EquationOfStateMixingRules.cpp:735-860)
 #pragma unroll
-    for (int si = 0; si < NS; si++) Zra[si] = double(1) / double(2) * (ld(si, 2) + ld(si, 3));
-    const double ra = double(1) / double(2) * (ld(NEQ + 1, 2) + ld(NEQ + 1, 3));
-    const double ca = double(1) / double(2) * (ld(NEQ, 2) + ld(NEQ, 3));
+    for (int si = 0; si < NS; si++) {
+        const double zL = ldq(si, 2), zR = ldq(si, 3);
+        Zra[si] = double(1) / double(2) * (zL + zR);
+        rL += zL;
+        rR += zR;
+    }
+    const double ra = double(1) / double(2) * (rL + rR);
+    const double ca = double(1) / double(2) * (ldp(M::PC, 2) + ldp(M::PC, 3));
 
     // Characteristic fields (FlowModelBasicUtilitiesFiveEqnAllaire.cpp:8232-9178),
     // one at a time: a runtime loop keeps a single field's WENO interpolation
@@ -353,7 +369,7 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     const LDConst ldk{k.p, k.q, k.C, k.alpha_tau, k.inv_thr};
     double ps[6];
 #pragma unroll
-    for (int m = 0; m < 6; m++) ps[m] = ld(IP, m);
+    for (int m = 0; m < 6; m++) ps[m] = ldp(M::PP, m);
     {
         const double rc = ra * ca;
         const double irc = div_rn(double(1), rc);
@@ -376,10 +392,14 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 #pragma unroll 1
     for (int f = 0; f < NEQ; f++) {
         const int comp = int(comps >> (4 * f)) & 15;
-        pin_offset(off);
+        const bool in_q = comp < NS || comp > IP;
+        const double* base = ld_constant(&P.vb[comp]);
+        const int64_t step = ld_constant(&P.vst[A][in_q ? 1 : 0]);
+        uint32_t o = in_q ? qoff : off;
+        pin_offset(o);
         Six s;
 #pragma unroll
-        for (int m = 0; m < 6; m++) s.v[m] = ld(comp, m);
+        for (int m = 0; m < 6; m++) s.v[m] = ldg_byte(base + (m - 3) * step, o);
         if (f <= NS || f == NEQ - 1) {
             const double cf = wl[f * kBlock];
 #pragma unroll
@@ -427,10 +447,11 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     // Bounds on both sides, else first-order values (WCNS56-HLLC-HLL.cpp:947-1032).
     if (!(bounded_multi<D, NS, FOUR, A>(VL, k) && bounded_multi<D, NS, FOUR, A>(VR, k))) {
         pin_offset(off);
+        pin_offset(qoff);
 #pragma unroll
         for (int e = 0; e < NEQ; e++) {
-            VL[e] = ld(e, 2);
-            VR[e] = ld(e, 3);
+            VL[e] = ldv(e, 2);
+            VR[e] = ldv(e, 3);
         }
     }
 
@@ -701,12 +722,12 @@ __device__ __forceinline__ void combine_face_multi(const DevPatch& P, const Boxe
 template <int D, int NS, bool FOUR, int A>
 __device__ __forceinline__ void cell_node_flux_multi(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
                                                      double* nf, int stride) {
-    constexpr int NEQ = Multi<D, NS, FOUR>::NEQ;
-    constexpr int IP = NS + D;
+    using M = Multi<D, NS, FOUR>;
+    constexpr int NEQ = M::NEQ;
     const int64_t v4 = B.vol(kGc);
     const uint32_t pc = uint32_t(B.idx(kGc, c0, c1, c2));
     const uint32_t q = uint32_t(q_idx<D>(P, c0, c1, c2));
-    const double ua = ldg(P.prim + (NS + A) * v4, pc), pr = ldg(P.prim + IP * v4, pc);
+    const double ua = ldg(P.prim + (M::PU + A) * v4, pc), pr = ldg(P.prim + M::PP * v4, pc);
 #pragma unroll
     for (int e = 0; e < NEQ; e++) nf[e * stride] = node_flux_multi<D, NS, A>(P, q, ua, pr, e);
 }
@@ -715,7 +736,7 @@ __device__ __forceinline__ void cell_node_flux_multi(const DevPatch& P, const Bo
 template <int D, int NS, bool FOUR, int A, class MF>
 __device__ __forceinline__ void store_face_multi(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
                                                  double dt, MF&& m) {
-    constexpr int IP = NS + D;
+    using M = Multi<D, NS, FOUR>;
     const int64_t v4 = B.vol(kGc);
     const uint32_t st4 = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGc)) : uint32_t(B.ext(0, kGc) * B.ext(1, kGc));
     const uint32_t pR = uint32_t(B.idx(kGc, c0, c1, c2)), pL = pR - st4;
@@ -723,8 +744,8 @@ __device__ __forceinline__ void store_face_multi(const DevPatch& P, const Boxes<
                          : (A == 1) ? uint32_t(P.n[0] + 2 * P.gq[0])
                                     : uint32_t((P.n[0] + 2 * P.gq[0]) * (P.n[1] + 2 * P.gq[1]));
     const uint32_t qR = uint32_t(q_idx<D>(P, c0, c1, c2)), qL = qR - qst;
-    const double uaL = ldg(P.prim + (NS + A) * v4, pL), uaR = ldg(P.prim + (NS + A) * v4, pR);
-    const double prL = ldg(P.prim + IP * v4, pL), prR = ldg(P.prim + IP * v4, pR);
+    const double uaL = ldg(P.prim + (M::PU + A) * v4, pL), uaR = ldg(P.prim + (M::PU + A) * v4, pR);
+    const double prL = ldg(P.prim + M::PP * v4, pL), prR = ldg(P.prim + M::PP * v4, pR);
     combine_face_multi<D, NS, FOUR, A>(P, B, c0, c1, c2, dt, m, [&](int side, int e) {
         return side < 0 ? node_flux_multi<D, NS, A>(P, qL, uaL, prL, e) : node_flux_multi<D, NS, A>(P, qR, uaR, prR, e);
     });
@@ -882,7 +903,7 @@ __global__ __launch_bounds__(kBlock) void k_source_five(W w, KParams k) {
         const int64_t m = B.mid_idx(a, i, j, kk);  // face between cells i-1 and i along a
         const double* us = P->ustar[a];
         const double uLL = us[m - mst], uL = us[m], uR = us[m + mst], uRR = us[m + 2 * mst];
-        const double* u = P->prim + (NS + a) * v4;
+        const double* u = P->prim + a * v4;
         const double cL = u[pc - st4], cR = u[pc + st4];
         const double term = (double(3) / double(2) * (uR - uL) - double(3) / double(10) * (cR - cL) +
                              double(1) / double(30) * (uRR - uLL)) /

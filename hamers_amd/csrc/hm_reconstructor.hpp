@@ -149,9 +149,16 @@ class ConvectiveFluxReconstructorGPU {
     // also hands over the last species' volume fraction (stored, not evolved).
     int numConservativeArrays() const { return cfg_.model == HM_MODEL_FIVE_EQN_ALLAIRE ? neq_ + 1 : neq_; }
 
-    // Scratch components per cell of the 4-ghost box: V, c (and rho for the
-    // multi-species models).
-    int prim_comps() const { return cfg_.model == HM_MODEL_SINGLE_SPECIES ? neq_ + 1 : neq_ + 2; }
+    // Scratch components per cell of the 4-ghost box: V and c, or u.., p and c
+    // for the multi-species models (the rest of V is in the caller's arrays).
+    int prim_comps() const { return cfg_.model == HM_MODEL_SINGLE_SPECIES ? neq_ + 1 : cfg_.dim + 2; }
+
+    // Scratch a patch counts for at the allocation-free entry point, whose
+    // limit takes all of V, c and rho per cell.
+    size_t limitDoubles(const hm_patch_view& v, const ScratchLayout& L) const {
+        if (cfg_.model == HM_MODEL_SINGLE_SPECIES) return L.total;
+        return L.total - L.prim + align_up(size_t(neq_ + 2) * extents(v).vol4, kAlignDoubles);
+    }
 
     // ConvectiveFluxReconstructor::getConvectiveFluxNumberOfGhostCells (4 for WCNS56).
     int getConvectiveFluxNumberOfGhostCells() const { return kGc; }
@@ -180,12 +187,12 @@ class ConvectiveFluxReconstructorGPU {
         if (int st = check_view(v, 0)) return st;
         if (int st = select_device()) return st;
         const ScratchLayout L = layout(v);
-        if (L.total > cap) {
+        if (limitDoubles(v, L) > cap) {
             char buf[200];
             snprintf(buf, sizeof buf,
                      "patch needs %zu doubles of scratch; the allocation-free entry point holds %zu "
                      "(use hm_compute_convective_flux_and_source_on_patch)",
-                     L.total, cap);
+                     limitDoubles(v, L), cap);
             return fail(HM_ERR_INVALID_ARGUMENT, buf);
         }
         const Plan<SegSingle> plan = patch_plan(v, scratch, L);
@@ -680,6 +687,19 @@ class ConvectiveFluxReconstructorGPU {
         p.S = v.S;
         double* q = base;
         p.prim = q;
+        if (cfg_.model != HM_MODEL_SINGLE_SPECIES) {
+            for (int e = 0; e < nq; e++) {
+                const int c = e - cfg_.num_species;  // u.., p are stored, the others are read from Q
+                p.vb[e] = (c >= 0 && c <= d) ? p.prim + size_t(c) * extents(v).vol4 : p.Q[e];
+            }
+            int64_t sp = 1, sq = 1;
+            for (int a = 0; a < d; a++) {
+                p.vst[a][0] = sp;
+                p.vst[a][1] = sq;
+                sp *= v.n[a] + 2 * kGc;
+                sq *= v.n[a] + 2 * v.ghost[a];
+            }
+        }
         q += L.prim;
         p.sens = L.sens ? q : nullptr;
         q += L.sens;

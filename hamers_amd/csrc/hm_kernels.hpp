@@ -175,6 +175,7 @@ struct Plan {
     W work[kStages];
     int64_t items[kStages];
     int tile_rows;  // rows of the tiled flux stage (single-species model): 4, 8 or 24
+    int direct;     // single-species, one patch: no derived-data pass (tile_rows 4)
     int xcd;        // KParams::xcd of the plan's launches
     int persistent; // multi-species midpoint flux from a work queue (KParams::queue)
     unsigned* queue;

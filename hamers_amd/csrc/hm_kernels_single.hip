@@ -12,6 +12,8 @@
 //                       879-1194, 1746-2320) and the sixth-order midpoint-to-face
 //                       flux times dt (1197-1282, 2327-2490), fused per wavefront
 //   k_flux_tile_single  axes 1 and 2: the same, fused per 64 x 24 tile
+//   k_flux_patch_single one patch: all axes in one launch, and for a small
+//                       patch the derived cell data too
 #include <type_traits>
 
 #include "hm_cell.hpp"
@@ -86,23 +88,94 @@ __global__ __launch_bounds__(kBlock) void k_derived_single(W w, KParams k) {
 // in tiles whose lanes lie across the sweep (coalesced loads), below.
 // ----------------------------------------------------------------------------
 
+// Shock sensor of a face from the dilatations and vorticity magnitudes of its
+// two cells (WCNS56-HLLC-HLL.cpp:1066-1113): whether it takes HLLC-HLL.
+__device__ __forceinline__ bool takes_hll(double thL, double thR, double omL, double omR) {
+    const double th_avg = 0.5 * (thL + thR);
+    const double om_avg = 0.5 * (omL + omR);
+    const double sensor = div_rn(-th_avg, fabs(th_avg) + om_avg + kEps);
+    return sensor > 0.65;
+}
+
+// The same of the face whose right cell is (c0, c1, c2) along A, from the
+// patch's sensor array.
+template <int D, int A>
+__device__ __forceinline__ bool takes_hll_at(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2) {
+    if constexpr (D == 1) return false;
+    const int64_t vs = B.vol(kGs);
+    const uint32_t tR = uint32_t(B.idx(kGs, c0, c1, c2));
+    const uint32_t sts = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGs)) : uint32_t(B.ext(0, kGs) * B.ext(1, kGs));
+    return takes_hll(ldg(P.sens, tR - sts), ldg(P.sens, tR), ldg(P.sens + vs, tR - sts), ldg(P.sens + vs, tR));
+}
+
+// Cells of one patch straight from Q, for calls whose cells are not derived
+// beforehand: the same arithmetic as the derived-data kernel, so the same bits.
+// Each face derives its six stencil cells and its sensor's neighbours again;
+// a call too small to fill the device pays less for that than for the
+// derived-data kernel before it (4.7 us and a launch of a 128^2 patch's 20.2).
+template <int D>
+struct QCells {
+    const DevPatch& P;
+    const KParams& k;
+    uint32_t st[3];
+    __device__ __forceinline__ QCells(const DevPatch& P_, const KParams& k_) : P(P_), k(k_) {
+        st[0] = 1u;
+        st[1] = uint32_t(P.n[0] + 2 * P.gq[0]);
+        st[2] = st[1] * uint32_t(P.n[1] + 2 * P.gq[1]);
+    }
+    __device__ __forceinline__ double q(int e, uint32_t at) const { return ldg(P.Q[e] + k.qoff, at); }
+    __device__ __forceinline__ double state(uint32_t at, double (&V)[D + 2]) const {
+        double u[3], c;
+        cell_state_single<D>([&](int e, uint32_t i) { return q(e, i); }, at, k.gamma[0], V[0], u, V[D + 1], c);
+#pragma unroll
+        for (int b = 0; b < D; b++) V[1 + b] = u[b];
+        return c;
+    }
+    __device__ __forceinline__ void velocity(uint32_t at, double (&v)[3]) const {
+        const double r = q(0, at), rr = rcp_rn(r);
+#pragma unroll
+        for (int b = 0; b < D; b++) v[b] = quot(q(1 + b, at), r, rr);
+    }
+    // Stencil and sound speeds of the face along A whose right cell is at qR.
+    template <int A>
+    __device__ __forceinline__ void stencil(uint32_t qR, double (&V)[6][D + 2], double& cL, double& cR) const {
+#pragma unroll
+        for (int m = 0; m < 6; m++) {
+            const double c = state(qR + uint32_t(m - 3) * st[A], V[m]);
+            if (m == 2) cL = c;
+            if (m == 3) cR = c;
+        }
+    }
+    // The face's sensor: the velocities along A are the stencil's own.
+    template <int A>
+    __device__ __forceinline__ bool hll(uint32_t qR, const double (&V)[6][D + 2]) const {
+        if constexpr (D == 1) return false;
+        double th[2], om[2];
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            sensor_values<D>(
+                P,
+                [&](int a, int side, double (&v)[3]) {
+                    if (a == A) {
+#pragma unroll
+                        for (int b = 0; b < D; b++) v[b] = V[2 + s + side][1 + b];
+                    } else {
+                        const uint32_t at = qR + uint32_t(s - 1) * st[A];
+                        velocity(side > 0 ? at + st[a] : at - st[a], v);
+                    }
+                },
+                th[s], om[s]);
+        return takes_hll(th[0], th[1], om[0], om[1]);
+    }
+};
+
 // Midpoint flux of the face whose right cell is (c0, c1, c2) along A, from its
 // stencil V (cells i-3 .. i+2) and the sound speeds of cells i-1, i.
 template <int D, int A, int SCHEME, int PP, int QQ, bool REC>
 __device__ __forceinline__ void midpoint_flux_at(const DevPatch& P, const Boxes<D>& B, const KParams& k,
-                                                 const double (&V)[6][D + 2], double cL, double cR, int c0, int c1,
-                                                 int c2, double (&Fo)[D + 2]) {
+                                                 const double (&V)[6][D + 2], double cL, double cR, bool use_hll,
+                                                 int c0, int c1, int c2, double (&Fo)[D + 2]) {
     constexpr int NEQ = D + 2;
-    bool use_hll = false;
-    if constexpr (D > 1) {
-        const int64_t vs = B.vol(kGs);
-        const uint32_t tR = uint32_t(B.idx(kGs, c0, c1, c2));
-        const uint32_t sts = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGs)) : uint32_t(B.ext(0, kGs) * B.ext(1, kGs));
-        const double th_avg = 0.5 * (ldg(P.sens, tR - sts) + ldg(P.sens, tR));
-        const double om_avg = 0.5 * (ldg(P.sens + vs, tR - sts) + ldg(P.sens + vs, tR));
-        const double sensor = div_rn(-th_avg, fabs(th_avg) + om_avg + kEps);
-        use_hll = sensor > 0.65;
-    }
     if constexpr (REC) {
         const uint32_t mv = uint32_t(B.mid_vol(A)), mi = uint32_t(B.mid_idx(A, c0, c1, c2));
         double* wr = k.wrec + P.wrec[A];
@@ -144,7 +217,7 @@ __device__ __forceinline__ void store_face_flux(double* out, int64_t fv, int64_t
                   double(23) / double(15) * mM[e]));
 }
 
-template <int D, int A, int SCHEME, int PP, int QQ, bool REC>
+template <int D, int A, int SCHEME, int PP, int QQ, bool REC, bool DIRECT = false>
 __device__ __forceinline__ void fused_chunk(const DevPatch& P, int64_t loc, const KParams& k) {
     constexpr int NEQ = D + 2;
     constexpr int IP = D + 1;
@@ -170,17 +243,27 @@ __device__ __forceinline__ void fused_chunk(const DevPatch& P, int64_t loc, cons
 
     const int64_t v4 = B.vol(kGc);
     const uint32_t st = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGc)) : uint32_t(B.ext(0, kGc) * B.ext(1, kGc));
-    const uint32_t iR = uint32_t(B.idx(kGc, c0, c1, c2));
-    const double* pr = P.prim;
     double V[6][NEQ];
+    double cL, cR;
+    bool use_hll;
+    if constexpr (DIRECT) {
+        const QCells<D> cells(P, k);
+        const uint32_t qc = uint32_t(q_idx<D>(P, c0, c1, c2));
+        cells.template stencil<A>(qc, V, cL, cR);
+        use_hll = cells.template hll<A>(qc, V);
+    } else {
+        const uint32_t iR = uint32_t(B.idx(kGc, c0, c1, c2));
+        const double* pr = P.prim;
 #pragma unroll
-    for (int m = 0; m < 6; m++)
+        for (int m = 0; m < 6; m++)
 #pragma unroll
-        for (int e = 0; e < NEQ; e++) V[m][e] = ldg(pr + e * v4, iR + uint32_t(m - 3) * st);
-    const double cL = ldg(pr + NEQ * v4, iR - st);
-    const double cR = ldg(pr + NEQ * v4, iR);
+            for (int e = 0; e < NEQ; e++) V[m][e] = ldg(pr + e * v4, iR + uint32_t(m - 3) * st);
+        cL = ldg(pr + NEQ * v4, iR - st);
+        cR = ldg(pr + NEQ * v4, iR);
+        use_hll = takes_hll_at<D, A>(P, B, c0, c1, c2);
+    }
     double mM[NEQ];
-    midpoint_flux_at<D, A, SCHEME, PP, QQ, REC>(P, B, k, V, cL, cR, c0, c1, c2, mM);
+    midpoint_flux_at<D, A, SCHEME, PP, QQ, REC>(P, B, k, V, cL, cR, use_hll, c0, c1, c2, mM);
 
     // Neighbours' midpoint fluxes (every lane takes part in the shuffles).
     double mL[NEQ], mR[NEQ];
@@ -224,7 +307,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SCHEME =
 // The stage's segments hold whole tiles (256 items each; every segment of the
 // stage is a tile segment, so each starts on a multiple of 256) and every
 // block lies in one tile: the barrier is reached by all four wavefronts.
-template <int D, int A, int R, int SCHEME, int PP, int QQ, bool REC>
+template <int D, int A, int R, int SCHEME, int PP, int QQ, bool REC, bool DIRECT = false>
 __device__ __forceinline__ void fused_tile(const DevPatch& P, int64_t loc, const KParams& k, double* lds) {
     constexpr int NEQ = D + 2;
     constexpr int IP = D + 1;
@@ -257,15 +340,26 @@ __device__ __forceinline__ void fused_tile(const DevPatch& P, int64_t loc, const
         if (j > nA + 1) break;  // past the last midpoint face (uniform per wavefront: one row each)
         int c0, c1, c2;
         cell(j, c0, c1, c2);
-        const uint32_t iR = uint32_t(B.idx(kGc, c0, c1, c2));
         double V[6][NEQ];
+        double cL, cR;
+        bool use_hll;
+        if constexpr (DIRECT) {
+            const QCells<D> cells(P, k);
+            const uint32_t qc = uint32_t(q_idx<D>(P, c0, c1, c2));
+            cells.template stencil<A>(qc, V, cL, cR);
+            use_hll = cells.template hll<A>(qc, V);
+        } else {
+            const uint32_t iR = uint32_t(B.idx(kGc, c0, c1, c2));
 #pragma unroll
-        for (int m = 0; m < 6; m++)
+            for (int m = 0; m < 6; m++)
 #pragma unroll
-            for (int e = 0; e < NEQ; e++) V[m][e] = ldg(pr + e * v4, iR + uint32_t(m - 3) * st);
-        const double cL = ldg(pr + NEQ * v4, iR - st), cR = ldg(pr + NEQ * v4, iR);
+                for (int e = 0; e < NEQ; e++) V[m][e] = ldg(pr + e * v4, iR + uint32_t(m - 3) * st);
+            cL = ldg(pr + NEQ * v4, iR - st);
+            cR = ldg(pr + NEQ * v4, iR);
+            use_hll = takes_hll_at<D, A>(P, B, c0, c1, c2);
+        }
         double m[NEQ];
-        midpoint_flux_at<D, A, SCHEME, PP, QQ, REC>(P, B, k, V, cL, cR, c0, c1, c2, m);
+        midpoint_flux_at<D, A, SCHEME, PP, QQ, REC>(P, B, k, V, cL, cR, use_hll, c0, c1, c2, m);
 #pragma unroll
         for (int e = 0; e < NEQ; e++) lds[(e * R + row) * kTileX + tx] = m[e];
     }
@@ -278,10 +372,20 @@ __device__ __forceinline__ void fused_tile(const DevPatch& P, int64_t loc, const
         if (row < 1 || row > R - 2 || !vx || f > nA) continue;
         int c0, c1, c2;
         cell(f, c0, c1, c2);
-        const uint32_t pR = uint32_t(B.idx(kGc, c0, c1, c2)), pL = pR - st;
         const uint32_t qR = uint32_t(q_idx<D>(P, c0, c1, c2)), qL = qR - qst;
-        const double uaL = ldg(pr + (1 + A) * v4, pL), uaR = ldg(pr + (1 + A) * v4, pR);
-        const double prL = ldg(pr + IP * v4, pL), prR = ldg(pr + IP * v4, pR);
+        double uaL, uaR, prL, prR;
+        if constexpr (DIRECT) {
+            const QCells<D> cells(P, k);
+            double VL[NEQ], VR[NEQ];
+            cells.state(qL, VL);
+            cells.state(qR, VR);
+            uaL = VL[1 + A], uaR = VR[1 + A];
+            prL = VL[IP], prR = VR[IP];
+        } else {
+            const uint32_t pR = uint32_t(B.idx(kGc, c0, c1, c2)), pL = pR - st;
+            uaL = ldg(pr + (1 + A) * v4, pL), uaR = ldg(pr + (1 + A) * v4, pR);
+            prL = ldg(pr + IP * v4, pL), prR = ldg(pr + IP * v4, pR);
+        }
         double mL[NEQ], mM[NEQ], mR[NEQ], nL[NEQ], nR[NEQ];
 #pragma unroll
         for (int e = 0; e < NEQ; e++) {
@@ -318,7 +422,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SCHEME =
 // 1 and 2 in one launch, so that the two flux stages of a small call overlap
 // instead of running one after the other.  The axis-0 segment is padded to a
 // multiple of 256 items, so a block holds either chunks or one tile.
-template <int D, int R, int SCHEME, int PP, int QQ, class W>
+// DIRECT: the cells' derived data straight from Q, without the pass before.
+template <int D, int R, int SCHEME, int PP, int QQ, bool DIRECT, class W>
 __global__ __launch_bounds__(kBlock) void k_flux_patch_single(W w, KParams k) {
     __shared__ double lds[(D > 1) ? R * kTileX * (D + 2) : 1];
     const int64_t gid = int64_t(rhs_block(k)) * kBlock + threadIdx.x;
@@ -327,12 +432,12 @@ __global__ __launch_bounds__(kBlock) void k_flux_patch_single(W w, KParams k) {
     int64_t loc;
     if (!w.find(gid, P, ax, loc)) return;  // holes lie in axis-0 blocks only
     if (ax == 0) {
-        fused_chunk<D, 0, SCHEME, PP, QQ, false>(*P, loc, k);
+        fused_chunk<D, 0, SCHEME, PP, QQ, false, DIRECT>(*P, loc, k);
     } else if constexpr (D > 1) {
         if (ax == 1) {
-            fused_tile<D, 1, R, SCHEME, PP, QQ, false>(*P, loc, k, lds);
+            fused_tile<D, 1, R, SCHEME, PP, QQ, false, DIRECT>(*P, loc, k, lds);
         } else if constexpr (D > 2) {
-            fused_tile<D, 2, R, SCHEME, PP, QQ, false>(*P, loc, k, lds);
+            fused_tile<D, 2, R, SCHEME, PP, QQ, false, DIRECT>(*P, loc, k, lds);
         }
     }
 }
@@ -353,20 +458,27 @@ hipError_t launch_single_dsq(const Plan<W>& plan, const KParams& k, hipStream_t 
         // one patch: both flux stages in one launch (stage 2's table holds all axes)
         if (plan.items[2] > 0) {
             const dim3 grid(unsigned((plan.items[2] + kBlock - 1) / kBlock));
-            switch (plan.tile_rows) {
-                case 24:
-                    hipLaunchKernelGGL((k_flux_patch_single<D, 24, SCHEME, PP, QQ, W>), grid, dim3(kBlock), 0, s,
-                                       plan.work[2], k);
-                    break;
-                case 8:
-                    hipLaunchKernelGGL((k_flux_patch_single<D, 8, SCHEME, PP, QQ, W>), grid, dim3(kBlock), 0, s,
-                                       plan.work[2], k);
-                    break;
-                case 4:
-                    hipLaunchKernelGGL((k_flux_patch_single<D, 4, SCHEME, PP, QQ, W>), grid, dim3(kBlock), 0, s,
-                                       plan.work[2], k);
-                    break;
-                default: return hipErrorInvalidValue;
+            auto patch = [&](auto rows, auto direct) {
+                hipLaunchKernelGGL((k_flux_patch_single<D, decltype(rows)::value, SCHEME, PP, QQ, decltype(direct)::value, W>),
+                                   grid, dim3(kBlock), 0, s, plan.work[2], k);
+            };
+            using std::integral_constant;
+            if (plan.direct) {
+                patch(integral_constant<int, 4>{}, std::true_type{});
+            } else if constexpr (D > 1) {  // (1D patches and 2D patches of 4-row tiles are all direct)
+                switch (plan.tile_rows) {
+                    case 24: patch(integral_constant<int, 24>{}, std::false_type{}); break;
+                    case 8: patch(integral_constant<int, 8>{}, std::false_type{}); break;
+                    case 4:
+                        if constexpr (D == 3) {
+                            patch(integral_constant<int, 4>{}, std::false_type{});
+                            break;
+                        }
+                        [[fallthrough]];
+                    default: return hipErrorInvalidValue;
+                }
+            } else {
+                return hipErrorInvalidValue;
             }
         }
         return hipGetLastError();

@@ -565,6 +565,14 @@ class ConvectiveFluxReconstructorGPU {
             w.start[d] = acc;
             plan.items[2] = acc;
             plan.items[3] = 0;
+            // Small calls derive their cells in the flux kernel (one launch
+            // instead of two): every 1D patch (200 cells 14.9 -> 10.7 us, 2e5
+            // 20.7 -> 16.9), 2D patches of 4-row tiles (64^2 16.0 -> 11.8, 128^2
+            // 20.2 -> 16.0, 400^2 41.6 -> 35.8), 3D patches up to 2^18 work items
+            // (16^3 19.7 -> 17.2, 24^3 22.6 -> 22.0; at 32^3, 3.2e5 items, the
+            // six-fold work loses: 30.1 -> 31.3).
+            plan.direct = plan.tile_rows == 4 && (d < 3 || acc <= (int64_t(1) << 18));
+            if (plan.direct) plan.items[0] = 0;
         }
         // advective source cells
         plan.work[4].p = dp;

@@ -9,14 +9,13 @@ namespace hm {
 
 // Dilatation theta and vorticity magnitude Omega of cell (i, j, kk) from
 // second-order central derivatives of the velocity (DerivativeFirstOrder.cpp:
-// 216-228; WCNS56-HLLC-HLL.cpp:626-731 (2D), 1470-1656 (3D)), written to the
-// patch's sensor array.  vel(a, s, v) returns the velocity components v[b] of
-// the face neighbour at side s (+1, -1) along axis a, computed exactly as the
+// 216-228; WCNS56-HLLC-HLL.cpp:626-731 (2D), 1470-1656 (3D)).  vel(a, s, v)
+// returns the velocity components v[b] of the face neighbour at side s (+1, -1) along axis a, computed exactly as the
 // derived-data kernel computes a cell's own velocity, so the values equal
 // those the kernel stores for that neighbour.  Quotients by dx_a use quot,
 // which rounds as the division does.
 template <int D, class Vel>
-__device__ __forceinline__ void sensor_cell(const DevPatch& P, const Boxes<D>& B, int i, int j, int kk, Vel vel) {
+__device__ __forceinline__ void sensor_values(const DevPatch& P, Vel vel, double& theta, double& Omega) {
     double g[3][3];  // d u_b / d x_a
 #pragma unroll
     for (int a = 0; a < D; a++) {
@@ -27,7 +26,6 @@ __device__ __forceinline__ void sensor_cell(const DevPatch& P, const Boxes<D>& B
 #pragma unroll
         for (int b = 0; b < D; b++) g[b][a] = quot(double(1) / double(2) * (vp[b] - vm[b]), P.dx[a], rdx);
     }
-    double theta, Omega;
     if constexpr (D == 2) {
         theta = g[0][0] + g[1][1];
         Omega = fabs(g[1][0] - g[0][1]);
@@ -38,6 +36,13 @@ __device__ __forceinline__ void sensor_cell(const DevPatch& P, const Boxes<D>& B
         const double oz = g[1][0] - g[0][1];
         Omega = sqrt(ox * ox + oy * oy + oz * oz);
     }
+}
+
+// The same, written to the patch's sensor array.
+template <int D, class Vel>
+__device__ __forceinline__ void sensor_cell(const DevPatch& P, const Boxes<D>& B, int i, int j, int kk, Vel vel) {
+    double theta, Omega;
+    sensor_values<D>(P, vel, theta, Omega);
     const int64_t vs = B.vol(kGs);
     const uint32_t ls = uint32_t(B.idx(kGs, i, j, kk));
     stg(P.sens, ls, theta);

@@ -26,6 +26,8 @@
 
 #include <algorithm>
 
+#include <type_traits>
+
 #include "hm_kernels.hpp"
 #include "hm_numerics.hpp"
 #include "hm_sensor.hpp"
@@ -179,6 +181,18 @@ __device__ __forceinline__ void cell_state_multi(const KParams& k, QF&& q, uint3
 // fractions and rho stored too, nine components instead of five, it took 5.30 ms
 // on the uneven 3D five-equation level of 2744 patches, 4.34 ms without them.
 // ----------------------------------------------------------------------------
+// Velocity components of the cell at `at`, from q(e, at): the same bits as
+// cell_state_multi's.
+template <int D, int NS, class QF>
+__device__ __forceinline__ void cell_velocity_multi(QF&& q, uint32_t at, double (&v)[3]) {
+    double rho = double(0);
+#pragma unroll
+    for (int si = 0; si < NS; si++) rho += q(si, at);
+    const double rrho = rcp_rn(rho);
+#pragma unroll
+    for (int b = 0; b < D; b++) v[b] = quot(q(NS + b, at), rho, rrho);
+}
+
 template <int D, int NS, bool FOUR, class W>
 __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
     const int64_t gid = int64_t(rhs_block(k)) * kBlock + threadIdx.x;
@@ -216,13 +230,7 @@ __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
         const uint32_t qs[3] = {1u, uint32_t(P->n[0] + 2 * P->gq[0]),
                                 uint32_t((P->n[0] + 2 * P->gq[0]) * (P->n[1] + 2 * P->gq[1]))};
         sensor_cell<D>(*P, B, i, j, kk, [&](int a, int side, double (&v)[3]) {
-            const uint32_t at = side > 0 ? iq + qs[a] : iq - qs[a];
-            double rn = double(0);
-#pragma unroll
-            for (int si = 0; si < NS; si++) rn += q(si, at);
-            const double rrn = rcp_rn(rn);
-#pragma unroll
-            for (int b = 0; b < D; b++) v[b] = quot(q(NS + b, at), rn, rrn);
+            cell_velocity_multi<D, NS>(q, side > 0 ? iq + qs[a] : iq - qs[a], v);
         });
     }
 }
@@ -307,14 +315,66 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
 // (4357 at 75 % before its loads took scalar bases, a field's loads went out
 // together and the WENO weights lost a quarter of their instructions): 36.4 ms
 // -> 24.2 ms.
-// Midpoint flux Fo of the face normal to axis A between cells (c0, c1, c2)
-// - e_A and (c0, c1, c2), and its HLLC normal velocity u* (five-equation).
-// The prim and sensor arrays are read at 32-bit offsets from per-component
-// bases (every patch's ghost box is below 2^29 cells).
-template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
-__device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
-                                                 const KParams& k, double (&Fo)[Multi<D, NS, FOUR>::NEQ],
-                                                 double& ustar, double* wl) {
+// Stencil and sensor of the face normal to axis A between cells (c0, c1, c2) -
+// e_A and (c0, c1, c2) from the patch's arrays: at 32-bit offsets from
+// wave-uniform bases (every patch's ghost box is below 2^29 cells) that hold the
+// component and the stencil position, so that every load of an array takes the
+// same vector offset.
+template <int D, int NS, bool FOUR, int A>
+struct MemFace {
+    using M = Multi<D, NS, FOUR>;
+    const DevPatch& P;
+    const Boxes<D>& B;
+    int c0, c1, c2;
+    int64_t v4, st, qst;
+    uint32_t off, qoff;
+    __device__ __forceinline__ MemFace(const DevPatch& P_, const Boxes<D>& B_, int c0_, int c1_, int c2_)
+        : P(P_), B(B_), c0(c0_), c1(c1_), c2(c2_) {
+        v4 = B.vol(kGc);
+        st = (A == 0) ? 1 : (A == 1) ? int64_t(B.ext(0, kGc)) : int64_t(B.ext(0, kGc)) * B.ext(1, kGc);
+        off = uint32_t(B.idx(kGc, c0, c1, c2)) * 8u;
+        qst = (A == 0)   ? 1
+              : (A == 1) ? int64_t(P.n[0] + 2 * P.gq[0])
+                         : int64_t(P.n[0] + 2 * P.gq[0]) * (P.n[1] + 2 * P.gq[1]);
+        qoff = uint32_t(q_idx<D>(P, c0, c1, c2)) * 8u;
+    }
+    // derived component / conservative variable at stencil position m (cell i - 3 + m)
+    __device__ __forceinline__ double p(int comp, int m) const {
+        return ldg_byte(ld_constant(&P.prim) + (comp * v4 + (m - 3) * st), off);
+    }
+    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(ld_constant(&P.Q[e]) + (m - 3) * qst, qoff); }
+    // the six values of variable `comp` of V, chosen at run time
+    __device__ __forceinline__ void six(int comp, bool in_q, Six& s) const {
+        const double* base = ld_constant(&P.vb[comp]);
+        const int64_t step = ld_constant(&P.vst[A][in_q ? 1 : 0]);
+        uint32_t o = in_q ? qoff : off;
+        pin_offset(o);
+#pragma unroll
+        for (int m = 0; m < 6; m++) s.v[m] = ldg_byte(base + (m - 3) * step, o);
+    }
+    __device__ __forceinline__ void pin() {
+        pin_offset(off);
+        pin_offset(qoff);
+    }
+    __device__ __forceinline__ void sensor(double (&th)[2], double (&om)[2]) const {
+        const int64_t vs = B.vol(kGs);
+        const uint32_t tR = uint32_t(B.idx(kGs, c0, c1, c2));
+        const uint32_t sts = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGs)) : uint32_t(B.ext(0, kGs) * B.ext(1, kGs));
+        const uint32_t tL = tR - sts;
+        const double* se = ld_constant(&P.sens);
+        th[0] = ldg(se, tL), th[1] = ldg(se, tR);
+        om[0] = ldg(se + vs, tL), om[1] = ldg(se + vs, tR);
+    }
+};
+
+// Midpoint flux Fo of a face normal to axis A from its source (MemFace,
+// TileFace), and its HLLC normal velocity u* (five-equation).  wl: 2 NEQ LDS
+// slots at stride S.  NW wavefronts share the face's fields (wavefront wv takes
+// wv, wv + NW, ..); NW > 1 meets one block barrier and only wavefront 0 goes on
+// to the flux.
+template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ, int S, int NW, class Face>
+__device__ __forceinline__ void midflux_multi_of(Face& face, const KParams& k, double (&Fo)[Multi<D, NS, FOUR>::NEQ],
+                                                 double& ustar, double* wl, int wv = 0) {
     using M = Multi<D, NS, FOUR>;
     constexpr int NEQ = M::NEQ;
     constexpr int NZ = M::NZ;
@@ -322,19 +382,8 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     constexpr int IP = NS + D;   // pressure slot
     constexpr int IZ = NS + D + 1;
 
-    const int64_t v4 = B.vol(kGc);
-    const int64_t st = (A == 0) ? 1 : (A == 1) ? int64_t(B.ext(0, kGc)) : int64_t(B.ext(0, kGc)) * B.ext(1, kGc);
-    uint32_t off = uint32_t(B.idx(kGc, c0, c1, c2)) * 8u;
-    const double* pr = P.prim;
-    // the caller's box
-    const int64_t qst = (A == 0)   ? 1
-                        : (A == 1) ? int64_t(P.n[0] + 2 * P.gq[0])
-                                   : int64_t(P.n[0] + 2 * P.gq[0]) * (P.n[1] + 2 * P.gq[1]);
-    uint32_t qoff = uint32_t(q_idx<D>(P, c0, c1, c2)) * 8u;
-    // component and stencil position in the wave-uniform base, so that every
-    // load of an array takes the same 32-bit vector offset
-    auto ldp = [&](int comp, int m) { return ldg_byte(pr + (comp * v4 + (m - 3) * st), off); };
-    auto ldq = [&](int e, int m) { return ldg_byte(P.Q[e] + (m - 3) * qst, qoff); };
+    auto ldp = [&](int comp, int m) { return face.p(comp, m); };
+    auto ldq = [&](int e, int m) { return face.q(e, m); };
     // variable e of V
     auto ldv = [&](int e, int m) {
         if (e < NS || e > IP) return ldq(e, m);
@@ -363,7 +412,7 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     // of a field are issued before the first use: with one variant per kind of
     // field the compiler waited for each pair of loads in turn and kept the
     // load addresses of all variants in registers.  Each field's two
-    // reconstructed values go to wl[f], wl[NEQ + f] (stride kBlock): the field
+    // reconstructed values go to wl[f], wl[NEQ + f] (stride S): the field
     // index is wave-uniform, so the store is one address add, where storing
     // into a register array by a runtime index would select over every slot.
     const LDConst ldk{k.p, k.q, k.C, k.alpha_tau, k.inv_thr};
@@ -371,13 +420,16 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 #pragma unroll
     for (int m = 0; m < 6; m++) ps[m] = ldp(M::PP, m);
     {
+        // (a field's slots belong to the wavefront that takes it)
+        auto mine = [&](int f) { return NW == 1 || f % NW == wv; };
         const double rc = ra * ca;
         const double irc = div_rn(double(1), rc);
-        wl[0] = -irc;
-        wl[(NEQ - 1) * kBlock] = irc;
+        if (mine(0)) wl[0] = -irc;
+        if (mine(NEQ - 1)) wl[(NEQ - 1) * S] = irc;
         const double rcc = rc * ca, r = rcp_rn(rcc);
 #pragma unroll
-        for (int si = 0; si < NS; si++) wl[(1 + si) * kBlock] = -quot(Zra[si], rcc, r);
+        for (int si = 0; si < NS; si++)
+            if (mine(1 + si)) wl[(1 + si) * S] = -quot(Zra[si], rcc, r);
     }
     // component of V of field f, four bits each
     constexpr uint64_t comps = [] {
@@ -390,31 +442,30 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
         return c;
     }();
 #pragma unroll 1
-    for (int f = 0; f < NEQ; f++) {
+    for (int f = wv; f < NEQ; f += NW) {
         const int comp = int(comps >> (4 * f)) & 15;
         const bool in_q = comp < NS || comp > IP;
-        const double* base = ld_constant(&P.vb[comp]);
-        const int64_t step = ld_constant(&P.vst[A][in_q ? 1 : 0]);
-        uint32_t o = in_q ? qoff : off;
-        pin_offset(o);
         Six s;
-#pragma unroll
-        for (int m = 0; m < 6; m++) s.v[m] = ldg_byte(base + (m - 3) * step, o);
+        face.six(comp, in_q, s);
         if (f <= NS || f == NEQ - 1) {
-            const double cf = wl[f * kBlock];
+            const double cf = wl[f * S];
 #pragma unroll
             for (int m = 0; m < 6; m++) s.v[m] = s.v[m] + cf * ps[m];
         }
         double wm, wp;
         reconstruct_pair<SCHEME, PP, QQ>(s, ldk, wm, wp);
-        wl[f * kBlock] = wm;
-        wl[(NEQ + f) * kBlock] = wp;
+        wl[f * S] = wm;
+        wl[(NEQ + f) * S] = wp;
+    }
+    if constexpr (NW > 1) {
+        __syncthreads();
+        if (wv != 0) return;
     }
     double Wm[NEQ], Wp[NEQ];
 #pragma unroll
     for (int e = 0; e < NEQ; e++) {
-        Wm[e] = wl[e * kBlock];
-        Wp[e] = wl[(NEQ + e) * kBlock];
+        Wm[e] = wl[e * S];
+        Wp[e] = wl[(NEQ + e) * S];
     }
 
     // Back-projection (FlowModelBasicUtilitiesFiveEqnAllaire.cpp:9201-9974).
@@ -446,8 +497,7 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
 
     // Bounds on both sides, else first-order values (WCNS56-HLLC-HLL.cpp:947-1032).
     if (!(bounded_multi<D, NS, FOUR, A>(VL, k) && bounded_multi<D, NS, FOUR, A>(VR, k))) {
-        pin_offset(off);
-        pin_offset(qoff);
+        face.pin();
 #pragma unroll
         for (int e = 0; e < NEQ; e++) {
             VL[e] = ldv(e, 2);
@@ -498,12 +548,10 @@ __device__ __forceinline__ void midflux_multi_at(const DevPatch& P, const Boxes<
     // Sensor (WCNS56-HLLC-HLL.cpp:1066-1113).
     bool use_hll = false;
     if constexpr (D > 1) {
-        const int64_t vs = B.vol(kGs);
-        const uint32_t tR = uint32_t(B.idx(kGs, c0, c1, c2));
-        const uint32_t sts = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGs)) : uint32_t(B.ext(0, kGs) * B.ext(1, kGs));
-        const uint32_t tL = tR - sts;
-        const double th_avg = 0.5 * (ldg(P.sens, tL) + ldg(P.sens, tR));
-        const double om_avg = 0.5 * (ldg(P.sens + vs, tL) + ldg(P.sens + vs, tR));
+        double th[2], om[2];
+        face.sensor(th, om);
+        const double th_avg = 0.5 * (th[0] + th[1]);
+        const double om_avg = 0.5 * (om[0] + om[1]);
         const double sensor = div_rn(-th_avg, fabs(th_avg) + om_avg + kEps);
         use_hll = sensor > 0.65;
     }
@@ -627,7 +675,8 @@ __device__ __forceinline__ void midflux_multi_face(const DevPatch& P, int64_t lo
     if constexpr (A == 2) c2 -= 1;
     double Fo[NEQ];
     double ustar;
-    midflux_multi_at<D, NS, FOUR, A, SCHEME, PP, QQ>(P, B, c0, c1, c2, k, Fo, ustar, wl);
+    MemFace<D, NS, FOUR, A> face(P, B, c0, c1, c2);
+    midflux_multi_of<D, NS, FOUR, A, SCHEME, PP, QQ, kBlock, 1>(face, k, Fo, ustar, wl);
     const int64_t mv = B.mid_vol(A);
     double* out = P.fmid[A];
     const uint32_t l32 = uint32_t(loc);
@@ -690,10 +739,11 @@ __global__ void k_queue_reset(unsigned* queue) {
 template <int D, int NS, int A>
 __device__ __forceinline__ double node_flux_multi(const DevPatch& P, uint32_t q, double ua, double p, int e) {
     constexpr int IP = NS + D;
-    if (e == IP) return ua * (ldg(P.Q[IP], q) + p);
-    if (e == NS + A) return ua * ldg(P.Q[e], q) + p;
+    const double Q = ldg(ld_constant(&P.Q[e]), q);
+    if (e == IP) return ua * (Q + p);
+    if (e == NS + A) return ua * Q + p;
     // partial densities, transverse momentum and volume fractions: u_a * Q
-    return ua * ldg(P.Q[e], q);
+    return ua * Q;
 }
 
 // Output flux of face (c0, c1, c2) along A from the midpoint fluxes of faces
@@ -703,13 +753,14 @@ __device__ __forceinline__ double node_flux_multi(const DevPatch& P, uint32_t q,
 // 2327-2490).
 template <int D, int NS, bool FOUR, int A, class MF, class NF>
 __device__ __forceinline__ void combine_face_multi(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
-                                                   double dt, MF&& m, NF&& nf) {
+                                                   double dt, MF&& m, NF&& nf, int wv = 0, int nw = 1) {
     constexpr int NEQ = Multi<D, NS, FOUR>::NEQ;
     const int64_t fv = B.face_vol(A);
     const uint32_t fi = uint32_t(B.face_idx(A, c0, c1, c2));
     double* out = P.F[A];
 #pragma unroll
     for (int e = 0; e < NEQ; e++) {
+        if (nw > 1 && e % nw != wv) continue;  // (nw wavefronts share the equations)
         const double nL = nf(-1, e), nR = nf(0, e);
         const double mR = m(1, e), mL = m(-1, e), mM = m(0, e);
         stg(out + e * fv, fi,
@@ -727,7 +778,8 @@ __device__ __forceinline__ void cell_node_flux_multi(const DevPatch& P, const Bo
     const int64_t v4 = B.vol(kGc);
     const uint32_t pc = uint32_t(B.idx(kGc, c0, c1, c2));
     const uint32_t q = uint32_t(q_idx<D>(P, c0, c1, c2));
-    const double ua = ldg(P.prim + (M::PU + A) * v4, pc), pr = ldg(P.prim + M::PP * v4, pc);
+    const double* d = ld_constant(&P.prim);
+    const double ua = ldg(d + (M::PU + A) * v4, pc), pr = ldg(d + M::PP * v4, pc);
 #pragma unroll
     for (int e = 0; e < NEQ; e++) nf[e * stride] = node_flux_multi<D, NS, A>(P, q, ua, pr, e);
 }
@@ -835,7 +887,8 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
     if (in) {
         double Fo[NEQ];
         double ustar;
-        midflux_multi_at<D, NS, FOUR, A, SCHEME, PP, QQ>(P, B, c[0], c[1], c[2], k, Fo, ustar, wl);
+        MemFace<D, NS, FOUR, A> face(P, B, c[0], c[1], c[2]);
+        midflux_multi_of<D, NS, FOUR, A, SCHEME, PP, QQ, kBlock, 1>(face, k, Fo, ustar, wl);
 #pragma unroll
         for (int e = 0; e < NEQ; e++) wl[e * kBlock] = Fo[e];
         // node fluxes of the cell right of the face (the right cell of output face j - 1, the left of face j)
@@ -877,10 +930,196 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
 }
 
 // ----------------------------------------------------------------------------
+// The flux stage of one small patch: a block of four wavefronts takes a tile of
+// 64 midpoint faces (mtile_shape with 64 threads), derives the tile's cells and
+// their sensor values into LDS, shares the fields of a face over the wavefronts
+// (NEQ / 4 reconstructions in turn instead of NEQ), lets wavefront 0 form the
+// midpoint fluxes and shares the output faces' equations again.
+// Bound by the latency of one face's chain on a device it cannot fill, so the
+// chain is what it cuts: with the derived-data launch and whole faces per
+// thread an 8^3 five-equation patch took 29.9 us and a 16^3 one 29.6; here 18.9
+// and 21.4.
+// A call that fills the device takes k_flux_multi, whose four times larger
+// tiles share fewer faces and cells.
+// ----------------------------------------------------------------------------
+constexpr int kSmallCells = 144;   // (R + 5) W: at most 9 x 16
+constexpr int kSmallSensor = 80;   // (R + 1) W: at most 5 x 16
+
+// Derived values and sensor of a tile's face in LDS, the others in Q.
+template <int D, int NS, bool FOUR, int A>
+struct TileFace {
+    using M = Multi<D, NS, FOUR>;
+    const DevPatch& P;
+    const double* cells;  // the face's stencil cell 0 (stride cst along A), kSmallCells a component
+    int cst;
+    const double* sens;  // the face's left cell, kSmallSensor a component
+    int64_t qst;
+    uint32_t qoff;
+    __device__ __forceinline__ double p(int comp, int m) const { return cells[comp * kSmallCells + m * cst]; }
+    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(ld_constant(&P.Q[e]) + (m - 3) * qst, qoff); }
+    __device__ __forceinline__ void six(int comp, bool in_q, Six& s) const {
+        if (in_q) {
+            const double* base = ld_constant(&P.Q[comp]);
+            uint32_t o = qoff;
+            pin_offset(o);
+#pragma unroll
+            for (int m = 0; m < 6; m++) s.v[m] = ldg_byte(base + (m - 3) * qst, o);
+        } else {
+            const double* c = cells + (M::PU + comp - NS) * kSmallCells;
+#pragma unroll
+            for (int m = 0; m < 6; m++) s.v[m] = c[m * cst];
+        }
+    }
+    __device__ __forceinline__ void pin() { pin_offset(qoff); }
+    __device__ __forceinline__ void sensor(double (&th)[2], double (&om)[2]) const {
+        th[0] = sens[0], th[1] = sens[cst];
+        om[0] = sens[kSmallSensor], om[1] = sens[kSmallSensor + cst];
+    }
+};
+
+template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
+__device__ __forceinline__ void flux_multi_small_tile(const DevPatch& P, uint32_t tile, const KParams& k, double* wlds,
+                                                      double* cells, double* sens) {
+    using M = Multi<D, NS, FOUR>;
+    constexpr int NEQ = M::NEQ;
+    constexpr int U = (A == 0) ? 1 : 0;  // first axis across
+    constexpr int V = (A == 2) ? 1 : 2;  // second axis across
+    const Boxes<D> B(P);
+    const int nA = B.n[A];
+    const int R = P.tile[A][0], W = P.tile[A][1], ntA = P.tile[A][2];
+    const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
+    const int j0 = int(tA) * (R - 2);
+    const uint32_t qs[3] = {1u, uint32_t(P.n[0] + 2 * P.gq[0]),
+                            uint32_t((P.n[0] + 2 * P.gq[0]) * (P.n[1] + 2 * P.gq[1]))};
+    auto q = [&](int e, uint32_t at) { return ldg(P.Q[e], at); };
+    // number x of a tile's L rows by W columns -> row and column, and its cell
+    auto place = [&](uint32_t x, int L, int& r, int& w) {
+        if constexpr (A == 0) {
+            w = int(x / uint32_t(L));
+            r = int(x) - w * L;
+        } else {
+            r = int(x / uint32_t(W));
+            w = int(x) - r * W;
+        }
+    };
+    auto column = [&](int w, int (&c)[3]) {
+        uint32_t cu, cv;
+        tile_column(tw * uint32_t(W), uint32_t(w), uint32_t(W), uint32_t(B.n[U]), cu, cv);
+        c[U] = int(cu);
+        c[V] = int(cv);
+        return cv < uint32_t(B.n[V]);
+    };
+
+    // The tile's cells j0 - 4 .. j0 + R along A, and beside them (other threads)
+    // the sensor of its cells j0 - 2 .. j0 + R - 2.
+    const uint32_t t = threadIdx.x;
+    const uint32_t ncell = uint32_t((R + 5) * W), nsens = uint32_t((R + 1) * W);
+    const uint32_t s0 = ncell > 128u ? ncell : 128u;
+    int r, w, c[3];
+    if (t < ncell) {
+        place(t, R + 5, r, w);
+        const bool in = column(w, c);
+        c[A] = j0 - 4 + r;
+        if (in && c[A] < nA + kGc) {
+            double Zr[NS], Z[NS], rho, u[3], p, c2;
+            cell_state_multi<D, NS, FOUR>(k, q, uint32_t(q_idx<D>(P, c[0], c[1], c[2])), Zr, Z, rho, u, p, c2);
+#pragma unroll
+            for (int b = 0; b < D; b++) cells[(M::PU + b) * kSmallCells + t] = u[b];
+            cells[M::PP * kSmallCells + t] = p;
+            cells[M::PC * kSmallCells + t] = sqrt(c2);
+        }
+    }
+    if constexpr (D > 1) {
+        if (t >= s0 && t < s0 + nsens) {
+            place(t - s0, R + 1, r, w);
+            const bool in = column(w, c);
+            c[A] = j0 - 2 + r;
+            if (in && c[A] < nA + kGs) {
+                const uint32_t iq = uint32_t(q_idx<D>(P, c[0], c[1], c[2]));
+                double theta, Omega;
+                sensor_values<D>(
+                    P,
+                    [&](int a, int side, double (&v)[3]) {
+                        cell_velocity_multi<D, NS>(q, side > 0 ? iq + qs[a] : iq - qs[a], v);
+                    },
+                    theta, Omega);
+                sens[t - s0] = theta;
+                sens[kSmallSensor + t - s0] = Omega;
+            }
+        }
+    }
+    __syncthreads();
+
+    // This thread's face: lane of the tile; lanes without one take the tile's first.
+    const uint32_t lane = t & 63u;
+    const int wv = __builtin_amdgcn_readfirstlane(int(t >> 6));
+    place(lane, R, r, w);
+    bool in = column(w, c);
+    in = in && lane < uint32_t(R * W) && j0 + r < nA + 3;
+    if (!in) {
+        r = w = 0;
+        column(0, c);
+    }
+    const int j = j0 + r;
+    c[A] = j - 1;
+    const uint32_t qc = uint32_t(q_idx<D>(P, c[0], c[1], c[2]));
+    const int cst = (A == 0) ? 1 : W;
+    const double* mine = cells + ((A == 0) ? w * (R + 5) + r : r * W + w);
+    double* wl = wlds + lane;
+    {
+        TileFace<D, NS, FOUR, A> face{P, mine, cst, sens + ((A == 0) ? w * (R + 1) + r : r * W + w), int64_t(qs[A]), qc * 8u};
+        double Fo[NEQ];
+        double ustar;
+        midflux_multi_of<D, NS, FOUR, A, SCHEME, PP, QQ, 64, 4>(face, k, Fo, ustar, wl, wv);
+        if (wv == 0) {
+#pragma unroll
+            for (int e = 0; e < NEQ; e++) wl[e * 64] = Fo[e];
+            if constexpr (!FOUR) {
+                if (in && (r < R - 2 || int(tA) == ntA - 1))
+                    stg(P.ustar[A], uint32_t(B.mid_idx(A, c[0], c[1], c[2])), ustar);
+            }
+        }
+    }
+    __syncthreads();
+    if (!in || r < 1 || r > R - 2 || j > nA + 1) return;
+    const double uaL = mine[(M::PU + A) * kSmallCells + 2 * cst], uaR = mine[(M::PU + A) * kSmallCells + 3 * cst];
+    const double prL = mine[M::PP * kSmallCells + 2 * cst], prR = mine[M::PP * kSmallCells + 3 * cst];
+    const int step = (A == 0) ? 1 : W;  // lane distance of the neighbouring midpoint faces
+    combine_face_multi<D, NS, FOUR, A>(
+        P, B, c[0], c[1], c[2], kdt(k), [&](int side, int e) { return wl[e * 64 + side * step]; },
+        [&](int side, int e) {
+            return side < 0 ? node_flux_multi<D, NS, A>(P, qc - qs[A], uaL, prL, e)
+                            : node_flux_multi<D, NS, A>(P, qc, uaR, prR, e);
+        },
+        wv, 4);
+}
+
+template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
+__global__ __launch_bounds__(kBlock) void k_flux_multi_small(W w, KParams k) {
+    __shared__ double wlds[2 * Multi<D, NS, FOUR>::NEQ * 64];
+    __shared__ double cells[(D + 2) * kSmallCells];
+    __shared__ double sens[2 * kSmallSensor];
+    const DevPatch* P;
+    int ax;
+    uint32_t tile;
+    if (!find_block(w, rhs_block(k), P, ax, tile)) return;
+    if (ax == 0) {
+        flux_multi_small_tile<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+    } else if constexpr (D > 1) {
+        if (ax == 1) {
+            flux_multi_small_tile<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+        } else if constexpr (D > 2) {
+            flux_multi_small_tile<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------
 // Advective source of the volume-fraction equations (WCNS56-HLLC-HLL.cpp:491-535,
 // 1288-1369, 2492-2650).
 // ----------------------------------------------------------------------------
-template <int D, int NS, class W>
+// DIRECT: no derived data before, the velocities from Q.
+template <int D, int NS, bool DIRECT, class W>
 __global__ __launch_bounds__(kBlock) void k_source_five(W w, KParams k) {
     const int64_t gid = int64_t(rhs_block(k)) * kBlock + threadIdx.x;
     const DevPatch* P;
@@ -895,6 +1134,7 @@ __global__ __launch_bounds__(kBlock) void k_source_five(W w, KParams k) {
     const int kk = (D > 2) ? int(r / uint32_t(B.n[1])) : 0;
     const int64_t v4 = B.vol(kGc);
     const int64_t pc = B.idx(kGc, i, j, kk);
+    const int64_t iq = q_idx<D>(*P, i, j, kk);
     double acc = 0.0;
 #pragma unroll
     for (int a = 0; a < D; a++) {
@@ -903,15 +1143,27 @@ __global__ __launch_bounds__(kBlock) void k_source_five(W w, KParams k) {
         const int64_t m = B.mid_idx(a, i, j, kk);  // face between cells i-1 and i along a
         const double* us = P->ustar[a];
         const double uLL = us[m - mst], uL = us[m], uR = us[m + mst], uRR = us[m + 2 * mst];
-        const double* u = P->prim + a * v4;
-        const double cL = u[pc - st4], cR = u[pc + st4];
+        double cL, cR;
+        if constexpr (DIRECT) {
+            const uint32_t qst = (a == 0) ? 1u
+                                 : (a == 1) ? uint32_t(P->n[0] + 2 * P->gq[0])
+                                            : uint32_t((P->n[0] + 2 * P->gq[0]) * (P->n[1] + 2 * P->gq[1]));
+            auto q = [&](int e, uint32_t at) { return ldg(P->Q[e], at); };
+            double v[3];
+            cell_velocity_multi<D, NS>(q, uint32_t(iq) - qst, v);
+            cL = v[a];
+            cell_velocity_multi<D, NS>(q, uint32_t(iq) + qst, v);
+            cR = v[a];
+        } else {
+            const double* u = P->prim + a * v4;
+            cL = u[pc - st4], cR = u[pc + st4];
+        }
         const double term = (double(3) / double(2) * (uR - uL) - double(3) / double(10) * (cR - cL) +
                              double(1) / double(30) * (uRR - uLL)) /
                             P->dx[a];
         acc = (a == 0) ? term : acc + term;
     }
     const int64_t svol = int64_t(B.n[0]) * B.n[1] * B.n[2];
-    const int64_t iq = q_idx<D>(*P, i, j, kk);
 #pragma unroll
     for (int si = 0; si < NS - 1; si++) {
         const int e = NS + D + 1 + si;
@@ -932,6 +1184,7 @@ unsigned nblocks(const Plan<W>& plan, int stage) {
 
 template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
 hipError_t launch_multi_dsq(const Plan<W>& plan, const KParams& k, hipStream_t s) {
+    constexpr bool all_direct = D == 1 && std::is_same_v<W, SegSingle>;  // every 1D patch derives in the flux stage
     if (plan.items[0] > 0)
         hipLaunchKernelGGL((k_derived_multi<D, NS, FOUR, W>), dim3(nblocks(plan, 0)), dim3(kBlock), 0, s,
                            plan.work[0], k);
@@ -954,6 +1207,14 @@ hipError_t launch_multi_dsq(const Plan<W>& plan, const KParams& k, hipStream_t s
             hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, k.queue);
             hipLaunchKernelGGL((k_midflux_multi_queue<D, NS, FOUR, SCHEME, PP, QQ, W>),
                                dim3(std::min(nwork, resident)), dim3(kBlock), 0, s, plan.work[2], k, uint32_t(nwork));
+        } else if (plan.direct) {
+            if constexpr (std::is_same_v<W, SegSingle>)
+                hipLaunchKernelGGL((k_flux_multi_small<D, NS, FOUR, SCHEME, PP, QQ, W>), dim3(nblocks(plan, 2)),
+                                   dim3(kBlock), 0, s, plan.work[2], k);
+            else
+                return hipErrorInvalidValue;
+        } else if constexpr (all_direct) {
+            return hipErrorInvalidValue;
         } else {
             // fused midpoint and face flux over tiles (stage 3 is then empty)
             hipLaunchKernelGGL((k_flux_multi<D, NS, FOUR, SCHEME, PP, QQ, W>), dim3(nblocks(plan, 2)), dim3(kBlock),
@@ -964,9 +1225,20 @@ hipError_t launch_multi_dsq(const Plan<W>& plan, const KParams& k, hipStream_t s
         hipLaunchKernelGGL((k_faceflux_multi<D, NS, FOUR, W>), dim3(nblocks(plan, 3)), dim3(kBlock), 0, s,
                            plan.work[3], k);
     if constexpr (!FOUR) {
-        if (plan.items[4] > 0)
-            hipLaunchKernelGGL((k_source_five<D, NS, W>), dim3(nblocks(plan, 4)), dim3(kBlock), 0, s, plan.work[4],
-                               k);
+        if (plan.items[4] > 0) {
+            auto source = [&](auto direct) {
+                hipLaunchKernelGGL((k_source_five<D, NS, decltype(direct)::value, W>), dim3(nblocks(plan, 4)),
+                                   dim3(kBlock), 0, s, plan.work[4], k);
+            };
+            if constexpr (std::is_same_v<W, SegSingle>) {
+                if (plan.direct)
+                    source(std::true_type{});
+                else
+                    source(std::false_type{});
+            } else {
+                source(std::false_type{});
+            }
+        }
     }
     return hipGetLastError();
 }

@@ -574,6 +574,31 @@ class ConvectiveFluxReconstructorGPU {
             plan.direct = plan.tile_rows == 4 && (d < 3 || acc <= (int64_t(1) << 18));
             if (plan.direct) plan.items[0] = 0;
         }
+        if (!fused_) {
+            const int nn[3] = {v.n[0], d > 1 ? v.n[1] : 1, d > 2 ? v.n[2] : 1};
+            // A small patch takes 64-face tiles that derive their cells (five
+            // equations, WCNS6-LD: 8^3 29.9 -> 18.9 us, 16^3 29.6 -> 21.4, 24^3
+            // 30.1 -> 26.0, 28^3, 294 tiles of 256 faces, 36.0 -> 32.5, 128^2
+            // 28.0 -> 20.5, 256^2, 640 tiles, 39.2 -> 35.5) until the device is
+            // full of the larger tiles: 32^3 with 441 of them 37.5 -> 38.8, 64^3
+            // 130 -> 171, 320^2 with 960 47.2 -> 47.6.  A 1D patch has one column,
+            // which fills a quarter of a 256-face tile: 2e5 cells 42.9 -> 33.7.
+            plan.direct = d == 1 || plan.items[2] <= int64_t(kBlock) * (d == 2 ? 640 : 400);
+            if (plan.direct) {
+                SegSingle& w = plan.work[2];
+                int64_t acc = 0;
+                for (int a = 0; a < d; a++) {
+                    int* t = w.p.tile[a];
+                    mtile_shape(nn[a], t[0], t[1], t[2], true, d);
+                    w.start[a] = acc;
+                    w.cnt[a] = mtile_items(a, nn, d, true);
+                    acc += w.cnt[a];
+                }
+                w.start[d] = acc;
+                plan.items[2] = acc;
+                plan.items[0] = 0;
+            }
+        }
         // advective source cells
         plan.work[4].p = dp;
         plan.work[4].nseg = 1;

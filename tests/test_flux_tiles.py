@@ -12,7 +12,7 @@ from oracle import oracle as O
 
 def _shape(nA, kind):
     """Rows, columns and tiles per column: mtile_shape of hm_kernels.hpp, dtile_shape of hm_diffusive.hpp."""
-    threads, most, shared = {"flux": (256, 62, 2), "diff": (512, 74, 11), "diff1d": (512, 501, 11)}[kind]
+    threads, most, shared = {"flux": (256, 62, 2), "small": (64, 14, 2), "small1d": (64, 62, 2), "diff": (512, 74, 11), "diff1d": (512, 501, 11)}[kind]
     nt = (nA + 1 + most - 1) // most
     R = (nA + 1 + nt - 1) // nt + shared
     return R, threads // R, nt, threads, shared
@@ -29,7 +29,15 @@ def test_small_divisions_are_exact():
         assert np.array_equal(_div(x, d), x // d), d
 
 
-@pytest.mark.parametrize("kind", ["flux", "diff", "diff1d"])
+def test_small_tiles_fit_their_block():
+    """Cells and sensor cells of a 64-face tile: one thread and one LDS slot each."""
+    for nA, kind in [(n, kind) for kind in ("small", "small1d") for n in range(1, 2000)]:
+        R, W = _shape(nA, kind)[:2]
+        cells, sensor = (R + 5) * W, (R + 1) * W
+        assert R * W <= 64 and cells <= 144 and sensor <= 80 and max(cells, 128) + sensor <= 256, nA
+
+
+@pytest.mark.parametrize("kind", ["flux", "small", "small1d", "diff", "diff1d"])
 @pytest.mark.parametrize("axis", [0, 1])
 def test_tiles_cover_every_face_once(axis, kind):
     for nA in (1, 2, 7, 8, 61, 62, 64, 73, 74, 123, 124, 125, 148, 200, 500, 501, 502):
@@ -58,7 +66,7 @@ def test_tiles_cover_every_face_once(axis, kind):
                 inside = (lane < R * Wd) & (j < nA + 1 + shared) & (tv < nV)
                 col = tv * nU + cu
                 np.add.at(mid, (col[inside], j[inside]), 1)
-                if kind == "flux":
+                if kind in ("flux", "small", "small1d"):
                     writes, face = inside & (r >= 1) & (r <= R - 2) & (j <= nA + 1), j - 1
                 else:
                     writes, face = inside & (r >= 6) & (r <= R - 6) & (j - 6 <= nA), j - 6

@@ -1,10 +1,10 @@
-"""One patch of the single-species model: small calls derive their cells in the
-flux kernel.  On both sides of the rule and at odd extents the results equal the
-batched pipeline's and the oracle's to the bit (the same operations in the same
-order on each cell)."""
+"""Calls on one patch: small ones derive their cells in the flux kernel.  On both
+sides of the rule and at odd extents the results equal the batched pipeline's and
+the oracle's to the bit (the same operations in the same order on each cell)."""
 import numpy as np
 import pytest
 
+from hamers_amd import workloads as W
 from oracle import oracle as O
 
 
@@ -15,7 +15,7 @@ from oracle import oracle as O
 def test_patch_equals_batch_and_oracle(n, scheme):
     import torch
 
-    from hamers_amd import ConvectiveFluxReconstructor, PatchData
+    from hamers_amd import ConvectiveFluxReconstructor
 
     assert torch.cuda.is_available(), "GPU tests need a visible GPU"
     d, gam = len(n), 1.4
@@ -31,12 +31,54 @@ def test_patch_equals_batch_and_oracle(n, scheme):
     rec = ConvectiveFluxReconstructor("direct", d, "SINGLE_SPECIES", "WCNS6_LD_HLLC_HLL" if scheme else "WCNS5_JS_HLLC_HLL",
                                       num_species=1, species_gamma=(gam,), species_R=(1.0,))
     prm = O.Params(dim=d, model=O.SINGLE_SPECIES, num_species=1, scheme=scheme, gamma=[gam], R=[1.0])
-    want = O.rhs_patch(prm, Q, n, g, dx, dt)[0]
-    cut = tuple(slice(g - w, s - (g - w)) for w, s in zip(reversed(ghost), shp))
+    _check(rec, prm, Q, n, ghost, dx, dt, f"single {n} scheme {scheme}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", [1, 0], ids=["WCNS6_LD", "WCNS5_JS"])
+@pytest.mark.parametrize("model", ["FIVE_EQN_ALLAIRE", "FOUR_EQN_CONSERVATIVE"])
+@pytest.mark.parametrize("n", [(1,), (500,), (1, 1), (131, 3), (13, 29), (1, 1, 1), (3, 15, 30), (13, 14, 16),
+                               (33, 32, 34)], ids=str)
+def test_multi_species_patch_equals_batch_and_oracle(n, model, scheme):
+    import torch
+
+    from hamers_amd import ConvectiveFluxReconstructor
+
+    assert torch.cuda.is_available(), "GPU tests need a visible GPU"
+    d, five, gamma = len(n), model == "FIVE_EQN_ALLAIRE", (1.4, 1.67)
+    ghost = (5, 4, 6)[:d]
+    g = max(ghost)
+    rng = np.random.default_rng(sum(n) + scheme)
+    shp = tuple(v + 2 * g for v in reversed(n))
+    Z = 0.5 + 0.45 * rng.uniform(-1, 1, shp)
+    vel = [0.8 * rng.uniform(-1, 1, shp) for _ in range(d)]
+    p = rng.uniform(0.5, 2.0, shp)
+    R = (1.0, 1.0 if five else 2.0)
+    if five:
+        Q = W.conservative_from_primitive_five([Z, 0.3 * (1 - Z)], vel, p, [Z, 1 - Z], gamma)
+    else:
+        Q = W.conservative_from_primitive_four([Z, 0.3 * (1 - Z)], vel, p, gamma, R)
+    dx, dt = tuple(1.0 / v for v in n), 1e-3
+    rec = ConvectiveFluxReconstructor("direct", d, model, "WCNS6_LD_HLLC_HLL" if scheme else "WCNS5_JS_HLLC_HLL",
+                                      num_species=2, species_gamma=gamma, species_R=R)
+    prm = O.Params(dim=d, model=O.FIVE_EQN_ALLAIRE if five else O.FOUR_EQN_CONSERVATIVE, num_species=2, scheme=scheme,
+                   gamma=list(gamma), R=list(R))
+    _check(rec, prm, Q, n, ghost, dx, dt, f"{model} {n} scheme {scheme}")
+
+
+def _check(rec, prm, Q, n, ghost, dx, dt, name):
+    import torch
+
+    from hamers_amd import PatchData
+
+    d, g = len(n), max(ghost)
+    Fr, Sr = O.rhs_patch(prm, Q, n, g, dx, dt)
+    cut = tuple(slice(g - w, s - (g - w)) for w, s in zip(reversed(ghost), Q.shape[1:]))
     dev = torch.from_numpy(np.ascontiguousarray(Q[(slice(None),) + cut])).to("cuda:0")
     for batched in (False, True):
         F = [torch.full(O.face_shape(rec.num_eqn, n, a), np.nan, dtype=torch.float64, device="cuda:0") for a in range(d)]
-        pd = PatchData(n, ghost, dx, dev, F, None)
+        S = torch.zeros((rec.num_eqn,) + tuple(reversed(n)), dtype=torch.float64, device="cuda:0")
+        pd = PatchData(n, ghost, dx, dev, F, S)
         if batched:
             rec.computeConvectiveFluxAndSourceOnPatches([pd], 0.0, dt)
         else:
@@ -44,5 +86,7 @@ def test_patch_equals_batch_and_oracle(n, scheme):
         torch.cuda.synchronize()
         for a in range(d):
             got = F[a].cpu().numpy()
-            print(f"{n} scheme {scheme} batched {batched} axis {a}: {int(np.sum(got != want[a]))} differ", flush=True)
-            assert np.array_equal(got, want[a])
+            print(f"{name} batched {batched} axis {a}: {int(np.sum(got != Fr[a]))} differ", flush=True)
+            assert np.array_equal(got, Fr[a])
+        if Sr is not None:
+            assert np.array_equal(S.cpu().numpy(), Sr)

@@ -47,11 +47,11 @@ FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 (vector and matrix)
 HEADLINE_KERNEL_COUNTS = {
     "k_flux_multi": {
         "cells": 68726784,
-        # 64 x (4 082 214 738 + 6 044 320 354 + 443 484 271 + 2 x 3 195 942 072)
-        "fp64_ops": 64 * (4082214738 + 6044320354 + 443484271 + 2 * 3195942072),
-        # FETCH_SIZE 54 973 956 KiB x 2.0 + WRITE_SIZE 26 786 422 KiB x 1.0 (includes the 72 B/lane spill)
-        "dram_bytes": 54973956 * 1024 * 2 + 26786422 * 1024,
-        "valu_issue_frac": 0.755,
+        # 64 x (3 183 943 166 + 5 225 870 196 + 173 290 695 + 2 x 1 816 869 361)
+        "fp64_ops": 64 * (3183943166 + 5225870196 + 173290695 + 2 * 1816869361),
+        # FETCH_SIZE 14 264 514 KiB x 2.0 + WRITE_SIZE 13 681 375 KiB x 1.0
+        "dram_bytes": 14264514 * 1024 * 2 + 13681375 * 1024,
+        "valu_issue_frac": 0.841,
         "source": "profiles/rhs_uneven3d_five_eqn_counters.md",
     },
 }
@@ -418,7 +418,7 @@ def bench_2d(args, torch, np):
             "flux_kernel": {"kernel": STAGE_KERNEL_SINGLE.get(dominant, dominant), "kernel_ms": stage[dominant],
                             "bytes_per_cell": 8 * (neq + neq), "achieved_gbs": kgbs, "hbm_frac": kgbs / HBM_PEAK_GBS,
                             "traffic": traffic, "bound": "valu",
-                            "counts_source": "profiles/flux_kernels_2048sq_counters.md (73-77 % of VALU issue)"},
+                            "counts_source": "profiles/flux_kernels_2048sq_counters.md (72-79 % of VALU issue)"},
             "rhs_hbm_frac": 8 * (neq + 2 * neq) * cells / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
 
 

@@ -311,10 +311,10 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
 }
 
 // Bound by VALU issue: on the uneven 3D five-equation level of 2744 patches the
-// fused flux issues 3246 VALU instructions per wavefront at 82 % of the rate
+// fused flux issues 3193 VALU instructions per wavefront at 84 % of the rate
 // (4357 at 75 % before its loads took scalar bases, a field's loads went out
 // together and the WENO weights lost a quarter of their instructions): 36.4 ms
-// -> 24.2 ms.
+// -> 24.0 ms.
 // Stencil and sensor of the face normal to axis A between cells (c0, c1, c2) -
 // e_A and (c0, c1, c2) from the patch's arrays: at 32-bit offsets from
 // wave-uniform bases (every patch's ghost box is below 2^29 cells) that hold the

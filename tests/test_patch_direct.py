@@ -36,16 +36,17 @@ def test_patch_equals_batch_and_oracle(n, scheme):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("scheme", [1, 0], ids=["WCNS6_LD", "WCNS5_JS"])
-@pytest.mark.parametrize("model", ["FIVE_EQN_ALLAIRE", "FOUR_EQN_CONSERVATIVE"])
+@pytest.mark.parametrize("model,ns", [("FIVE_EQN_ALLAIRE", 2), ("FOUR_EQN_CONSERVATIVE", 2), ("FIVE_EQN_ALLAIRE", 3),
+                                      ("FOUR_EQN_CONSERVATIVE", 3)])
 @pytest.mark.parametrize("n", [(1,), (500,), (1, 1), (131, 3), (13, 29), (1, 1, 1), (3, 15, 30), (13, 14, 16),
                                (33, 32, 34)], ids=str)
-def test_multi_species_patch_equals_batch_and_oracle(n, model, scheme):
+def test_multi_species_patch_equals_batch_and_oracle(n, model, ns, scheme):
     import torch
 
     from hamers_amd import ConvectiveFluxReconstructor
 
     assert torch.cuda.is_available(), "GPU tests need a visible GPU"
-    d, five, gamma = len(n), model == "FIVE_EQN_ALLAIRE", (1.4, 1.67)
+    d, five, gamma = len(n), model == "FIVE_EQN_ALLAIRE", (1.4, 1.67, 1.3)[:ns]
     ghost = (5, 4, 6)[:d]
     g = max(ghost)
     rng = np.random.default_rng(sum(n) + scheme)
@@ -53,17 +54,19 @@ def test_multi_species_patch_equals_batch_and_oracle(n, model, scheme):
     Z = 0.5 + 0.45 * rng.uniform(-1, 1, shp)
     vel = [0.8 * rng.uniform(-1, 1, shp) for _ in range(d)]
     p = rng.uniform(0.5, 2.0, shp)
-    R = (1.0, 1.0 if five else 2.0)
+    R = (1.0, 1.0 if five else 2.0, 1.0 if five else 0.5)[:ns]
+    Zs = [Z, 1 - Z] if ns == 2 else [Z, 0.6 * (1 - Z), 0.4 * (1 - Z)]
+    rhos = [r * z for r, z in zip((1.0, 0.3, 0.7), Zs)]
     if five:
-        Q = W.conservative_from_primitive_five([Z, 0.3 * (1 - Z)], vel, p, [Z, 1 - Z], gamma)
+        Q = W.conservative_from_primitive_five(rhos, vel, p, Zs, gamma)
     else:
-        Q = W.conservative_from_primitive_four([Z, 0.3 * (1 - Z)], vel, p, gamma, R)
+        Q = W.conservative_from_primitive_four(rhos, vel, p, gamma, R)
     dx, dt = tuple(1.0 / v for v in n), 1e-3
     rec = ConvectiveFluxReconstructor("direct", d, model, "WCNS6_LD_HLLC_HLL" if scheme else "WCNS5_JS_HLLC_HLL",
-                                      num_species=2, species_gamma=gamma, species_R=R)
-    prm = O.Params(dim=d, model=O.FIVE_EQN_ALLAIRE if five else O.FOUR_EQN_CONSERVATIVE, num_species=2, scheme=scheme,
+                                      num_species=ns, species_gamma=gamma, species_R=R)
+    prm = O.Params(dim=d, model=O.FIVE_EQN_ALLAIRE if five else O.FOUR_EQN_CONSERVATIVE, num_species=ns, scheme=scheme,
                    gamma=list(gamma), R=list(R))
-    _check(rec, prm, Q, n, ghost, dx, dt, f"{model} {n} scheme {scheme}")
+    _check(rec, prm, Q, n, ghost, dx, dt, f"{model} ns={ns} {n} scheme {scheme}")
 
 
 def _check(rec, prm, Q, n, ghost, dx, dt, name):

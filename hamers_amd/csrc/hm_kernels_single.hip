@@ -12,6 +12,7 @@
 //                       879-1194, 1746-2320) and the sixth-order midpoint-to-face
 //                       flux times dt (1197-1282, 2327-2490), fused per wavefront
 //   k_flux_tile_single  axes 1 and 2: the same, fused per 64 x 24 tile
+//   k_flux_both_single  small batched calls: both in one launch
 //   k_flux_patch_single one patch: all axes in one launch, and for a small
 //                       patch the derived cell data too
 #include <type_traits>
@@ -418,6 +419,35 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SCHEME =
     }
 }
 
+// Small batched calls: the tiles of axes 1 and 2 (the first nb3 blocks) and axis
+// 0's chunks behind them in one launch.  Each of the two alone is one or two
+// rounds of resident blocks and ends in a partly filled one: 512^2 in 16 patches
+// (WCNS6-LD, 704 tiles and 1104 chunk blocks on 768 places) took 32.4 + 26.8 us
+// and takes 49.4; WCNS5-JS, whose chunks alone run at 4 wavefronts per SIMD
+// instead of the tiles' 3, gains as well (the whole call 53.0 -> 46.8 us).  From
+// 24-row tiles on a call has rounds enough and the chunks keep their 4.
+template <int D, int R, int SCHEME, int PP, int QQ, class W, bool REC>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SCHEME == kWCNS5_JS && D == 2 ? HM_TILE_WAVES : 1))) void k_flux_both_single(
+    W w3, W w2, uint32_t nb3, KParams k) {
+    if constexpr (D > 1) {
+        __shared__ double lds[R * kTileX * (D + 2)];
+        const bool tiles = blockIdx.x < nb3;
+        const uint32_t b = tiles ? blockIdx.x : blockIdx.x - nb3, nb = tiles ? nb3 : gridDim.x - nb3;
+        const int64_t gid = int64_t(k.xcd ? xcd_block(b, nb) : b) * kBlock + threadIdx.x;
+        const DevPatch* P;
+        int ax;
+        int64_t loc;
+        if (!(tiles ? w3 : w2).find(gid, P, ax, loc)) return;  // (tile segments are whole blocks)
+        if (ax == 0) {
+            fused_chunk<D, 0, SCHEME, PP, QQ, REC>(*P, loc, k);
+        } else if (ax == 1) {
+            fused_tile<D, 1, R, SCHEME, PP, QQ, REC>(*P, loc, k, lds);
+        } else if constexpr (D > 2) {
+            fused_tile<D, 2, R, SCHEME, PP, QQ, REC>(*P, loc, k, lds);
+        }
+    }
+}
+
 // One patch (the per-patch entry point): axis 0's chunks and the tiles of axes
 // 1 and 2 in one launch, so that the two flux stages of a small call overlap
 // instead of running one after the other.  The axis-0 segment is padded to a
@@ -484,29 +514,38 @@ hipError_t launch_single_dsq(const Plan<W>& plan, const KParams& k, hipStream_t 
         return hipGetLastError();
     } else {
         const bool rec = k.wrec != nullptr;  // recording runs (patch tables only)
-        if (plan.items[2] > 0) {
-            const dim3 grid(unsigned((plan.items[2] + kBlock - 1) / kBlock));
+        const unsigned nb2 = unsigned((plan.items[2] + kBlock - 1) / kBlock);
+        const unsigned nb3 = unsigned((plan.items[3] + kBlock - 1) / kBlock);
+        // Tiles of fewer rows are a small call's (tile_rows_for), or asked for.
+        const bool both = D > 1 && plan.tile_rows != 24 && nb3 > 0;
+        if (nb2 > 0 && !both) {
             if (rec)
-                hipLaunchKernelGGL((k_flux_single<D, SCHEME, PP, QQ, W, true>), grid, dim3(kBlock), 0, s, plan.work[2], k);
+                hipLaunchKernelGGL((k_flux_single<D, SCHEME, PP, QQ, W, true>), dim3(nb2), dim3(kBlock), 0, s, plan.work[2], k);
             else
-                hipLaunchKernelGGL((k_flux_single<D, SCHEME, PP, QQ, W>), grid, dim3(kBlock), 0, s, plan.work[2], k);
+                hipLaunchKernelGGL((k_flux_single<D, SCHEME, PP, QQ, W>), dim3(nb2), dim3(kBlock), 0, s, plan.work[2], k);
         }
-        if (plan.items[3] > 0) {
-            if constexpr (D > 1) {
-                const dim3 grid(unsigned((plan.items[3] + kBlock - 1) / kBlock));
-                auto tiles = [&](auto rows) {
-                    constexpr int R = decltype(rows)::value;
-                    if (rec)
-                        hipLaunchKernelGGL((k_flux_tile_single<D, R, SCHEME, PP, QQ, W, true>), grid, dim3(kBlock), 0, s,
-                                           plan.work[3], k);
-                    else
-                        hipLaunchKernelGGL((k_flux_tile_single<D, R, SCHEME, PP, QQ, W>), grid, dim3(kBlock), 0, s,
-                                           plan.work[3], k);
-                };
+        if constexpr (D > 1) {
+            auto launch_both = [&](auto rows) {
+                constexpr int R = decltype(rows)::value;
+                if (rec)
+                    hipLaunchKernelGGL((k_flux_both_single<D, R, SCHEME, PP, QQ, W, true>), dim3(nb3 + nb2), dim3(kBlock),
+                                       0, s, plan.work[3], plan.work[2], nb3, k);
+                else
+                    hipLaunchKernelGGL((k_flux_both_single<D, R, SCHEME, PP, QQ, W, false>), dim3(nb3 + nb2), dim3(kBlock),
+                                       0, s, plan.work[3], plan.work[2], nb3, k);
+            };
+            if (nb3 > 0) {
                 switch (plan.tile_rows) {
-                    case 24: tiles(std::integral_constant<int, 24>{}); break;
-                    case 8: tiles(std::integral_constant<int, 8>{}); break;
-                    case 4: tiles(std::integral_constant<int, 4>{}); break;
+                    case 24:
+                        if (rec)
+                            hipLaunchKernelGGL((k_flux_tile_single<D, 24, SCHEME, PP, QQ, W, true>), dim3(nb3),
+                                               dim3(kBlock), 0, s, plan.work[3], k);
+                        else
+                            hipLaunchKernelGGL((k_flux_tile_single<D, 24, SCHEME, PP, QQ, W>), dim3(nb3), dim3(kBlock), 0,
+                                               s, plan.work[3], k);
+                        break;
+                    case 8: launch_both(std::integral_constant<int, 8>{}); break;
+                    case 4: launch_both(std::integral_constant<int, 4>{}); break;
                     default: return hipErrorInvalidValue;
                 }
             }

@@ -132,7 +132,8 @@ __global__ __launch_bounds__(kBlock) void k_rk_accumulate(W w, AccTerms t) {
 
 template <class W>
 hipError_t launch_rk_accumulate(int dim, const W& acc, int64_t acc_items, const AccTerms& terms, hipStream_t s) {
-    if (acc_items <= 0 || terms.n == 0) return hipSuccess;
+    // (sums that start at zero are written by a tableau without gamma too: they would keep the last step's)
+    if (acc_items <= 0 || (terms.n == 0 && !terms.init)) return hipSuccess;
     const unsigned na = unsigned((acc_items + kBlock - 1) / kBlock);
     switch (dim) {
         case 1: hipLaunchKernelGGL((k_rk_accumulate<1, W>), dim3(na), dim3(kBlock), 0, s, acc, terms); break;

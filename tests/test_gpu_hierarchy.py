@@ -13,7 +13,9 @@ restatement (oracle/amr.py, pinned in test_oracle_amr.py).
   two fine patches, one coarse step; 2D with REFLECT / FLOW x sides.
 Coarse and fine states: max-norm relative error <= 1e-12 (FP64; the
 restatement keeps the kernels' operation order).  The GPU result keeps the
-composite sums of the conserved variables to rounding.  Errors: misaligned
+composite sums of the conserved variables to rounding.  A step with a tableau
+without gamma takes nothing over from the step before it: the same bits as a
+hierarchy that starts there.  Errors: misaligned
 fine boxes, a ratio other than 2, and destroying a level that a hierarchy uses.
 """
 import ctypes
@@ -218,3 +220,60 @@ def test_two_level_2d_navier_stokes_walls(torch_dev):
           0.2 * dx[0], 2, 0, "2D four-equation Navier-Stokes, REFLECT / FLOW x sides, fine patches against both",
           bc=bc, transport=NS_TR)
     del diff
+
+
+def _tableau_cases():
+    from tests.test_oracle_amr import NS_TR, ns_state
+
+    Qi, n, dx = W.density_wave_convergence(16, dim=2)
+    yield ("2D single species", Qi, n, dx, O.Params(dim=2, model=O.SINGLE_SPECIES, scheme=1), lambda: (_rec(2), None),
+           [((i, j), (8, 8)) for j in (0, 8) for i in (0, 8)], [((8, 8), (12, 16)), ((20, 8), (4, 8))], None)
+    Qi, n, dx = W.interface_advection_convergence(8, dim=3)
+    prm = O.Params(dim=3, model=O.FIVE_EQN_ALLAIRE, num_species=2, scheme=0, gamma=[1.6, 1.4])
+    yield ("3D five-equation", Qi, n, dx, prm,
+           lambda: (_rec(3, "FIVE_EQN_ALLAIRE", "WCNS5_JS_HLLC_HLL", 2, (1.6, 1.4)), None),
+           [((0, 0, 0), (8, 8, 4)), ((0, 0, 4), (8, 8, 4))], [((4, 4, 2), (6, 8, 10)), ((10, 4, 2), (4, 4, 10))], None)
+    Qi, n, dx, prm = ns_state(16)
+    yield ("2D Navier-Stokes", Qi, n, dx, prm, lambda: _ns_context(prm), [((0, 0), (16, 16))],
+           [((8, 8), (12, 14)), ((20, 10), (6, 8))], NS_TR)
+
+
+@pytest.mark.parametrize("case", range(3), ids=["single_2d", "five_3d", "navier_stokes_2d"])
+def test_tableau_without_gamma_after_a_step(torch_dev, case):
+    """gamma is optional: without it a step's flux and source sums are zero, also
+    after a step that had them."""
+    from hamers_amd import Hierarchy
+    from hamers_amd.integrator import SSP_RK3_ALPHA as a, SSP_RK3_BETA as b
+
+    label, Qi, n, dx, prm, context, coarse, fine, transport = list(_tableau_cases())[case]
+    _say(f"case: {label}, SSP-RK3 without gamma after a step with it")
+    rec, diff = context()
+    T = amr.TwoLevel(prm, n, dx, fine, transport=transport)
+    dt = 0.2 * dx[0]
+
+    def hierarchy(Q, patches):
+        C, F = _levels(rec, n, dx, coarse, fine, T)
+        C.write_global(Q)
+        for i, q in enumerate(patches):
+            F.write_patch(i, q)
+        return Hierarchy(C, F), C, F
+
+    def state(C, F):
+        torch_dev.cuda.synchronize()
+        return [C.read_global(Qi.shape)] + [F.read_patch(i) for i in range(len(fine))]
+
+    H, C, F = hierarchy(Qi, T.refine_patches(Qi))
+    H.advance(dt, 1)
+    mid = state(C, F)
+    for lvl in (C, F):
+        lvl.set_rk_coefficients(a, b)
+    H.advance(dt, 2)
+    got = state(C, F)
+    H2, C2, F2 = hierarchy(mid[0], mid[1:])
+    for lvl in (C2, F2):
+        lvl.set_rk_coefficients(a, b)
+    H2.advance(dt, 2)
+    ref = state(C2, F2)
+    _say(f"  {label}: max rel err {max(max_rel_err(x, y) for x, y in zip(got, ref)):.3e}")
+    assert all(np.array_equal(x, y) for x, y in zip(got, ref))
+    del H, H2, diff

@@ -148,16 +148,26 @@ __device__ __forceinline__ const T* as_constant(const T* p) {
     return (const T*)(ctype*)p;
 }
 
-// One wave-uniform word of such memory by a runtime index, as a scalar load.
-template <class T>
-__device__ __forceinline__ T ld_constant(const T* p) {
-    typedef __attribute__((address_space(4))) const uint64_t cword;
-    static_assert(sizeof(T) == sizeof(uint64_t));
-    return (T)*(cword*)p;
+// A word of a patch of the work W, by a runtime index or after a store: a scalar
+// load where the patch lies in a table (as_constant).  A patch that travels by
+// value is read as it is: its address is constant memory only as long as the
+// compiler makes no copy of the parameter, which is the compiler's to decide
+// (it did for kernels that read the patch in a loop around a barrier, whose
+// constant reads then went to no meaningful address).
+template <class W, class T>
+__device__ __forceinline__ T ld_field(const T& f) {
+    if constexpr (W::kTable) {
+        typedef __attribute__((address_space(4))) const uint64_t cword;
+        static_assert(sizeof(T) == sizeof(uint64_t));
+        return (T)*(cword*)&f;
+    } else {
+        return f;
+    }
 }
 
 template <class T>
 struct SegSingleT {  // one patch, up to 4 segments (one per axis, one extra), all by value
+    static constexpr bool kTable = false;
     T p;
     int64_t start[5];
     int64_t cnt[4];
@@ -176,6 +186,7 @@ struct SegSingleT {  // one patch, up to 4 segments (one per axis, one extra), a
 
 template <class T>
 struct SegTableT {  // many patches: device arrays
+    static constexpr bool kTable = true;
     const T* patches;
     const int64_t* start;  // nseg + 1 entries
     const int64_t* cnt;    // nseg entries

@@ -320,7 +320,7 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
 // wave-uniform bases (every patch's ghost box is below 2^29 cells) that hold the
 // component and the stencil position, so that every load of an array takes the
 // same vector offset.
-template <int D, int NS, bool FOUR, int A>
+template <int D, int NS, bool FOUR, int A, class W>
 struct MemFace {
     using M = Multi<D, NS, FOUR>;
     const DevPatch& P;
@@ -340,13 +340,13 @@ struct MemFace {
     }
     // derived component / conservative variable at stencil position m (cell i - 3 + m)
     __device__ __forceinline__ double p(int comp, int m) const {
-        return ldg_byte(ld_constant(&P.prim) + (comp * v4 + (m - 3) * st), off);
+        return ldg_byte(ld_field<W>(P.prim) + (comp * v4 + (m - 3) * st), off);
     }
-    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(ld_constant(&P.Q[e]) + (m - 3) * qst, qoff); }
+    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(ld_field<W>(P.Q[e]) + (m - 3) * qst, qoff); }
     // the six values of variable `comp` of V, chosen at run time
     __device__ __forceinline__ void six(int comp, bool in_q, Six& s) const {
-        const double* base = ld_constant(&P.vb[comp]);
-        const int64_t step = ld_constant(&P.vst[A][in_q ? 1 : 0]);
+        const double* base = ld_field<W>(P.vb[comp]);
+        const int64_t step = ld_field<W>(P.vst[A][in_q ? 1 : 0]);
         uint32_t o = in_q ? qoff : off;
         pin_offset(o);
 #pragma unroll
@@ -361,7 +361,7 @@ struct MemFace {
         const uint32_t tR = uint32_t(B.idx(kGs, c0, c1, c2));
         const uint32_t sts = (A == 0) ? 1u : (A == 1) ? uint32_t(B.ext(0, kGs)) : uint32_t(B.ext(0, kGs) * B.ext(1, kGs));
         const uint32_t tL = tR - sts;
-        const double* se = ld_constant(&P.sens);
+        const double* se = ld_field<W>(P.sens);
         th[0] = ldg(se, tL), th[1] = ldg(se, tR);
         om[0] = ldg(se + vs, tL), om[1] = ldg(se + vs, tR);
     }
@@ -660,7 +660,7 @@ __device__ __forceinline__ void midflux_multi_of(Face& face, const KParams& k, d
 
 // Midpoint face `loc` (numbered with x fastest over faces -1..n_A+1 along A)
 // of the unfused pipeline: its flux to fmid[A], u* to ustar[A].
-template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
+template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ, class W>
 __device__ __forceinline__ void midflux_multi_face(const DevPatch& P, int64_t loc, const KParams& k, double* wl) {
     constexpr int NEQ = Multi<D, NS, FOUR>::NEQ;
     const Boxes<D> B(P);
@@ -675,7 +675,7 @@ __device__ __forceinline__ void midflux_multi_face(const DevPatch& P, int64_t lo
     if constexpr (A == 2) c2 -= 1;
     double Fo[NEQ];
     double ustar;
-    MemFace<D, NS, FOUR, A> face(P, B, c0, c1, c2);
+    MemFace<D, NS, FOUR, A, W> face(P, B, c0, c1, c2);
     midflux_multi_of<D, NS, FOUR, A, SCHEME, PP, QQ, kBlock, 1>(face, k, Fo, ustar, wl);
     const int64_t mv = B.mid_vol(A);
     double* out = P.fmid[A];
@@ -709,12 +709,12 @@ k_midflux_multi_queue(W w, KParams k, uint32_t nwork) {
         int64_t loc;
         if (w.find(gid, P, ax, loc)) {
             if (ax == 0) {
-                midflux_multi_face<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, loc, k, wl);
+                midflux_multi_face<D, NS, FOUR, 0, SCHEME, PP, QQ, W>(*P, loc, k, wl);
             } else if constexpr (D > 1) {
                 if (ax == 1) {
-                    midflux_multi_face<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, loc, k, wl);
+                    midflux_multi_face<D, NS, FOUR, 1, SCHEME, PP, QQ, W>(*P, loc, k, wl);
                 } else if constexpr (D > 2) {
-                    midflux_multi_face<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, loc, k, wl);
+                    midflux_multi_face<D, NS, FOUR, 2, SCHEME, PP, QQ, W>(*P, loc, k, wl);
                 }
             }
         }
@@ -736,10 +736,10 @@ __global__ void k_queue_reset(unsigned* queue) {
 // FlowModelFourEqnConservative.cpp:5499-5700) along A, from its conservative
 // variables at `q` in the Q box (below 2^29 cells) and its velocity ua along A
 // and pressure p.
-template <int D, int NS, int A>
+template <int D, int NS, int A, class W>
 __device__ __forceinline__ double node_flux_multi(const DevPatch& P, uint32_t q, double ua, double p, int e) {
     constexpr int IP = NS + D;
-    const double Q = ldg(ld_constant(&P.Q[e]), q);
+    const double Q = ldg(ld_field<W>(P.Q[e]), q);
     if (e == IP) return ua * (Q + p);
     if (e == NS + A) return ua * Q + p;
     // partial densities, transverse momentum and volume fractions: u_a * Q
@@ -770,7 +770,7 @@ __device__ __forceinline__ void combine_face_multi(const DevPatch& P, const Boxe
 }
 
 // Node fluxes of the cell (c0, c1, c2) along A, nf[e] for every equation.
-template <int D, int NS, bool FOUR, int A>
+template <int D, int NS, bool FOUR, int A, class W>
 __device__ __forceinline__ void cell_node_flux_multi(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
                                                      double* nf, int stride) {
     using M = Multi<D, NS, FOUR>;
@@ -778,14 +778,14 @@ __device__ __forceinline__ void cell_node_flux_multi(const DevPatch& P, const Bo
     const int64_t v4 = B.vol(kGc);
     const uint32_t pc = uint32_t(B.idx(kGc, c0, c1, c2));
     const uint32_t q = uint32_t(q_idx<D>(P, c0, c1, c2));
-    const double* d = ld_constant(&P.prim);
+    const double* d = ld_field<W>(P.prim);
     const double ua = ldg(d + (M::PU + A) * v4, pc), pr = ldg(d + M::PP * v4, pc);
 #pragma unroll
-    for (int e = 0; e < NEQ; e++) nf[e * stride] = node_flux_multi<D, NS, A>(P, q, ua, pr, e);
+    for (int e = 0; e < NEQ; e++) nf[e * stride] = node_flux_multi<D, NS, A, W>(P, q, ua, pr, e);
 }
 
 // Output flux of face (c0, c1, c2) along A with the node fluxes formed here.
-template <int D, int NS, bool FOUR, int A, class MF>
+template <int D, int NS, bool FOUR, int A, class W, class MF>
 __device__ __forceinline__ void store_face_multi(const DevPatch& P, const Boxes<D>& B, int c0, int c1, int c2,
                                                  double dt, MF&& m) {
     using M = Multi<D, NS, FOUR>;
@@ -799,12 +799,13 @@ __device__ __forceinline__ void store_face_multi(const DevPatch& P, const Boxes<
     const double uaL = ldg(P.prim + (M::PU + A) * v4, pL), uaR = ldg(P.prim + (M::PU + A) * v4, pR);
     const double prL = ldg(P.prim + M::PP * v4, pL), prR = ldg(P.prim + M::PP * v4, pR);
     combine_face_multi<D, NS, FOUR, A>(P, B, c0, c1, c2, dt, m, [&](int side, int e) {
-        return side < 0 ? node_flux_multi<D, NS, A>(P, qL, uaL, prL, e) : node_flux_multi<D, NS, A>(P, qR, uaR, prR, e);
+        return side < 0 ? node_flux_multi<D, NS, A, W>(P, qL, uaL, prL, e)
+                        : node_flux_multi<D, NS, A, W>(P, qR, uaR, prR, e);
     });
 }
 
 // Output face `loc` of the unfused pipeline, from the midpoint fluxes in fmid[A].
-template <int D, int NS, bool FOUR, int A>
+template <int D, int NS, bool FOUR, int A, class W>
 __device__ __forceinline__ void faceflux_multi_face(const DevPatch& P, int64_t loc, const KParams& k) {
     const Boxes<D> B(P);
     const int f0 = B.face_ext(A, 0), f1 = B.face_ext(A, 1);
@@ -817,8 +818,8 @@ __device__ __forceinline__ void faceflux_multi_face(const DevPatch& P, int64_t l
     const uint32_t mC = uint32_t(B.mid_idx(A, c0, c1, c2));
     const uint32_t mst = (A == 0) ? 1u : (A == 1) ? uint32_t(B.mid_ext(A, 0)) : uint32_t(B.mid_ext(A, 0) * B.mid_ext(A, 1));
     const double* fm = P.fmid[A];
-    store_face_multi<D, NS, FOUR, A>(P, B, c0, c1, c2, kdt(k),
-                                     [&](int side, int e) { return ldg(fm + e * mv, mC + uint32_t(side) * mst); });
+    store_face_multi<D, NS, FOUR, A, W>(P, B, c0, c1, c2, kdt(k),
+                                        [&](int side, int e) { return ldg(fm + e * mv, mC + uint32_t(side) * mst); });
 }
 
 template <int D, int NS, bool FOUR, class W>
@@ -829,12 +830,12 @@ __global__ __launch_bounds__(kBlock) void k_faceflux_multi(W w, KParams k) {
     int64_t loc;
     if (!w.find(gid, P, ax, loc)) return;
     if (ax == 0) {
-        faceflux_multi_face<D, NS, FOUR, 0>(*P, loc, k);
+        faceflux_multi_face<D, NS, FOUR, 0, W>(*P, loc, k);
     } else if constexpr (D > 1) {
         if (ax == 1) {
-            faceflux_multi_face<D, NS, FOUR, 1>(*P, loc, k);
+            faceflux_multi_face<D, NS, FOUR, 1, W>(*P, loc, k);
         } else if constexpr (D > 2) {
-            faceflux_multi_face<D, NS, FOUR, 2>(*P, loc, k);
+            faceflux_multi_face<D, NS, FOUR, 2, W>(*P, loc, k);
         }
     }
 }
@@ -855,7 +856,7 @@ __global__ __launch_bounds__(kBlock) void k_faceflux_multi(W w, KParams k) {
 // first R - 2 faces, and the last tile of a column all of its faces).
 static_assert(kBlock == 256, "a fused multi-species tile is one 256-thread block");
 
-template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
+template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ, class Work>
 __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile, const KParams& k, double* wlds) {
     constexpr int NEQ = Multi<D, NS, FOUR>::NEQ;
     const Boxes<D> B(P);
@@ -887,12 +888,12 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
     if (in) {
         double Fo[NEQ];
         double ustar;
-        MemFace<D, NS, FOUR, A> face(P, B, c[0], c[1], c[2]);
+        MemFace<D, NS, FOUR, A, Work> face(P, B, c[0], c[1], c[2]);
         midflux_multi_of<D, NS, FOUR, A, SCHEME, PP, QQ, kBlock, 1>(face, k, Fo, ustar, wl);
 #pragma unroll
         for (int e = 0; e < NEQ; e++) wl[e * kBlock] = Fo[e];
         // node fluxes of the cell right of the face (the right cell of output face j - 1, the left of face j)
-        cell_node_flux_multi<D, NS, FOUR, A>(P, B, c[0], c[1], c[2], wl + NEQ * kBlock, kBlock);
+        cell_node_flux_multi<D, NS, FOUR, A, Work>(P, B, c[0], c[1], c[2], wl + NEQ * kBlock, kBlock);
         if constexpr (!FOUR) {
             if (int(r) < R - 2 || int(tA) == ntA - 1)
                 stg(P.ustar[A], uint32_t(B.mid_idx(A, c[0], c[1], c[2])), ustar);
@@ -919,12 +920,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
     uint32_t tile;
     if (!find_block(w, rhs_block(k), P, ax, tile)) return;
     if (ax == 0) {
-        flux_multi_tile<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, tile, k, wlds);
+        flux_multi_tile<D, NS, FOUR, 0, SCHEME, PP, QQ, W>(*P, tile, k, wlds);
     } else if constexpr (D > 1) {
         if (ax == 1) {
-            flux_multi_tile<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, tile, k, wlds);
+            flux_multi_tile<D, NS, FOUR, 1, SCHEME, PP, QQ, W>(*P, tile, k, wlds);
         } else if constexpr (D > 2) {
-            flux_multi_tile<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, tile, k, wlds);
+            flux_multi_tile<D, NS, FOUR, 2, SCHEME, PP, QQ, W>(*P, tile, k, wlds);
         }
     }
 }
@@ -956,10 +957,10 @@ struct TileFace {
     int64_t qst;
     uint32_t qoff;
     __device__ __forceinline__ double p(int comp, int m) const { return cells[comp * kSmallCells + m * cst]; }
-    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(ld_constant(&P.Q[e]) + (m - 3) * qst, qoff); }
+    __device__ __forceinline__ double q(int e, int m) const { return ldg_byte(P.Q[e] + (m - 3) * qst, qoff); }
     __device__ __forceinline__ void six(int comp, bool in_q, Six& s) const {
         if (in_q) {
-            const double* base = ld_constant(&P.Q[comp]);
+            const double* base = P.Q[comp];
             uint32_t o = qoff;
             pin_offset(o);
 #pragma unroll
@@ -977,7 +978,7 @@ struct TileFace {
     }
 };
 
-template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ>
+template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ, class Work>
 __device__ __forceinline__ void flux_multi_small_tile(const DevPatch& P, uint32_t tile, const KParams& k, double* wlds,
                                                       double* cells, double* sens) {
     using M = Multi<D, NS, FOUR>;
@@ -1088,8 +1089,8 @@ __device__ __forceinline__ void flux_multi_small_tile(const DevPatch& P, uint32_
     combine_face_multi<D, NS, FOUR, A>(
         P, B, c[0], c[1], c[2], kdt(k), [&](int side, int e) { return wl[e * 64 + side * step]; },
         [&](int side, int e) {
-            return side < 0 ? node_flux_multi<D, NS, A>(P, qc - qs[A], uaL, prL, e)
-                            : node_flux_multi<D, NS, A>(P, qc, uaR, prR, e);
+            return side < 0 ? node_flux_multi<D, NS, A, Work>(P, qc - qs[A], uaL, prL, e)
+                            : node_flux_multi<D, NS, A, Work>(P, qc, uaR, prR, e);
         },
         wv, 4);
 }
@@ -1104,12 +1105,12 @@ __global__ __launch_bounds__(kBlock) void k_flux_multi_small(W w, KParams k) {
     uint32_t tile;
     if (!find_block(w, rhs_block(k), P, ax, tile)) return;
     if (ax == 0) {
-        flux_multi_small_tile<D, NS, FOUR, 0, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+        flux_multi_small_tile<D, NS, FOUR, 0, SCHEME, PP, QQ, W>(*P, tile, k, wlds, cells, sens);
     } else if constexpr (D > 1) {
         if (ax == 1) {
-            flux_multi_small_tile<D, NS, FOUR, 1, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+            flux_multi_small_tile<D, NS, FOUR, 1, SCHEME, PP, QQ, W>(*P, tile, k, wlds, cells, sens);
         } else if constexpr (D > 2) {
-            flux_multi_small_tile<D, NS, FOUR, 2, SCHEME, PP, QQ>(*P, tile, k, wlds, cells, sens);
+            flux_multi_small_tile<D, NS, FOUR, 2, SCHEME, PP, QQ, W>(*P, tile, k, wlds, cells, sens);
         }
     }
 }
@@ -1184,31 +1185,37 @@ unsigned nblocks(const Plan<W>& plan, int stage) {
 
 template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
 hipError_t launch_multi_dsq(const Plan<W>& plan, const KParams& k, hipStream_t s) {
-    constexpr bool all_direct = D == 1 && std::is_same_v<W, SegSingle>;  // every 1D patch derives in the flux stage
+    constexpr bool one = std::is_same_v<W, SegSingle>;
+    constexpr bool all_direct = D == 1 && one;  // every 1D patch derives in the flux stage
     if (plan.items[0] > 0)
         hipLaunchKernelGGL((k_derived_multi<D, NS, FOUR, W>), dim3(nblocks(plan, 0)), dim3(kBlock), 0, s,
                            plan.work[0], k);
     // (stage 1 is empty: the derived-data kernel computes the dilatation and vorticity)
     if (plan.items[2] > 0) {
         if (plan.persistent) {
-            // unfused: midpoint faces from the work queue here, output faces in stage 3
-            if (!k.queue) return hipErrorInvalidValue;
-            // resident blocks of this kernel on the device (queried once per instance)
-            static const unsigned resident = [] {
-                int dev = 0, cus = 0, per_cu = 0;
-                (void)hipGetDevice(&dev);
-                (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-                (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void*>(&k_midflux_multi_queue<D, NS, FOUR, SCHEME, PP, QQ, W>),
-                    kBlock, 0);
-                return unsigned(std::max(1, cus) * std::max(1, per_cu));
-            }();
-            const unsigned nwork = nblocks(plan, 2);
-            hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, k.queue);
-            hipLaunchKernelGGL((k_midflux_multi_queue<D, NS, FOUR, SCHEME, PP, QQ, W>),
-                               dim3(std::min(nwork, resident)), dim3(kBlock), 0, s, plan.work[2], k, uint32_t(nwork));
+            // unfused: midpoint faces from the work queue here, output faces in stage 3 (patch lists only)
+            if constexpr (one) {
+                return hipErrorInvalidValue;
+            } else {
+                if (!k.queue) return hipErrorInvalidValue;
+                // resident blocks of this kernel on the device (queried once per instance)
+                static const unsigned resident = [] {
+                    int dev = 0, cus = 0, per_cu = 0;
+                    (void)hipGetDevice(&dev);
+                    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+                    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                        &per_cu, reinterpret_cast<const void*>(&k_midflux_multi_queue<D, NS, FOUR, SCHEME, PP, QQ, W>),
+                        kBlock, 0);
+                    return unsigned(std::max(1, cus) * std::max(1, per_cu));
+                }();
+                const unsigned nwork = nblocks(plan, 2);
+                hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, k.queue);
+                hipLaunchKernelGGL((k_midflux_multi_queue<D, NS, FOUR, SCHEME, PP, QQ, W>),
+                                   dim3(std::min(nwork, resident)), dim3(kBlock), 0, s, plan.work[2], k,
+                                   uint32_t(nwork));
+            }
         } else if (plan.direct) {
-            if constexpr (std::is_same_v<W, SegSingle>)
+            if constexpr (one)
                 hipLaunchKernelGGL((k_flux_multi_small<D, NS, FOUR, SCHEME, PP, QQ, W>), dim3(nblocks(plan, 2)),
                                    dim3(kBlock), 0, s, plan.work[2], k);
             else
@@ -1221,16 +1228,20 @@ hipError_t launch_multi_dsq(const Plan<W>& plan, const KParams& k, hipStream_t s
                                0, s, plan.work[2], k);
         }
     }
-    if (plan.items[3] > 0)
-        hipLaunchKernelGGL((k_faceflux_multi<D, NS, FOUR, W>), dim3(nblocks(plan, 3)), dim3(kBlock), 0, s,
-                           plan.work[3], k);
+    if (plan.items[3] > 0) {
+        if constexpr (one)
+            return hipErrorInvalidValue;
+        else
+            hipLaunchKernelGGL((k_faceflux_multi<D, NS, FOUR, W>), dim3(nblocks(plan, 3)), dim3(kBlock), 0, s,
+                               plan.work[3], k);
+    }
     if constexpr (!FOUR) {
         if (plan.items[4] > 0) {
             auto source = [&](auto direct) {
                 hipLaunchKernelGGL((k_source_five<D, NS, decltype(direct)::value, W>), dim3(nblocks(plan, 4)),
                                    dim3(kBlock), 0, s, plan.work[4], k);
             };
-            if constexpr (std::is_same_v<W, SegSingle>) {
+            if constexpr (one) {
                 if (plan.direct)
                     source(std::true_type{});
                 else

@@ -21,6 +21,13 @@ namespace hm {
 
 constexpr double kEps = 1.0e-15;  // HAMERS_EPSILON, include/HAMeRS_config.hpp.in:16
 
+// The hardware reciprocal estimate.  A host build divides, unless it defines
+// HM_RCP_ESTIMATE(b), an estimate of its own: then it follows the device's
+// division step by step.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define HM_RCP_ESTIMATE(b) __builtin_amdgcn_rcp(b)
+#endif
+
 // Correctly rounded FP64 division in fewer instructions than the compiler's
 // general sequence, for operands whose quotient and remainder are normal
 // numbers (every quotient of the scheme: denominators are state values or
@@ -35,11 +42,15 @@ constexpr double kEps = 1.0e-15;  // HAMERS_EPSILON, include/HAMeRS_config.hpp.i
 // scaling and special-value fixup, so a zero dividend gives +0 for -0 and a
 // zero divisor gives NaN; neither reaches a branch of the scheme.  Checked bit
 // for bit against a / b on the GPU over 1e10 random operand pairs (exponents
-// -80..79) and by the parity tests against the oracle's IEEE divisions.  Host
-// builds divide.
+// -80..79), on the host with a perturbed estimate over 2e7 pairs (all-ones
+// significands and near-midpoint quotients included) and by the parity tests
+// against the oracle's IEEE divisions.  Reciprocals of several denominators
+// from one estimate of their product (each then 2 or 3 units off) gave other
+// last places for significands of all ones and overflowed for indicators past
+// 1e100; they saved 1 % of a right-hand side.
 HM_HD double rcp_rn(double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const double r = __builtin_amdgcn_rcp(b);
+#if defined(HM_RCP_ESTIMATE)
+    const double r = HM_RCP_ESTIMATE(b);
     const double e = fma(-b, r, 1.0);
     return fma(r, fma(e, e, e), r);
 #else
@@ -48,7 +59,7 @@ HM_HD double rcp_rn(double b) {
 }
 
 HM_HD double quot(double a, double b, double r) {
-#if defined(__HIP_DEVICE_COMPILE__)
+#if defined(HM_RCP_ESTIMATE)
     const double q0 = a * r;
     return fma(fma(-b, q0, a), r, q0);
 #else
@@ -62,8 +73,8 @@ HM_HD double quot(double a, double b, double r) {
 // stencils just above the indicators' rounding noise the sweep magnifies that
 // to 1e-3 of a gradient, so it keeps this form's bits.
 HM_HD double rcp_two(double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    double r = __builtin_amdgcn_rcp(b);
+#if defined(HM_RCP_ESTIMATE)
+    double r = HM_RCP_ESTIMATE(b);
     double e = fma(-b, r, 1.0);
     r = fma(r, e, r);
     e = fma(-b, r, 1.0);
@@ -74,30 +85,6 @@ HM_HD double rcp_two(double b) {
 }
 
 HM_HD double div_rn(double a, double b) { return quot(a, b, rcp_rn(b)); }
-
-// Reciprocals of several denominators from one hardware estimate (it issues at
-// a quarter of the FMA rate): the reciprocal of their product, times the other
-// factors.  They are within 2 (pair) and 3 (triple) units in the last place,
-// not rounded to nearest, and are meant for quot only: its correction leaves
-// an error of at most a few reciprocal errors times 2^-53 of a unit in the
-// last place before the final rounding (below 2^-48), so a quotient rounds
-// like a / b unless it lies that close to the midpoint of two numbers (none
-// seen in 1e10 random quotients).  The products stay normal numbers for
-// factors between 1e-100 and 1e100.
-HM_HD void rcp_pair(double a, double b, double& ra, double& rb) {
-    const double r = rcp_rn(a * b);
-    ra = r * b;
-    rb = r * a;
-}
-
-HM_HD void rcp_triple(double a, double b, double c, double& ra, double& rb, double& rc) {
-    const double ab = a * b;
-    const double r = rcp_rn(ab * c);
-    const double rab = r * c;
-    ra = rab * b;
-    rb = rab * a;
-    rc = r * ab;
-}
 
 // Whether cond holds on every active lane of the wavefront (host builds: cond).
 HM_HD bool wave_all(bool cond) {
@@ -244,13 +231,11 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
                    double(25) / double(256) * s.v[4] + double(3) / double(256) * s.v[5];
     }
 
-    double r0, r1, r2, r3;
-    rcp_pair(e0, e1, r0, r1);
-    rcp_pair(e2, e3, r2, r3);
+    const double r0 = rcp_rn(e0), r1 = rcp_rn(e1), r2 = rcp_rn(e2);
     double w0 = k.C + rep_pow<Q>(quot(tau6, e0, r0), k.q);
     double w1 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e1, r1), k.q));
     double w2 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e2, r2), k.q));
-    double w3 = k.C + rep_pow<Q>(quot(tau6, e3, r3), k.q);
+    double w3 = k.C + rep_pow<Q>(div_rn(tau6, e3), k.q);
     const double ws = w0 + w1 + w2 + w3;
     const double rws = rcp_rn(ws);
     w0 = quot(w0, ws, rws);
@@ -286,28 +271,14 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
 }
 
 // One side of WCNS5-JS (WCNS5-JS-HLLC-HLL.cpp:78-118; plus side 124-164 on
-// flip(s)).  With the default exponent 2 the three reciprocals of (beta_k +
-// eps)^2 are squares of reciprocals from one estimate (rcp_triple).
+// flip(s)).
 template <int P>
 HM_HD double js_side(const Six& s, int p_rt) {
     double b0, b1, b2;
     beta3(s, b0, b1, b2);
-    const double e0 = b0 + kEps, e1 = b1 + kEps, e2 = b2 + kEps;
-    const double d0 = rep_pow<P>(e0, p_rt), d1 = rep_pow<P>(e1, p_rt), d2 = rep_pow<P>(e2, p_rt);
-    double r0, r1, r2;
-    if constexpr (P == 2) {
-        rcp_triple(e0, e1, e2, r0, r1, r2);
-        r0 *= r0;
-        r1 *= r1;
-        r2 *= r2;
-    } else {
-        r0 = rcp_rn(d0);
-        r1 = rcp_rn(d1);
-        r2 = rcp_rn(d2);
-    }
-    double w0 = quot(double(1.0) / double(16), d0, r0);
-    double w1 = quot(double(5.0) / double(8), d1, r1);
-    double w2 = quot(double(5.0) / double(16), d2, r2);
+    double w0 = div_rn(double(1.0) / double(16), rep_pow<P>((b0 + kEps), p_rt));
+    double w1 = div_rn(double(5.0) / double(8), rep_pow<P>((b1 + kEps), p_rt));
+    double w2 = div_rn(double(5.0) / double(16), rep_pow<P>((b2 + kEps), p_rt));
     const double ws = w0 + w1 + w2;
     const double rws = rcp_rn(ws);
     w0 = quot(w0, ws, rws);

@@ -1,10 +1,12 @@
-"""WCNS midpoint interpolation: the kernels' rearranged weights (shared
-reciprocals, exact products taken into FMAs, constant weights where the ratios
-vanish in the sum with C, the upwind switch decided without its quotient)
-against the formulas written out term by term, bit for bit: on the host over
-random stencils (wcns_weights_check.cpp), and on the GPU against the oracle
-over the scheme constants that turn the constant-weight rule on and off, on a
-patch whose wavefronts hold resolved data, rough data and both."""
+"""WCNS midpoint interpolation: the kernels' rearranged weights (exact products
+taken into FMAs, constant weights where the ratios vanish in the sum with C, the
+upwind switch decided without its quotient) against the formulas written out
+term by term, bit for bit: on the host over random stencils
+(wcns_weights_check.cpp), with the host's division and with the device's
+(estimate, Newton step, corrected quotient) followed step by step, and on the
+GPU against the oracle over the scheme constants that turn the constant-weight
+rule on and off, on a patch whose wavefronts hold resolved data, rough data and
+both, in units up to pressures of 1e75."""
 import os
 import shutil
 import subprocess
@@ -19,9 +21,10 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_host_weights_match_plain_formulas(tmp_path):
+@pytest.mark.parametrize("division", [[], ["-DDEVICE_DIVISION"]], ids=["host_division", "device_division"])
+def test_host_weights_match_plain_formulas(tmp_path, division):
     exe = tmp_path / "weights_check"
-    subprocess.check_call(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-Wno-unknown-pragmas",
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-Wno-unknown-pragmas", *division,
                            os.path.join(ROOT, "tests", "wcns_weights_check.cpp"), "-o", str(exe)])
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     print(out.stdout)
@@ -33,10 +36,13 @@ CONSTANTS = [(1, 2, 4, 1e9, 35.0), (1, 2, 4, 1.0, 35.0), (1, 2, 4, 1e9, 1e-3), (
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("scale", [1.0, 1e7])
+@pytest.mark.parametrize("scale", [1.0, 1e7, 1e75])
 @pytest.mark.parametrize("scheme,p,q,C,alpha", CONSTANTS)
 def test_constants_against_oracle(scheme, p, q, C, alpha, scale):
-    """Same bits as the oracle (its quotients and sums round as the kernel's do); pressures scaled to 1e7 as in SI units."""
+    """Same bits as the oracle (its quotients and sums round as the kernel's do); pressures scaled to 1e7 as in SI
+    units, and to 1e75, where the default exponent's powers of the indicators (1e150) are still numbers."""
+    if scale > 1e70 and (p, q) != (2, 4):
+        pytest.skip("the powers overflow")
     import torch
 
     from hamers_amd import ConvectiveFluxReconstructor, PatchData

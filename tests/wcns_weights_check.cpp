@@ -2,12 +2,30 @@
 // reference's formulas written out term by term (WCNS6-LD-HLLC-HLL.cpp:24-223,
 // WCNS5-JS-HLLC-HLL.cpp:32-118; no fused multiply-add, no constant weights),
 // bit for bit, over stencils from rough to resolved and over scheme constants
-// that do and do not admit the constant-weight rule.  Prints the number of
-// differing values and how often the rule held; exits 1 on any difference.
+// that do and do not admit the constant-weight rule, with the exponents at
+// compile time and at run time.  Prints the number of differing values and how
+// often the rule held; exits 1 on any difference.
+//
+// Built with -DDEVICE_DIVISION it runs the device's division instead of the
+// host's: reciprocals refined from an estimate that is off by up to 2^-24.3
+// either way (the bound measured on gfx950) and quotients corrected by FMAs.
+// That division is checked by itself too, against a / b.
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 
+#if defined(DEVICE_DIVISION)
+static uint64_t estimate_state = 0x9e3779b97f4a7c15ull;
+static double estimate(double b) {
+    estimate_state ^= estimate_state << 13;
+    estimate_state ^= estimate_state >> 7;
+    estimate_state ^= estimate_state << 17;
+    const double off = 2.0 * (double(estimate_state >> 11) / 9007199254740992.0) - 1.0;
+    return 1.0 / b * (1.0 + off * 4.84e-8);  // 2^-24.3 = 4.84e-8
+}
+#define HM_RCP_ESTIMATE(b) estimate(b)
+#endif
 #include "../hamers_amd/csrc/hm_numerics.hpp"
 
 using namespace hm;
@@ -72,7 +90,52 @@ static double plain_js(const double* u, int p) {
            1.0 / 8.0 * w[2] * u[4];
 }
 
+static bool differs(double a, double b) { return std::memcmp(&a, &b, 8) != 0 && !(a != a && b != b); }
+
+// Both sides of a field against the plain values pm, pp.
+template <int SCHEME, int P, int Q>
+static int wrong(const Six& s, const LDConst& k, double pm, double pp) {
+    double um, up;
+    reconstruct_pair<SCHEME, P, Q>(s, k, um, up);
+    return differs(um, pm) + differs(up, pp);
+}
+
+#if defined(DEVICE_DIVISION)
+// A positive number of random exponent in [-range, range]; a quarter of them
+// with all ones below the leading bits, or nearly so.
+static double operand(int range) {
+    double m = 1.0 + 0.5 * (rnd() + 1.0);
+    uint64_t b;
+    std::memcpy(&b, &m, 8);
+    const int how = int(state >> 40) & 7;
+    if (how == 0) b |= (uint64_t(1) << 52) - 1;
+    if (how == 1) b |= (uint64_t(1) << 50) - 1, b ^= (state >> 20) & 3;
+    std::memcpy(&m, &b, 8);
+    return std::ldexp(m, int(range * rnd()));
+}
+
+// The quotient by a refined reciprocal is a / b to the last place, all-ones
+// significands and quotients made to lie next to the midpoint of two numbers
+// (a within half a unit of b times it) among them.
+static int check_division() {
+    long bad = 0;
+    const long count = 10000000;
+    for (long it = 0; it < count; it++) {
+        const int range = it % 2 ? 60 : 420;
+        const double a = operand(range), b = operand(range), q = operand(3);
+        bad += differs(quot(a, b, rcp_rn(b)), a / b);
+        const double near = double(((long double)q + 0.5L * (std::nextafter(q, 1e300) - q)) * b);
+        bad += differs(div_rn(near, b), near / b);
+    }
+    std::printf("division: %ld of %ld quotients differ\n", bad, 2 * count);
+    return bad != 0;
+}
+#endif
+
 int main() {
+#if defined(DEVICE_DIVISION)
+    if (check_division()) return 1;
+#endif
     struct Set {
         int p, q;
         double C, alpha;
@@ -87,30 +150,31 @@ int main() {
         for (int it = 0; it < 200000; it++) {
             // polynomial data of a random resolution, noise of a random size and offset
             const double h = std::pow(10.0, -3.0 * std::fabs(rnd())), noise = it % 3 ? std::pow(10.0, -16.0 * std::fabs(rnd())) : 0.0;
-            const double off0 = it % 5 ? rnd() : 0.0, a1 = rnd(), a2 = rnd(), a3 = rnd(), scale = it % 7 ? 1.0 : 1e8;
+            const double off0 = it % 5 ? rnd() : 0.0, a1 = rnd(), a2 = rnd(), a3 = rnd();
+            // (indicators of 1e120 and 1e156: no product of two of them, or of their squares, is a number)
+            const double scale = it % 7 == 0 ? 1e8 : it % 77 == 1 ? 1e60 : it % 77 == 2 ? 1e78 : 1.0;
             Six s;
             for (int m = 0; m < 6; m++) {
                 const double x = (m - 2.5) * h;
                 s.v[m] = scale * (off0 + a1 * x + a2 * x * x + a3 * x * x * x * x * x + noise * rnd());
             }
-            double um, up, pm, pp;
-            reconstruct_pair<kWCNS6_LD, -1, -1>(s, k, um, up);
             double r[6];
             for (int m = 0; m < 6; m++) r[m] = s.v[5 - m];
-            pm = plain_ld(s.v, ld_sigma(s), k);
-            pp = plain_ld(r, ld_sigma(s), k);
-            bad += std::memcmp(&um, &pm, 8) != 0;
-            bad += std::memcmp(&up, &pp, 8) != 0;
+            const double sigma = ld_sigma(s);
+            const double lm = plain_ld(s.v, sigma, k), lp = plain_ld(r, sigma, k);
+            bad += wrong<kWCNS6_LD, -1, -1>(s, k, lm, lp);
+            if (c.p == 2 && c.q == 4) bad += wrong<kWCNS6_LD, 2, 4>(s, k, lm, lp);
+            total += c.p == 2 && c.q == 4 ? 4 : 2;
             double b[3];
             betas(s.v, b);
             const double tau6 = std::fabs(beta6(s) - 1.0 / 8.0 * (b[0] + b[2] + 6.0 * b[1]));
             flat += tau6 * k.inv_thr < b[1] + kEps;
-            reconstruct_pair<kWCNS5_JS, -1, -1>(s, k, um, up);
-            pm = plain_js(s.v, c.p);
-            pp = plain_js(r, c.p);
-            bad += std::memcmp(&um, &pm, 8) != 0;
-            bad += std::memcmp(&up, &pp, 8) != 0;
-            total += 4;
+            if (scale < 1e70) {  // (squares of the indicators are beyond the numbers there)
+                const double jm = plain_js(s.v, c.p), jp = plain_js(r, c.p);
+                bad += wrong<kWCNS5_JS, -1, -1>(s, k, jm, jp);
+                if (c.p == 2) bad += wrong<kWCNS5_JS, 2, 4>(s, k, jm, jp);
+                total += c.p == 2 ? 4 : 2;
+            }
         }
         std::printf("p %d q %d C %g alpha %g: rule %s, held about %ld times\n", c.p, c.q, c.C, c.alpha, off ? "off" : "on", flat);
         const bool expect_off = c.C == 1e31 || c.C == 0.0 || c.alpha < 0.01;

@@ -108,6 +108,13 @@ inline int tile_rows_for(int64_t blocks24, int64_t blocks8) {
     return 4;
 }
 
+// Whether a batched single-species call takes both flux stages in one launch
+// (k_flux_both_single): tiles of fewer rows are a small call's (tile_rows_for),
+// or asked for.
+inline bool both_flux_stages(int dim, int tile_rows, int64_t items3) {
+    return dim > 1 && tile_rows != 24 && items3 > 0;
+}
+
 // Work items of the fused axis-a segment of one patch (whole wavefronts).
 __host__ __device__ inline int64_t fused_items(int axis, const int* n, int dim) {
     int64_t mid = 1;

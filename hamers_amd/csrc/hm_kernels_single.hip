@@ -516,8 +516,7 @@ hipError_t launch_single_dsq(const Plan<W>& plan, const KParams& k, hipStream_t 
         const bool rec = k.wrec != nullptr;  // recording runs (patch tables only)
         const unsigned nb2 = unsigned((plan.items[2] + kBlock - 1) / kBlock);
         const unsigned nb3 = unsigned((plan.items[3] + kBlock - 1) / kBlock);
-        // Tiles of fewer rows are a small call's (tile_rows_for), or asked for.
-        const bool both = D > 1 && plan.tile_rows != 24 && nb3 > 0;
+        const bool both = both_flux_stages(D, plan.tile_rows, plan.items[3]);
         if (nb2 > 0 && !both) {
             if (rec)
                 hipLaunchKernelGGL((k_flux_single<D, SCHEME, PP, QQ, W, true>), dim3(nb2), dim3(kBlock), 0, s, plan.work[2], k);

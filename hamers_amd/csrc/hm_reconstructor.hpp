@@ -963,14 +963,18 @@ class ConvectiveFluxReconstructorGPU {
     template <class W>
     int run(const Plan<W>& plan, const KParams& k, hipStream_t s) {
         if (!profiling_) return run_stages(plan, k, s, 0, kStages);
-        // One launch per stage, bracketed by events.
-        for (int stage = 0; stage < kStages; stage++) {
+        // Every stage's launch bracketed by events; flux stages that share a
+        // launch are timed together, as the call runs them.
+        int next = 0;
+        for (int stage = 0; stage < kStages; stage = next) {
+            next = stage + 1;
             if (plan.items[stage] == 0) continue;
+            if (stage == 2 && fused_ && both_flux_stages(cfg_.dim, plan.tile_rows, plan.items[3])) next = 4;
             if (prof_used_ + 2 > int(prof_events_.size()))
                 if (int st = collect_profile()) return st;
             hipEvent_t e0 = prof_events_[prof_used_], e1 = prof_events_[prof_used_ + 1];
             if (hipEventRecord(e0, s) != hipSuccess) return fail(HM_ERR_DEVICE, "hipEventRecord failed");
-            if (int st = run_stages(plan, k, s, stage, stage + 1)) return st;
+            if (int st = run_stages(plan, k, s, stage, next)) return st;
             if (hipEventRecord(e1, s) != hipSuccess) return fail(HM_ERR_DEVICE, "hipEventRecord failed");
             prof_stage_[prof_used_ / 2] = stage;
             prof_used_ += 2;

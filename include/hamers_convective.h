@@ -196,10 +196,14 @@ int hm_get_schedule_on_patches(hm_ctx* ctx, const hm_patch_view* patches, int nu
 /*
  * Stage timing (instrumentation; no counterpart in the reference).  While
  * enabled, every RHS call records HIP events on its stream around each of the
- * pipeline stages: 0 derived cell data, 1 dilatation/vorticity, 2 fused
- * midpoint flux, 3 midpoint-to-face flux, 4 advective source.  hm_profile_read
- * waits for the recorded events and returns the summed milliseconds and launch
- * counts per stage since the last hm_profile_enable.
+ * launches it makes, counted as the pipeline stages 0 derived cell data (with
+ * the dilatation and vorticity; none where a small per-patch call derives its
+ * cells in the flux), 1 unused, 2 and 3 flux, 4 advective source.  The flux is
+ * one launch, stage 2, but for two: a large batched single-species call (2: the
+ * first axis, 3: the others) and the persistent schedule of the four- and
+ * five-equation models (2: midpoint flux, 3: midpoint-to-face flux).
+ * hm_profile_read waits for the recorded events and returns the summed
+ * milliseconds and launch counts per stage since the last hm_profile_enable.
  */
 #define HM_NUM_STAGES 5
 int hm_profile_enable(hm_ctx* ctx, int enable);

@@ -515,6 +515,9 @@ class Level {
             for (int e = 0; e < nq_; e++) views[p].Q[e] = patch_[p].Q[1] + size_t(e) * gvol(p);
         const bool single = rec_->config().model == HM_MODEL_SINGLE_SPECIES;
         ConvectiveFluxReconstructorGPU::OwnedPlan trial;
+        DiffusiveFluxReconstructorGPU::OwnedPlan diff_trial;
+        if (diff_)
+            if (int st = build_diff_plan(0, views, diff_trial)) return st;
         const Schedule dflt = rec_->defaultSchedule(views.data(), np_);
         int st = rec_->tuneSchedules(
             s, reps,
@@ -525,12 +528,13 @@ class Level {
             },
             [&]() {
                 if (int e = rec_->runOwnedPlan(trial, dt, s, nullptr, nullptr, true)) return e;
-                if (diff_) return diff_->runOwnedPlan(diff_plan_[0], dt, s);
+                if (diff_) return diff_->runOwnedPlan(diff_trial, dt, s);
                 return int(HM_OK);
             },
             best, best_ms, default_ms, dflt);
         if (hipStreamSynchronize(s) != hipSuccess && st == HM_OK) st = rec_->fail(HM_ERR_DEVICE, "stream synchronize failed");
         rec_->releaseOwnedPlan(trial);
+        if (diff_) diff_->releaseOwnedPlan(diff_trial);
         if (st) return st;
         return setSchedule(best);
     }
@@ -556,7 +560,7 @@ class Level {
             for (int e = 0; e < nq_; e++) views_[0][p].Q[e] = patch_[p].Q[1] + size_t(e) * gvol(p);
         if (int st = build_rhs_plans()) return st;
         if (diff_)
-            if (int st = build_diff_plan(0)) return st;
+            if (int st = build_diff_plan(0, views_[0], diff_plan_[0])) return st;
         return build_rk_tables();
     }
 
@@ -947,7 +951,7 @@ class Level {
                 return rec_->fail(HM_ERR_OUT_OF_MEMORY, "level diffusive scratch");
             }
             for (int s = 0; s < kMaxRK; s++)
-                if (int st = build_diff_plan(s)) return st;
+                if (int st = build_diff_plan(s, views_[s], diff_plan_[s])) return st;
         }
         if (hipStreamCreateWithFlags(&cap_stream_, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&ev_a_, hipEventDisableTiming) != hipSuccess ||
@@ -966,14 +970,13 @@ class Level {
         return HM_OK;
     }
 
-    // Diffusive RHS of stage s's intermediate into the stage's diffusive fluxes.
-    int build_diff_plan(int s) {
-        std::vector<hm_patch_view> dv = views_[s];
+    // Diffusive RHS of the state that dv's patches hold into stage s's diffusive fluxes.
+    int build_diff_plan(int s, std::vector<hm_patch_view> dv, DiffusiveFluxReconstructorGPU::OwnedPlan& out) {
         for (int p = 0; p < np_; p++) {
             for (int a = 0; a < d_; a++) dv[p].F[a] = fdl_[(size_t(p) * kMaxRK + s) * 3 + a];
             dv[p].S = nullptr;
         }
-        return diff_->buildOwnedPlan(dv.data(), np_, static_cast<double*>(diff_scratch_), diff_plan_[s]);
+        return diff_->buildOwnedPlan(dv.data(), np_, static_cast<double*>(diff_scratch_), out);
     }
 
     // State buffer of stage s's intermediate (0: the scratch state).

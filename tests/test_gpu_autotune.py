@@ -189,3 +189,29 @@ def test_level_five_eqn_every_schedule(torch_dev, use_graph):
         torch.cuda.synchronize()
         assert np.array_equal(lvl.read_global(Qi.shape), want), sc
     _say(f"five-equation level, graph {use_graph}: {len(CANDIDATES_MULTI)} schedules bit-identical")
+
+
+def test_navier_stokes_level_autotune_keeps_results(torch_dev):
+    """The trials run both fluxes on a ghost-filled copy of the state; the level
+    steps as without them."""
+    from hamers_amd import ConvectiveFluxReconstructor, DiffusiveFluxReconstructor, Level
+    from tests.test_oracle_amr import NS_TR, ns_state
+
+    torch = torch_dev
+    Qi, n, dx, prm = ns_state(16)
+    rec = ConvectiveFluxReconstructor("lvl_ns", 2, "FOUR_EQN_CONSERVATIVE", "WCNS6_LD_HLLC_HLL", num_species=2,
+                                      species_gamma=tuple(prm.gamma), species_R=tuple(prm.R))
+    diff = DiffusiveFluxReconstructor(rec, NS_TR.mu, NS_TR.mu_v, NS_TR.kappa, NS_TR.D, NS_TR.M)
+    boxes = [((0, 0), (10, 16)), ((10, 0), (6, 16))]
+    dt = 0.2 * dx[0]
+    out = []
+    for tuned in (False, True):
+        lvl = Level(rec, boxes, ((0, 0), n), (1, 1), dx)
+        lvl.write_global(Qi)
+        if tuned:
+            _say(f"case Navier-Stokes level autotune: {lvl.autotune(dt, repetitions=2)}")
+        lvl.advance(dt, 2)
+        torch.cuda.synchronize()
+        out.append(lvl.read_global(Qi.shape))
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
+    del diff

@@ -260,8 +260,8 @@ __device__ __forceinline__ void diff_node(const DiffPatch& P, uint32_t c, uint32
 // node fluxes to memory and a second kernel the pair took 2.75 + 1.47 ms on a
 // level of 448 uneven patches (Navier-Stokes, 6-cell halos) and moved 13 GB;
 // fused with every derivative from memory 3.09 ms, now 2.66.  Blocks of 512 threads keep a
-// tile's rows 6 to 15 cells wide, XCD-contiguous blocks the lines at their edges
-// in one L2.
+// tile's rows 6 cells wide (axes of 63 cells or more) to 39 (one cell), and
+// XCD-contiguous blocks the lines at their edges in one L2.
 template <int D, int NS, int A>
 __device__ __forceinline__ void diff_tile(const DiffPatch& P, uint32_t tile, const DParams& k, double* lds) {
     constexpr int NEQ = NS + D + 1;
@@ -269,10 +269,9 @@ __device__ __forceinline__ void diff_tile(const DiffPatch& P, uint32_t tile, con
     const int R = P.tile[A][0], W = P.tile[A][1], ntA = P.tile[A][2];
     const uint32_t lane = threadIdx.x;
     const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
-    const uint32_t first = small_div(lane, uint32_t(P.tile[A][3]));  // lane / R on axis 0, lane / W on the others
-    const uint32_t rest = lane - first * uint32_t(A == 0 ? R : W);
-    const uint32_t r = A == 0 ? rest : first, w = A == 0 ? first : rest;
-    const int x = int(tA) * (R - 11) - 6 + int(r);  // cell along A
+    uint32_t r, w;
+    tile_place(A, lane, uint32_t(R), uint32_t(W), uint32_t(P.tile[A][3]), r, w);
+    const int x = int(tA) * (R - kDTileShared) - 6 + int(r);  // cell along A
     constexpr int U = (A == 0) ? 1 : 0;  // first axis across
     constexpr int V = (A == 2) ? 1 : 2;  // second axis across
     uint32_t cu, tv;

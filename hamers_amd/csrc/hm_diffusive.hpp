@@ -31,21 +31,6 @@ namespace hm {
 constexpr int kGd = 6;  // diffusive ghost width (DiffusiveFluxReconstructorNodeSixthOrder.cpp:22)
 constexpr int kDiffStages = 2;
 
-// Tile of the diffusive flux (k_diff_flux): a block of kDTile threads takes R
-// consecutive cells along the axis by W columns (R W <= kDTile) and outputs
-// R - 11 faces of each column (a face takes six nodes, a node seven cells).  A
-// column of n_A + 12 cells (n_A + 1 faces) takes ntA tiles of equal length that
-// share eleven cells, of at most 74 faces in 2D and 3D (W >= 6 columns, so that
-// a row of them is most of a cache line), of as many as the block holds in 1D.
-constexpr int kDTile = 512;
-
-inline void dtile_shape(int dim, int nA, int& R, int& W, int& ntA) {
-    const int most = dim == 1 ? kDTile - 11 : 74;
-    ntA = (nA + 1 + most - 1) / most;
-    R = (nA + 1 + ntA - 1) / ntA + 11;
-    W = kDTile / R;
-}
-
 struct DiffPatch {
     int n[3];                     // interior extents (1 on unused axes)
     int gq[3];                    // ghost width of Q (0 on unused axes)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "hm_device.hpp"
+#include "hm_tiles.hpp"
 
 namespace hm {
 
@@ -120,59 +121,6 @@ __host__ __device__ inline int64_t fused_items(int axis, const int* n, int dim) 
     int64_t mid = 1;
     for (int b = 0; b < dim; b++) mid *= (b == axis) ? n[b] + 3 : n[b];
     return int64_t(64) * ((mid - 3) / kChunk + 1);
-}
-
-// Fused midpoint and face flux of the multi-species models (k_flux_multi): a
-// 256-thread block owns a tile of R consecutive midpoint faces along the axis
-// by W positions across it (R W <= 256), keeps the tile's midpoint fluxes in
-// LDS and outputs the R - 2 inner faces of each of its W columns.  A column of
-// n_A + 3 midpoint faces (n_A + 1 output faces) takes ntA tiles of at most
-// kMTileFaces output faces each, of equal length, which share two midpoint
-// faces; W is as many columns as fit.
-constexpr int kMTileFaces = 62;
-
-
-// small: tiles of 64 faces (k_flux_multi_small) of at most 14 output faces, so
-// that the columns of a tile are a few neighbours in memory (30 instead of 14:
-// 24^3 five-equation call 27.3 us instead of 26.0); a 1D patch has one column.
-__host__ __device__ inline void mtile_shape(int nA, int& R, int& W, int& ntA, bool small = false, int dim = 3) {
-    const int most = small && dim > 1 ? 14 : kMTileFaces;
-    ntA = (nA + 1 + most - 1) / most;
-    R = (nA + 1 + ntA - 1) / ntA + 2;
-    W = (small ? 64 : 256) / R;
-}
-
-// Exact division of a thread number x by d, both up to 512, as a product: m d
-// exceeds 2^20 by less than d, so x m is off by less than x d < 2^20, under one
-// in the quotient's last place.
-__host__ __device__ inline uint32_t small_div_mul(uint32_t d) { return ((1u << 20) + d - 1u) / d; }
-__host__ __device__ inline uint32_t small_div(uint32_t x, uint32_t m) { return (x * m) >> 20; }
-
-// Column (u, v) of a tile's position w: columns run u fastest over nU by nV
-// positions, the tile's first one is t0 (block-uniform), W of them per tile.
-__device__ __forceinline__ void tile_column(uint32_t t0, uint32_t w, uint32_t W, uint32_t nU, uint32_t& u,
-                                            uint32_t& v) {
-    const uint32_t v0 = t0 / nU;
-    u = t0 - v0 * nU + w;
-    if (nU >= W) {  // at most one row on
-        const bool over = u >= nU;
-        v = v0 + (over ? 1u : 0u);
-        u -= over ? nU : 0u;
-    } else {  // u < nU + W
-        const uint32_t q = small_div(u, small_div_mul(nU));
-        v = v0 + q;
-        u -= q * nU;
-    }
-}
-
-// Work items of the fused axis-a segment of one patch: a block of 256 per tile.
-__host__ __device__ inline int64_t mtile_items(int axis, const int* n, int dim, bool small = false) {
-    int64_t trans = 1;  // columns: positions across the axis
-    for (int b = 0; b < dim; b++)
-        if (b != axis) trans *= n[b];
-    int R, W, ntA;
-    mtile_shape(n[axis], R, W, ntA, small, dim);
-    return int64_t(256) * ntA * ((trans + W - 1) / W);
 }
 
 // Work of one RHS evaluation: one work source per pipeline stage

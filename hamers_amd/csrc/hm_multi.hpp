@@ -854,7 +854,7 @@ __global__ __launch_bounds__(kBlock) void k_faceflux_multi(W w, KParams k) {
 // neighbours' midpoint fluxes and its own and its lower neighbour's node fluxes.  Every output face has one such
 // thread; the five-equation u* of a midpoint face is written by one tile (its
 // first R - 2 faces, and the last tile of a column all of its faces).
-static_assert(kBlock == 256, "a fused multi-species tile is one 256-thread block");
+static_assert(kBlock == kMTileThreads, "a fused multi-species tile is one 256-thread block");
 
 template <int D, int NS, bool FOUR, int A, int SCHEME, int PP, int QQ, class Work>
 __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile, const KParams& k, double* wlds) {
@@ -865,13 +865,7 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
     const uint32_t lane = threadIdx.x;
     const uint32_t tw = tile / uint32_t(ntA), tA = tile - tw * uint32_t(ntA);
     uint32_t r, w;
-    if constexpr (A == 0) {
-        w = small_div(lane, uint32_t(P.tile[A][3]));  // lane / R
-        r = lane - w * uint32_t(R);
-    } else {
-        r = small_div(lane, uint32_t(P.tile[A][3]));  // lane / W
-        w = lane - r * uint32_t(W);
-    }
+    tile_place(A, lane, uint32_t(R), uint32_t(W), uint32_t(P.tile[A][3]), r, w);
     const int j = int(tA) * (R - 2) + int(r);
     // columns: positions across the axis, x fastest over the other axes; the
     // tile's first one is block-uniform, the others follow within a few rows
@@ -943,9 +937,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
 // A call that fills the device takes k_flux_multi, whose four times larger
 // tiles share fewer faces and cells.
 // ----------------------------------------------------------------------------
-constexpr int kSmallCells = 144;   // (R + 5) W: at most 9 x 16
-constexpr int kSmallSensor = 80;   // (R + 1) W: at most 5 x 16
-
 // Derived values and sensor of a tile's face in LDS, the others in Q.
 template <int D, int NS, bool FOUR, int A>
 struct TileFace {
@@ -1015,7 +1006,7 @@ __device__ __forceinline__ void flux_multi_small_tile(const DevPatch& P, uint32_
     // the sensor of its cells j0 - 2 .. j0 + R - 2.
     const uint32_t t = threadIdx.x;
     const uint32_t ncell = uint32_t((R + 5) * W), nsens = uint32_t((R + 1) * W);
-    const uint32_t s0 = ncell > 128u ? ncell : 128u;
+    const uint32_t s0 = small_sensor_first(ncell);
     int r, w, c[3];
     if (t < ncell) {
         place(t, R + 5, r, w);

@@ -47,17 +47,17 @@ FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 (vector and matrix)
 HEADLINE_KERNEL_COUNTS = {
     "k_flux_multi": {
         "cells": 68726784,
-        # 64 x (3 183 943 166 + 5 225 870 196 + 173 290 695 + 2 x 1 816 869 361)
-        "fp64_ops": 64 * (3183943166 + 5225870196 + 173290695 + 2 * 1816869361),
-        # FETCH_SIZE 14 264 514 KiB x 2.0 + WRITE_SIZE 13 681 375 KiB x 1.0
-        "dram_bytes": 14264514 * 1024 * 2 + 13681375 * 1024,
-        "valu_issue_frac": 0.841,
+        # 64 x (3 183 943 166 + 5 047 717 080 + 232 675 067 + 2 x 1 995 022 477)
+        "fp64_ops": 64 * (3183943166 + 5047717080 + 232675067 + 2 * 1995022477),
+        # FETCH_SIZE 14 242 311 KiB x 2.0 + WRITE_SIZE 13 685 662 KiB x 1.0
+        "dram_bytes": 14242311 * 1024 * 2 + 13685662 * 1024,
+        "valu_issue_frac": 0.834,
         "source": "profiles/rhs_uneven3d_five_eqn_counters.md",
     },
 }
 # The same for the 2D single-species leg's flux kernels (2048^2 in 128^2
 # patches, WCNS5-JS): DRAM bytes per launch.
-FLUX_TRAFFIC_2048_WCNS5 = {"midflux": 354.92e6 + 135.27e6, "faceflux": 506.47e6 + 135.27e6}
+FLUX_TRAFFIC_2048_WCNS5 = {"midflux": 354.81e6 + 135.27e6, "faceflux": 506.13e6 + 135.27e6}
 STAGE_KERNEL_SINGLE = {"midflux": "k_flux_single", "faceflux": "k_flux_tile_single"}
 # (the multi-species midpoint and face flux run fused in one kernel, timed as the midflux stage)
 STAGE_KERNEL_MULTI = {"derived": "k_derived_multi", "midflux": "k_flux_multi", "faceflux": "k_faceflux_multi",
@@ -418,7 +418,7 @@ def bench_2d(args, torch, np):
             "flux_kernel": {"kernel": STAGE_KERNEL_SINGLE.get(dominant, dominant), "kernel_ms": stage[dominant],
                             "bytes_per_cell": 8 * (neq + neq), "achieved_gbs": kgbs, "hbm_frac": kgbs / HBM_PEAK_GBS,
                             "traffic": traffic, "bound": "valu",
-                            "counts_source": "profiles/flux_kernels_2048sq_counters.md (72-79 % of VALU issue)"},
+                            "counts_source": "profiles/flux_kernels_2048sq_counters.md (71-76 % of VALU issue)"},
             "rhs_hbm_frac": 8 * (neq + 2 * neq) * cells / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
 
 

@@ -77,8 +77,8 @@ struct DevPatch {
     double* sens;                 // scratch: theta, Omega over the 2-ghost box
     double* fmid[3];              // scratch: midpoint flux per axis, neq comps over (n_a+3) x n_b box
     double* ustar[3];             // scratch: HLLC normal velocity per axis (advective models)
-    int tile[3][4];               // shape of the axis' multi-species flux tiles (mtile_shape), and a multiplier that
-                                  // divides a thread number by a tile row (mtile_row)
+    int tile[3][4];               // shape of the axis' multi-species flux tiles (mtile_shape), and the multiplier of
+                                  // tile_place
     const double* vb[HM_MAX_EQN]; // multi-species: component base of each variable of the reconstruction (Q or prim)
     int64_t vst[3][2];            // cell stride along axis a of the prim box and of Q's box
     int64_t wrec[3];              // offset of this patch's axis-a chunk in a face-state slot (KParams::wrec), -1: none

@@ -38,9 +38,10 @@ __device__ __forceinline__ int64_t dq_idx(const DiffPatch& P, int i, int j, int 
 // Component slots of the derived cell data: only what the node fluxes
 // differentiate, and the pressure.  The density is the sum of the caller's
 // partial densities, and the enthalpies and the mixture's transport
-// coefficients follow from Y_i, p and T where a node uses them.  Bound by HBM:
+// coefficients follow from Y_i, p and T where a node uses them.  Bound by memory:
 // twelve stored components instead of seven took 1.06 ms on a level of 448
-// uneven patches, now 0.73 (5.6 TB/s).
+// uneven patches, now 0.73 (5.6 TB/s of arrays read and written; how much of
+// it reaches HBM is not counted).
 template <int D, int NS>
 struct DiffSlots {
     static constexpr int Y = 0, U = NS, T = NS + D, P = NS + D + 1;

@@ -174,13 +174,6 @@ __device__ __forceinline__ void cell_state_multi(const KParams& k, QF&& q, uint3
     }
 }
 
-// ----------------------------------------------------------------------------
-// Derived cell data (FlowModelFiveEqnAllaire.cpp:3734-4876,
-// FlowModelFourEqnConservative.cpp:3877-5440).  Bound by HBM writes (a copy
-// reaches 4.2 TB/s here, read and written): with the partial densities, volume
-// fractions and rho stored too, nine components instead of five, it took 5.30 ms
-// on the uneven 3D five-equation level of 2744 patches, 4.34 ms without them.
-// ----------------------------------------------------------------------------
 // Velocity components of the cell at `at`, from q(e, at): the same bits as
 // cell_state_multi's.
 template <int D, int NS, class QF>
@@ -193,6 +186,14 @@ __device__ __forceinline__ void cell_velocity_multi(QF&& q, uint32_t at, double 
     for (int b = 0; b < D; b++) v[b] = quot(q(NS + b, at), rho, rrho);
 }
 
+// ----------------------------------------------------------------------------
+// Derived cell data (FlowModelFiveEqnAllaire.cpp:3734-4876,
+// FlowModelFourEqnConservative.cpp:3877-5440).  Bound by HBM: 3.9 TB/s of
+// counted traffic where a device copy reaches 4.25.  With the partial densities,
+// volume fractions and rho stored too, nine components instead of five, it took
+// 5.30 ms on the uneven 3D five-equation level of 2744 patches, 4.34 ms without
+// them.
+// ----------------------------------------------------------------------------
 template <int D, int NS, bool FOUR, class W>
 __global__ __launch_bounds__(kBlock) void k_derived_multi(W w, KParams k) {
     const int64_t gid = int64_t(rhs_block(k)) * kBlock + threadIdx.x;
@@ -310,11 +311,6 @@ __device__ __forceinline__ bool bounded_multi(const double* V, const KParams& k)
     return ok && (c2 > double(0));
 }
 
-// Bound by VALU issue: on the uneven 3D five-equation level of 2744 patches the
-// fused flux issues 3193 VALU instructions per wavefront at 84 % of the rate
-// (4357 at 75 % before its loads took scalar bases, a field's loads went out
-// together and the WENO weights lost a quarter of their instructions): 36.4 ms
-// -> 24.0 ms.
 // Stencil and sensor of the face normal to axis A between cells (c0, c1, c2) -
 // e_A and (c0, c1, c2) from the patch's arrays: at 32-bit offsets from
 // wave-uniform bases (every patch's ghost box is below 2^29 cells) that hold the
@@ -904,7 +900,11 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
 }
 
 // The fused flux stage: every block is one tile (the stage's segments hold
-// whole tiles), so all threads of a block reach the barrier.
+// whole tiles), so all threads of a block reach the barrier.  Bound by VALU
+// issue: on the uneven 3D five-equation level of 2744 patches it issues 3209
+// VALU instructions per wavefront at 83 % of the rate (4357 at 75 % before its
+// loads took scalar bases, a field's loads went out together and the WENO weights
+// lost a quarter of their instructions): 36.4 ms -> 24.3 ms.
 template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
     D == 3 ? HM_MIDFLUX_MULTI_WAVES_3D : HM_MIDFLUX_MULTI_WAVES))) void k_flux_multi(W w, KParams k) {

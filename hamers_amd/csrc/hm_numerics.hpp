@@ -71,7 +71,8 @@ HM_HD double quot(double a, double b, double r) {
 // Reciprocal by two quadratic steps, for the adjoint's reverse sweep, which
 // multiplies by it.  It equals rcp_rn except for a last place now and then; in
 // stencils just above the indicators' rounding noise the sweep magnifies that
-// to 1e-3 of a gradient, so it keeps this form's bits.
+// to 1e-3 of the gradient of a random final adjoint.  Neither form is known to
+// be the better one there; this one keeps the gradients as they were.
 HM_HD double rcp_two(double b) {
 #if defined(HM_RCP_ESTIMATE)
     double r = HM_RCP_ESTIMATE(b);

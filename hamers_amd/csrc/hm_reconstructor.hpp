@@ -566,23 +566,35 @@ class ConvectiveFluxReconstructorGPU {
             plan.items[2] = acc;
             plan.items[3] = 0;
             // Small calls derive their cells in the flux kernel (one launch
-            // instead of two): every 1D patch (200 cells 14.9 -> 10.7 us, 2e5
-            // 20.7 -> 16.9), 2D patches of 4-row tiles (64^2 16.0 -> 11.8, 128^2
-            // 20.2 -> 16.0, 400^2 41.6 -> 35.8), 3D patches up to 2^18 work items
-            // (16^3 19.7 -> 17.2, 24^3 22.6 -> 22.0; at 32^3, 3.2e5 items, the
-            // six-fold work loses: 30.1 -> 31.3).
+            // instead of two).  Per call, WCNS6-LD and WCNS5-JS (1D and 2D against
+            // the two launches with weights a few percent slower): every 1D patch
+            // (200 cells 14.2 -> 12.9 and 12.8 -> 9.3 us, 2e5 27.1 -> 23.6 and
+            // 18.6 -> 15.3), 2D patches of 4-row tiles (64^2 17.2 -> 14.9 and 14.0
+            // -> 10.7, 128^2 17.5 -> 14.9 and 14.3 -> 10.8, 256^2 36.1 -> 32.7 and
+            // 26.3 -> 20.1), 3D patches up to 2^18 work items (16^3 24.0 -> 21.9
+            // and 18.9 -> 16.9; even from 22^3, 29.7 -> 30.0 and 21.3 -> 21.7, to
+            // 28^3, 37.9 -> 37.5 and 26.1 -> 26.4; at 32^3, 3.2e5 items, the
+            // six-fold work loses: 44.7 -> 45.4 and 29.9 -> 31.2).
             plan.direct = plan.tile_rows == 4 && (d < 3 || acc <= (int64_t(1) << 18));
             if (plan.direct) plan.items[0] = 0;
         }
         if (!fused_) {
             const int nn[3] = {v.n[0], d > 1 ? v.n[1] : 1, d > 2 ? v.n[2] : 1};
-            // A small patch takes 64-face tiles that derive their cells (five
-            // equations, WCNS6-LD: 8^3 29.9 -> 18.9 us, 16^3 29.6 -> 21.4, 24^3
-            // 30.1 -> 26.0, 28^3, 294 tiles of 256 faces, 36.0 -> 32.5, 128^2
-            // 28.0 -> 20.5, 256^2, 640 tiles, 39.2 -> 35.5) until the device is
-            // full of the larger tiles: 32^3 with 441 of them 37.5 -> 38.8, 64^3
-            // 130 -> 171, 320^2 with 960 47.2 -> 47.6.  A 1D patch has one column,
-            // which fills a quarter of a 256-face tile: 2e5 cells 42.9 -> 33.7.
+            // A small patch takes 64-face tiles that derive their cells, until
+            // the device is full of the 256-face tiles.  Per call with the large
+            // tiles -> the small ones, two species, five equations with WCNS6-LD,
+            // WCNS5-JS, four equations with WCNS6-LD, WCNS5-JS (us): 16^3 28.5 ->
+            // 19.7, 23.7 -> 18.0, 23.2 -> 14.4, 19.1 -> 12.3; 28^3, 294 tiles, 36.1
+            // -> 31.2, 28.3 -> 26.0, 29.7 -> 24.7, 22.4 -> 20.5; 30^3, 387 tiles,
+            // even; 32^3, 441 tiles, 37.9 -> 39.6, 29.8 -> 31.6, 31.2 -> 32.8, 23.9
+            // -> 25.6; 256^2, 640 tiles, 41.9 -> 38.6, 31.2 -> 29.6, 34.7 -> 32.5,
+            // 25.1 -> 22.5; 288^2, 720 tiles, 43.5 -> 45.0, 33.0 -> 34.0, 36.1 ->
+            // 38.0, 26.3 -> 25.6.  Three species cross at the same sizes (28^3
+            // 42.5 -> 37.4, 30^3 43.8 -> 45.1, 32^3 45.0 -> 50.0 with five equations
+            // and WCNS6-LD).  Inside the limits large tiles that happen to fill
+            // win here and there: 240^2, 480 tiles, 34.6 -> 36.2.  A 1D patch has
+            // one column, which fills a quarter of a 256-face tile: 2e5 cells
+            // (against slower weights by a few percent) 59.1 -> 36.3 and 38.5 -> 26.1, 48.7 -> 28.0 and 30.2 -> 20.6.
             plan.direct = d == 1 || plan.items[2] <= int64_t(kBlock) * (d == 2 ? 640 : 400);
             if (plan.direct) {
                 SegSingle& w = plan.work[2];

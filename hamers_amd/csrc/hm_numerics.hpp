@@ -210,9 +210,10 @@ HM_HD double ld_combine(const Six& s, double w0, double w1, double w2, double w3
 // Where no lane of the wavefront has a ratio tau6 / (beta_k + eps) that
 // reaches the sum C + ratio^q (resolved data: 30-50 % of the wavefronts of
 // shear layers, mixing layers and smooth modes), the weights are constants and
-// every quotient is left out.  Common factors that are powers of two (1/32 of
-// the central weights, 1/16 of the upwind ones, 1/8 of beta_avg) cancel or
-// scale exactly and are not multiplied out.
+// every quotient is left out.  Factors that are powers of two scale exactly:
+// 1/32 of the outer central weights and 1/16 of the first upwind one are taken
+// into the sum as an FMA (left out, the sums would overflow before the
+// reference's do), 1/8 of beta_avg into the next operation.
 template <int P, int Q>
 HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k) {
     double b0, b1, b2;
@@ -233,10 +234,11 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
     }
 
     const double r0 = rcp_rn(e0), r1 = rcp_rn(e1), r2 = rcp_rn(e2);
-    double w0 = k.C + rep_pow<Q>(quot(tau6, e0, r0), k.q);
-    double w1 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e1, r1), k.q));
-    double w2 = double(15) * (k.C + rep_pow<Q>(quot(tau6, e2, r2), k.q));
-    double w3 = k.C + rep_pow<Q>(div_rn(tau6, e3), k.q);
+    const double c32 = double(1) / double(32) * k.C;
+    double w0 = fma(double(1) / double(32), rep_pow<Q>(quot(tau6, e0, r0), k.q), c32);
+    double w1 = double(15) / double(32) * (k.C + rep_pow<Q>(quot(tau6, e1, r1), k.q));
+    double w2 = double(15) / double(32) * (k.C + rep_pow<Q>(quot(tau6, e2, r2), k.q));
+    double w3 = fma(double(1) / double(32), rep_pow<Q>(div_rn(tau6, e3), k.q), c32);
     const double ws = w0 + w1 + w2 + w3;
     const double rws = rcp_rn(ws);
     w0 = quot(w0, ws, rws);
@@ -252,9 +254,9 @@ HM_HD double ld_side(const Six& s, const Six& s0, double& sig, const LDConst& k)
     if (over > double(0) || !(den > double(0))) {
         if ((den > double(0) && over > double(8.8817841970012523e-16) * tau6) || div_rn(tau6, den) > k.alpha_tau) {
             const double tau5 = fabs(b0 - b2);
-            double u0 = double(1) + rep_pow<P>(quot(tau5, e0, r0), k.p);
-            double u1 = double(10) * (double(1) + rep_pow<P>(quot(tau5, e1, r1), k.p));
-            double u2 = double(5) * (double(1) + rep_pow<P>(quot(tau5, e2, r2), k.p));
+            double u0 = fma(double(1) / double(16), rep_pow<P>(quot(tau5, e0, r0), k.p), double(1) / double(16));
+            double u1 = double(5) / double(8) * (double(1) + rep_pow<P>(quot(tau5, e1, r1), k.p));
+            double u2 = double(5) / double(16) * (double(1) + rep_pow<P>(quot(tau5, e2, r2), k.p));
             const double us = u0 + u1 + u2;
             const double rus = rcp_rn(us);
             u0 = quot(u0, us, rus);

@@ -176,6 +176,16 @@ int main() {
                 total += c.p == 2 ? 4 : 2;
             }
         }
+        // powers up to the largest number: one jump beside equal values (differing floors only)
+        for (double a = 1e10; a < 1e60; a *= 1.02) {
+            const double u[6] = {0, 0, 0, 0, 0, a}, r[6] = {a, 0, 0, 0, 0, 0};
+            Six s;
+            std::memcpy(s.v, u, sizeof s.v);
+            const double sigma = ld_sigma(s), lm = plain_ld(u, sigma, k), lp = plain_ld(r, sigma, k);
+            bad += wrong<kWCNS6_LD, -1, -1>(s, k, lm, lp);
+            if (c.p == 2 && c.q == 4) bad += wrong<kWCNS6_LD, 2, 4>(s, k, lm, lp);
+            total += c.p == 2 && c.q == 4 ? 4 : 2;
+        }
         std::printf("p %d q %d C %g alpha %g: rule %s, held about %ld times\n", c.p, c.q, c.C, c.alpha, off ? "off" : "on", flat);
         const bool expect_off = c.C == 1e31 || c.C == 0.0 || c.alpha < 0.01;
         if (off != expect_off || (!off && flat == 0)) {

@@ -47,11 +47,11 @@ FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 (vector and matrix)
 HEADLINE_KERNEL_COUNTS = {
     "k_flux_multi": {
         "cells": 68726784,
-        # 64 x (3 183 943 166 + 5 047 717 080 + 232 675 067 + 2 x 1 995 022 477)
-        "fp64_ops": 64 * (3183943166 + 5047717080 + 232675067 + 2 * 1995022477),
-        # FETCH_SIZE 14 242 311 KiB x 2.0 + WRITE_SIZE 13 685 662 KiB x 1.0
-        "dram_bytes": 14242311 * 1024 * 2 + 13685662 * 1024,
-        "valu_issue_frac": 0.834,
+        # 64 x (3 112 390 675 + 5 047 717 080 + 232 675 067 + 2 x 2 066 574 968)
+        "fp64_ops": 64 * (3112390675 + 5047717080 + 232675067 + 2 * 2066574968),
+        # FETCH_SIZE 14 239 185 KiB x 2.0 + WRITE_SIZE 13 690 380 KiB x 1.0
+        "dram_bytes": 14239185 * 1024 * 2 + 13690380 * 1024,
+        "valu_issue_frac": 0.836,
         "source": "profiles/rhs_uneven3d_five_eqn_counters.md",
     },
 }

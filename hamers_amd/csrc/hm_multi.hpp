@@ -901,10 +901,10 @@ __device__ __forceinline__ void flux_multi_tile(const DevPatch& P, uint32_t tile
 
 // The fused flux stage: every block is one tile (the stage's segments hold
 // whole tiles), so all threads of a block reach the barrier.  Bound by VALU
-// issue: on the uneven 3D five-equation level of 2744 patches it issues 3209
-// VALU instructions per wavefront at 83 % of the rate (4357 at 75 % before its
+// issue: on the uneven 3D five-equation level of 2744 patches it issues 3231
+// VALU instructions per wavefront at 84 % of the rate (4357 at 75 % before its
 // loads took scalar bases, a field's loads went out together and the WENO weights
-// lost a quarter of their instructions): 36.4 ms -> 24.3 ms.
+// lost a quarter of their instructions): 36.4 ms -> 24.5 ms.
 template <int D, int NS, bool FOUR, int SCHEME, int PP, int QQ, class W>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(
     D == 3 ? HM_MIDFLUX_MULTI_WAVES_3D : HM_MIDFLUX_MULTI_WAVES))) void k_flux_multi(W w, KParams k) {

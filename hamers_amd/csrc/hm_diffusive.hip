@@ -261,7 +261,7 @@ __device__ __forceinline__ void diff_node(const DiffPatch& P, uint32_t c, uint32
 // node fluxes to memory and a second kernel the pair took 2.75 + 1.47 ms on a
 // level of 448 uneven patches (Navier-Stokes, 6-cell halos) and moved 13 GB;
 // fused with every derivative from memory 3.09 ms, now 2.66.  Blocks of 512 threads keep a
-// tile's rows 6 cells wide (axes of 63 cells or more) to 39 (one cell), and
+// tile's rows 6 cells wide (62 to 73 cells along the axis) to 39 (one cell), and
 // XCD-contiguous blocks the lines at their edges in one L2.
 template <int D, int NS, int A>
 __device__ __forceinline__ void diff_tile(const DiffPatch& P, uint32_t tile, const DParams& k, double* lds) {
